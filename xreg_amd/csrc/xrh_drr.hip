@@ -667,12 +667,9 @@ TilePlan build_tiles(const std::vector<int32_t>& rows, const std::vector<int32_t
   for (int b = 0; b < p.bands; ++b) {
     uint32_t acc = 0;
     for (int64_t i = 0; i < n; ++i) {
-      const int TX = (cols[i] + kTile - 1) / kTile;
-      const int TY = (rows[i] + kTile - 1) / kTile;
-      const int r0 = (int)(((int64_t)b * TY) / p.bands);
-      const int r1 = (int)(((int64_t)(b + 1) * TY) / p.bands);
+      const int tiles = ((cols[i] + kTile - 1) / kTile) * ((rows[i] + kTile - 1) / kTile);
       p.band_start[(size_t)b * (n + 1) + i] = acc;
-      acc += (uint32_t)((r1 - r0) * TX);
+      acc += band_first_tile(i, tiles, b + 1, p.bands) - band_first_tile(i, tiles, b, p.bands);
     }
     p.band_start[(size_t)b * (n + 1) + n] = acc;
     if ((int64_t)acc > p.max_band_tiles) p.max_band_tiles = acc;

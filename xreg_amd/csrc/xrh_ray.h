@@ -256,11 +256,10 @@ __device__ inline TileRef decode_tile(const uint32_t* band_start, int64_t num_it
     if (bs[mid] <= j) lo = mid; else hi = mid - 1;
   }
   t.item = lo;
-  const uint32_t local = j - bs[lo];
   const int TX = items[lo * stride].tiles_x, TY = items[lo * stride].tiles_y;
-  const int row0 = (int)(((int64_t)band * TY) / bands);
-  t.ty = row0 + (int)(local / (uint32_t)TX);
-  t.tx = (int)(local % (uint32_t)TX);
+  const uint32_t tile = band_first_tile(lo, TX * TY, band, bands) + (j - bs[lo]);
+  t.ty = (int)(tile / (uint32_t)TX);
+  t.tx = (int)(tile % (uint32_t)TX);
   return t;
 }
 

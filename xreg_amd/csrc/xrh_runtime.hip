@@ -521,14 +521,15 @@ static void volume_create(xrh_ctx* ctx, const float* vox, const int64_t size[3],
 static int64_t build_tiles_uniform(int32_t rows, int32_t cols, int64_t num_projs, int32_t bands,
                                    uint32_t* band_start)
 {
-  const int TX = (cols + 15) / 16, TY = (rows + 15) / 16;
+  const int tiles = ((cols + 15) / 16) * ((rows + 15) / 16);
   int64_t max_tiles = 0;
   for (int b = 0; b < bands; ++b) {
-    const int r0 = (int)(((int64_t)b * TY) / bands);
-    const int r1 = (int)(((int64_t)(b + 1) * TY) / bands);
-    const uint32_t per = (uint32_t)((r1 - r0) * TX);
-    for (int64_t i = 0; i <= num_projs; ++i) band_start[(size_t)b * (num_projs + 1) + i] = (uint32_t)(i * per);
-    max_tiles = std::max<int64_t>(max_tiles, (int64_t)per * num_projs);
+    uint32_t acc = 0;
+    for (int64_t i = 0; i <= num_projs; ++i) {
+      band_start[(size_t)b * (num_projs + 1) + i] = acc;
+      acc += band_first_tile(i, tiles, b + 1, bands) - band_first_tile(i, tiles, b, bands);
+    }
+    max_tiles = std::max<int64_t>(max_tiles, band_start[(size_t)b * (num_projs + 1) + num_projs]);
   }
   return max_tiles;
 }
