@@ -420,10 +420,9 @@ xrh_status xrh_batch_last_timing(const xrh_batch* batch, float* drr_kernel_ms, f
 /* DRR launch variants. Every variant casts the same rays with the same arithmetic, so DRRs
  * are identical under all of them (fused NCC sums may differ in the last FP64 bits: the
  * per-tile summation order follows the wave footprint).
- *   cell_reuse  1: one sample per loop iteration, the current cell's 32 bytes kept in
- *               registers and loaded only when a sample enters a new cell; 0: two samples per
- *               iteration, each loading its cell; -1: by launch size (1 from 16 workgroups
- *               per CU up)
+ *   cell_reuse  1: one lane marches a whole ray; 0: two or four waves share each ray (the most
+ *               that keeps every workgroup resident, at least two); -1: by launch size (shared
+ *               when at least two waves per ray keep every workgroup resident)
  *   wave_shape  pixels per wave64 inside the 16x16 workgroup tile: 0 = 8x8, 1 = 16x4, 2 = 4x16
  *   bands       detector-row bands of the XCD-aware workgroup order, 1..16 (default 8)
  * The environment variable XRH_CELL_REUSE, when set, still overrides cell_reuse. */

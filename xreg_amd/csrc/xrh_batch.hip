@@ -69,6 +69,7 @@ struct xrh_batch {
   bool variant_set = false;
   DrrVariant variant;
   DrrVariant last_variant;         // the variant of the last staged launch
+  int32_t last_slab = 0;           // and its slab-marching choice
 };
 
 namespace {
@@ -309,6 +310,8 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
                 "the objects of one item must share the detector size");
   }
   int64_t off = 0;
+  double spacing = 0.0;
+  uint64_t vol_bytes = 0;
   groups.clear();
   for (int64_t i = 0; i < n; ++i) {
     const int32_t v = item_view[i * objs];
@@ -326,6 +329,8 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
       p.bg = (k == 0 && bg) ? bg + bg_off[(size_t)v] : nullptr;
       p.step = b->views[vk].step;
       p.pad_ = 0;
+      spacing += ray_spacing(b->views[vk].vol, b->views[vk].cam, p.pose);
+      vol_bytes = std::max<uint64_t>(vol_bytes, b->views[vk].vol->bytes);
     }
     rows[i] = w.cam.num_det_rows;
     cols[i] = w.cam.num_det_cols;
@@ -391,6 +396,9 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
   D.out = drr;
   D.ncc_partials = b->ncc_partials_dev;
   D.ncc_tiles_per_item = b->max_img_tiles;
+  D.ray_spacing = (float)(spacing / (double)(n * objs));
+  D.vol_bytes = vol_bytes;
+  b->last_slab = drr_slab_lds(D.ray_spacing, b->geom, vol_bytes);
   D.reuse = var.reuse;
   D.wave_shape = var.shape;
   D.objs = objs;
@@ -430,6 +438,7 @@ std::string signature(const xrh_batch* b, const int32_t* item_view, int64_t n, c
   key.append((const char*)&drr_out, sizeof(drr_out));
   key.append((const char*)&b->version, sizeof(b->version));
   key.append((const char*)&b->last_variant, sizeof(b->last_variant));
+  key.append((const char*)&b->last_slab, sizeof(b->last_slab));
   return key;
 }
 

@@ -26,6 +26,7 @@
 
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <climits>
 #include <cstdlib>
 #include <cstring>
@@ -35,16 +36,15 @@ namespace {
 
 // ---------------------------------------------------------------------------------------
 // trilinear sampling per layout. Formats: 0 f32 linear, 1 f32 quad, 2 f16 linear, 3 f16 oct,
-// 4 bf16 linear, 5 bf16 oct.
+// 4 bf16 linear, 5 bf16 oct, sampled one by one; 7 f32 coefficients, 11 f32 x-faces, 13 f32
+// x-faces in bricks, fetched cell by cell (two 16-byte loads) and marched with march_cells.
+constexpr bool is_cell_fmt(int fmt) { return fmt == 7 || fmt == 11 || fmt == 13; }
 
 struct VolView {
   __amdgpu_buffer_rsrc_t rsrc;
   uint32_t py;     // row pitch (elements)
   uint32_t pz;     // slice pitch (elements)
   uint32_t apron;  // 1 + py + pz: element index of voxel (0, 0, 0)
-  // last cell fetched (coefficient layout with cell reuse): its index and 32 bytes
-  uint32_t ce;
-  uint4 ca, cb;
 };
 
 // a (1 - w) + b w as two fused multiply-adds: as cheap as a + (b - a) w but without its
@@ -75,12 +75,12 @@ __device__ inline int cvt_floor(float x)
   return r;
 }
 
-// a * b + c for 24-bit unsigned a, b as one V_MAD_U32_U24 (the compiler otherwise forms two
-// multiplies and a three-way add)
+// a * b + c for 24-bit unsigned a and uniform b as one V_MAD_U32_U24 (the compiler otherwise
+// forms two multiplies and a three-way add)
 __device__ inline uint32_t mad_u24(uint32_t a, uint32_t b, uint32_t c)
 {
   uint32_t r;
-  asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
   return r;
 }
 
@@ -88,35 +88,39 @@ __device__ inline uint32_t mad_u24(uint32_t a, uint32_t b, uint32_t c)
 __device__ inline int32_t mad_i24(int32_t a, int32_t b, int32_t c)
 {
   int32_t r;
-  asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
   return r;
 }
 
-// kPadded: the position is already in the padded grid's index frame (FP64 ray set-up), so the
-// element index needs no apron offset: two 24-bit multiply-adds.
+// Element index of the base corner of cell (ix, iy, iz). kPadded: the position was already in the
+// padded grid's index frame (FP64 ray set-up), so no apron offset is needed.
 template <int kFmt, bool kPadded>
-__device__ inline float sample(VolView& v, float x, float y, float z)
+__device__ inline uint32_t element(const VolView& v, int ix, int iy, int iz)
 {
-  // x - floor(x) (V_FRACT_F32) and floor(x) as int: two instructions per axis
-  const float wx = __builtin_amdgcn_fractf(x), wy = __builtin_amdgcn_fractf(y), wz = __builtin_amdgcn_fractf(z);
-  const int ix = cvt_floor(x), iy = cvt_floor(y), iz = cvt_floor(z);
-  // element index of the base corner; ix, iy, iz >= -1 and the pitches < 2^23, so the
-  // signed 24-bit multiply-adds are exact; v.apron = 1 + py + pz shifts past the apron
-  uint32_t e;
-  if constexpr (kFmt == 12 || kFmt == 13) {
+  if constexpr (kFmt == 13) {
     // bricked x-faces: padded cell (ix+1, iy+1, iz+1), brick (./4) in brick order with the
     // brick pitches in py / pz, 5x4x4 faces per brick (x fastest, the last x-face repeated)
     const uint32_t ax = (uint32_t)(kPadded ? ix : ix + 1), ay = (uint32_t)(kPadded ? iy : iy + 1),
                    az = (uint32_t)(kPadded ? iz : iz + 1);
     const uint32_t brick = __umul24(az >> 2, v.pz) + __umul24(ay >> 2, v.py) + (ax >> 2);
     const uint32_t local = __umul24(az & 3u, 20u) + __umul24(ay & 3u, 5u) + (ax & 3u);
-    e = __umul24(brick, (uint32_t)kBrickFaces) + local;
+    return __umul24(brick, (uint32_t)kBrickFaces) + local;
   } else if constexpr (kPadded) {
     // padded indices are >= 0 for every position within a voxel of the index box
-    e = mad_u24((uint32_t)iz, v.pz, mad_u24((uint32_t)iy, v.py, (uint32_t)ix));
+    return mad_u24((uint32_t)iz, v.pz, mad_u24((uint32_t)iy, v.py, (uint32_t)ix));
   } else {
-    e = (uint32_t)mad_i24(iz, (int32_t)v.pz, mad_i24(iy, (int32_t)v.py, ix)) + v.apron;
+    // ix, iy, iz >= -1 and the pitches < 2^23, so the signed 24-bit multiply-adds are exact;
+    // v.apron = 1 + py + pz shifts past the apron
+    return (uint32_t)mad_i24(iz, (int32_t)v.pz, mad_i24(iy, (int32_t)v.py, ix)) + v.apron;
   }
+}
+
+template <int kFmt, bool kPadded>
+__device__ inline float sample(const VolView& v, float x, float y, float z)
+{
+  // x - floor(x) (V_FRACT_F32) and floor(x) as int: two instructions per axis
+  const float wx = __builtin_amdgcn_fractf(x), wy = __builtin_amdgcn_fractf(y), wz = __builtin_amdgcn_fractf(z);
+  const uint32_t e = element<kFmt, kPadded>(v, cvt_floor(x), cvt_floor(y), cvt_floor(z));
   if constexpr (kFmt == 0) {
     const int o = (int)(e * 4u);
     const int oy = (int)(v.py * 4u);
@@ -155,58 +159,6 @@ __device__ inline float sample(VolView& v, float x, float y, float z)
 #pragma unroll
     for (int i = 0; i < 8; ++i) f[i] = (kFmt == 2) ? h2f(r[i]) : bf2f(r[i]);
     return tri(f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7], wx, wy, wz);
-  } else if constexpr (kFmt == 10 || kFmt == 11 || kFmt == 12 || kFmt == 13) {
-    // face layout: faces normal to x at x and x+1 (adjacent 16-byte elements), bilinear in y, z
-    // then linear along x. 11 and 13 keep the faces while the sample stays in its cell; 12 and
-    // 13 read the bricked arrangement.
-    uint4 f0, f1;
-    if constexpr (kFmt == 10 || kFmt == 12) {
-      const auto a = __builtin_amdgcn_raw_buffer_load_b128(v.rsrc, (int)(e * 16u), 0, 0);
-      const auto b = __builtin_amdgcn_raw_buffer_load_b128(v.rsrc, (int)(e * 16u + 16u), 0, 0);
-      f0 = make_uint4(a[0], a[1], a[2], a[3]);
-      f1 = make_uint4(b[0], b[1], b[2], b[3]);
-    } else {
-      if (e != v.ce) {
-        const auto a = __builtin_amdgcn_raw_buffer_load_b128(v.rsrc, (int)(e * 16u), 0, 0);
-        const auto b = __builtin_amdgcn_raw_buffer_load_b128(v.rsrc, (int)(e * 16u + 16u), 0, 0);
-        v.ca = make_uint4(a[0], a[1], a[2], a[3]);
-        v.cb = make_uint4(b[0], b[1], b[2], b[3]);
-        v.ce = e;
-      }
-      f0 = v.ca;
-      f1 = v.cb;
-    }
-    const float p0 = fmaf(wz, fmaf(wy, __uint_as_float(f0.w), __uint_as_float(f0.z)),
-                          fmaf(wy, __uint_as_float(f0.y), __uint_as_float(f0.x)));
-    const float p1 = fmaf(wz, fmaf(wy, __uint_as_float(f1.w), __uint_as_float(f1.z)),
-                          fmaf(wy, __uint_as_float(f1.y), __uint_as_float(f1.x)));
-    return lerp(p0, p1, wx);
-  } else if constexpr (kFmt == 7) {
-    // coefficient layout, fetched only when the sample leaves the previous sample's cell
-    // (about half the samples at half-voxel steps); lanes that stay keep their registers
-    if (e != v.ce) {
-      const uint32_t ob = e * 32u;
-      const auto a = __builtin_amdgcn_raw_buffer_load_b128(v.rsrc, (int)ob, 0, 0);
-      const auto b = __builtin_amdgcn_raw_buffer_load_b128(v.rsrc, (int)(ob + 16u), 0, 0);
-      v.ca = make_uint4(a[0], a[1], a[2], a[3]);
-      v.cb = make_uint4(b[0], b[1], b[2], b[3]);
-      v.ce = e;
-    }
-    const float p0 = fmaf(wy, fmaf(wx, __uint_as_float(v.ca.w), __uint_as_float(v.ca.z)),
-                          fmaf(wx, __uint_as_float(v.ca.y), __uint_as_float(v.ca.x)));
-    const float p1 = fmaf(wy, fmaf(wx, __uint_as_float(v.cb.w), __uint_as_float(v.cb.z)),
-                          fmaf(wx, __uint_as_float(v.cb.y), __uint_as_float(v.cb.x)));
-    return fmaf(wz, p1, p0);
-  } else if constexpr (kFmt == 6) {
-    // trilinear polynomial coefficients of the cell: 2 adjacent 16-byte loads, 7 FMAs
-    const uint32_t ob = e * 32u;
-    const auto a = __builtin_amdgcn_raw_buffer_load_b128(v.rsrc, (int)ob, 0, 0);
-    const auto b = __builtin_amdgcn_raw_buffer_load_b128(v.rsrc, (int)(ob + 16u), 0, 0);
-    const float p0 = fmaf(wy, fmaf(wx, __uint_as_float(a[3]), __uint_as_float(a[2])),
-                          fmaf(wx, __uint_as_float(a[1]), __uint_as_float(a[0])));
-    const float p1 = fmaf(wy, fmaf(wx, __uint_as_float(b[3]), __uint_as_float(b[2])),
-                          fmaf(wx, __uint_as_float(b[1]), __uint_as_float(b[0])));
-    return fmaf(wz, p1, p0);
   } else {
     const int o = (int)(e * 16u);
     const auto q = __builtin_amdgcn_raw_buffer_load_b128(v.rsrc, o, 0, 0);
@@ -232,7 +184,7 @@ __device__ inline float sample(VolView& v, float x, float y, float z)
 // along an axis the ray does not move on. Its positions, start + i*step in float, differ from
 // the sample loop's by far less than the one-voxel dilation. Returns the first sample (in walk
 // order) that may be non-zero.
-__device__ inline int skip_empty(const DrrItem& it, const Ray& r, int i, int end, int dir, float org)
+__device__ __forceinline__ int skip_empty(const DrrItem& it, const Ray& r, int i, int end, int dir, float org)
 {
   const float B = (float)(1 << it.skip_shift), invB = __builtin_ldexpf(1.0f, -it.skip_shift);
   // ray in brick units
@@ -276,7 +228,7 @@ __device__ inline int skip_empty(const DrrItem& it, const Ray& r, int i, int end
 // Sample range [first, last] that can hold non-zero values (SUM with an empty-space map), or
 // the whole ray [0, n]. FP64 set-up rays start in the padded frame (org 1).
 template <int kOp, int kGeom>
-__device__ inline void sample_range(const DrrItem& it, const Ray& r, int& first, int& last)
+__device__ __forceinline__ void sample_range(const DrrItem& it, const Ray& r, int& first, int& last)
 {
   first = 0;
   last = r.n;
@@ -326,6 +278,10 @@ __global__ void drr_setup_kernel(const PoseIn* __restrict__ poses, const VolDesc
   it.cam = cams[p.cam];
   it.vol = v.data;
   it.vol_bytes = v.bytes;
+  it.raw = v.raw;
+  it.raw_bytes = v.raw_bytes;
+  it.raw_py = v.X + 2;
+  it.raw_pz = (v.X + 2) * (v.Y + 2);
   it.X = v.X;
   it.Y = v.Y;
   it.Z = v.Z;
@@ -345,68 +301,189 @@ __global__ void drr_setup_kernel(const PoseIn* __restrict__ poses, const VolDesc
   items[i] = it;
 }
 
-// Samples [i, last] of one ray into acc, in ray order.
-template <int kGeom, int kOp, int kFmt>
-__device__ inline float march(const Ray& ray, VolView& vv, int i, int last, float acc)
+// ---------------------------------------------------------------------------------------
+// marching. A ray's samples 0..n are summed in kSegs segments of seg_len(n) consecutive samples,
+// each segment from zero and the segments' sums in order. The order is a property of the ray, so
+// one lane can march a whole ray (large launches) or several waves can share it (small ones) and
+// every pixel comes out the same bit for bit.
+constexpr int kWindow = 16;
+constexpr int kSegs = 8;
+__device__ inline int seg_len(int n) { return (n + kSegs * kWindow) / (kSegs * kWindow) * kWindow; }
+
+template <int kOp>
+__device__ inline float line_init()
 {
+  return (kOp == XRH_LINE_INT_SUM) ? 0.0f : -3.402823466e+38f;
+}
+
+// Index of the segment that holds sample i (i < 2^23, exact after the correction).
+__device__ inline int seg_of(int i, int seg)
+{
+  int k = (int)((float)i * __builtin_amdgcn_rcpf((float)seg));
+  k -= (k * seg > i) ? 1 : 0;
+  k += ((k + 1) * seg <= i) ? 1 : 0;
+  return k;
+}
+
+// Position of the next sample under FP32 ray set-up: the reference advances by repeated float
+// addition (:276), over samples that are skipped too. (FP64 set-up: start + i * step.)
+struct Pos {
+  float x, y, z;
+  __device__ void advance(const Ray& r, int count)
+  {
+    for (int k = 0; k < count; ++k) {
+      x = x + r.dx;
+      y = y + r.dy;
+      z = z + r.dz;
+    }
+  }
+};
+
+// Two adjacent 16-byte elements: the cell's value at local coordinates (wx, wy, wz).
+template <int kFmt>
+__device__ inline float cell_value(const float (&a)[4], const float (&b)[4], float wx, float wy, float wz)
+{
+  if constexpr (kFmt == 7) {
+    // trilinear polynomial: planes w^0 and w^1
+    const float p0 = fmaf(wy, fmaf(wx, a[3], a[2]), fmaf(wx, a[1], a[0]));
+    const float p1 = fmaf(wy, fmaf(wx, b[3], b[2]), fmaf(wx, b[1], b[0]));
+    return fmaf(wz, p1, p0);
+  } else {
+    // the faces at x and x + 1: bilinear in y, z, then linear along x
+    const float p0 = fmaf(wz, fmaf(wy, a[3], a[2]), fmaf(wy, a[1], a[0]));
+    const float p1 = fmaf(wz, fmaf(wy, b[3], b[2]), fmaf(wy, b[1], b[0]));
+    return lerp(p0, p1, wx);
+  }
+}
+
+// Samples [i, last] of a ray, cell by cell: each iteration fetches the cell of the lane's next
+// sample and evaluates that sample and, if it is in the same cell, the one after it.
+//
+// What bounds the march is the gather: a 16-byte buffer load takes 16.5 clocks of a CU's
+// address/data path however many of the wave's lanes are active (measured, L1 resident), so a
+// loop that steps by samples and loads for the lanes that changed cell pays two loads per sample
+// (at half-voxel steps some lane of 64 always changes). Stepping by cells keeps every lane in
+// every load: about 0.6 pairs of loads per sample. The second sample's local coordinates are the
+// first's plus the step (FP64 set-up), which also saves its index arithmetic; under FP32 set-up
+// they are taken from the reference's own position, whose cell is exact. As unsigned integers
+// the three coordinates' largest is below that of 1.0f exactly when all lie in [0, 1).
+template <int kGeom, int kOp, int kFmt>
+__device__ __forceinline__ float march_cells(const Ray& ray, const VolView& vv, Pos& pos, int i, int last, int seg)
+{
+  float tot = line_init<kOp>(), acc = line_init<kOp>();
+  int seg_last = (seg_of(i, seg) + 1) * seg - 1, win_last = i | (kWindow - 1);
+  float f = (float)i;  // sample indices as floats (exact: n < 2^23)
+  for (;;) {
+    const float fstop = (float)min(win_last, last), fpair = (float)min(seg_last, last);
+    while (f <= fstop) {
+      float x, y, z;
+      if constexpr (kGeom == XRH_GEOM_FP32) {
+        x = pos.x;
+        y = pos.y;
+        z = pos.z;
+      } else {
+        x = fmaf(f, ray.dx, ray.sx);
+        y = fmaf(f, ray.dy, ray.sy);
+        z = fmaf(f, ray.dz, ray.sz);
+      }
+      float wx = __builtin_amdgcn_fractf(x), wy = __builtin_amdgcn_fractf(y), wz = __builtin_amdgcn_fractf(z);
+      const uint32_t e = element<kFmt, kGeom == XRH_GEOM_FP64>(vv, cvt_floor(x), cvt_floor(y), cvt_floor(z));
+      const uint32_t o = e * (kFmt == 7 ? 32u : 16u);
+      const auto la = __builtin_amdgcn_raw_buffer_load_b128(vv.rsrc, (int)o, 0, 0);
+      const auto lb = __builtin_amdgcn_raw_buffer_load_b128(vv.rsrc, (int)(o + 16u), 0, 0);
+      float a[4], b[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        a[k] = __uint_as_float(la[k]);
+        b[k] = __uint_as_float(lb[k]);
+      }
+      acc = line_op<kOp>(acc, cell_value<kFmt>(a, b, wx, wy, wz));
+      f = f + 1.0f;
+      if constexpr (kGeom == XRH_GEOM_FP32) {
+        const float bx = x - wx, by = y - wy, bz = z - wz;  // floor
+        pos.advance(ray, 1);
+        wx = pos.x - bx;
+        wy = pos.y - by;
+        wz = pos.z - bz;
+      } else {
+        wx = wx + ray.dx;
+        wy = wy + ray.dy;
+        wz = wz + ray.dz;
+      }
+      const uint32_t top = max(max(__float_as_uint(wx), __float_as_uint(wy)), __float_as_uint(wz));
+      if (top < 0x3f800000u && f <= fpair) {
+        acc = line_op<kOp>(acc, cell_value<kFmt>(a, b, wx, wy, wz));
+        f = f + 1.0f;
+        if constexpr (kGeom == XRH_GEOM_FP32) pos.advance(ray, 1);
+      }
+    }
+    const bool done = win_last >= last;
+    if (done || win_last >= seg_last) {
+      tot = line_op<kOp>(tot, acc);
+      acc = line_init<kOp>();
+      seg_last += seg;
+    }
+    if (done) break;
+    win_last += kWindow;
+  }
+  return tot;
+}
+
+// Samples [i, last] of one segment, two per iteration, each with its own loads.
+template <int kGeom, int kOp, int kFmt>
+__device__ __forceinline__ float march_samples(const Ray& ray, const VolView& vv, Pos& pos, int i, int last)
+{
+  float acc = line_init<kOp>();
   if constexpr (kGeom == XRH_GEOM_FP32) {
-    // positions advance by repeated float addition, as the reference does (:276),
-    // including over the leading samples that are skipped
-    float px = ray.sx, py = ray.sy, pz = ray.sz;
-    if (i <= last) {
-      for (int k = 0; k < i; ++k) {
-        px = px + ray.dx;
-        py = py + ray.dy;
-        pz = pz + ray.dz;
-      }
+    for (; i < last; i += 2) {
+      const float qx = pos.x + ray.dx, qy = pos.y + ray.dy, qz = pos.z + ray.dz;
+      const float s0 = sample<kFmt, false>(vv, pos.x, pos.y, pos.z);
+      const float s1 = sample<kFmt, false>(vv, qx, qy, qz);
+      acc = line_op<kOp>(line_op<kOp>(acc, s0), s1);
+      pos.x = qx + ray.dx;
+      pos.y = qy + ray.dy;
+      pos.z = qz + ray.dz;
     }
-    if constexpr (kFmt == 7 || kFmt == 11 || kFmt == 13) {
-      // one sample per iteration: the cell cache lives in fixed registers; the count runs
-      // in float (exact below 2^24) so the loop test is one float compare
-      const float flast = (float)last;
-      for (float fi = (float)i; fi <= flast; fi = fi + 1.0f) {
-        acc = line_op<kOp>(acc, sample<kFmt, false>(vv, px, py, pz));
-        px = px + ray.dx;
-        py = py + ray.dy;
-        pz = pz + ray.dz;
-      }
-    } else {
-      for (; i < last; i += 2) {
-        const float qx = px + ray.dx, qy = py + ray.dy, qz = pz + ray.dz;
-        const float s0 = sample<kFmt, false>(vv, px, py, pz);
-        const float s1 = sample<kFmt, false>(vv, qx, qy, qz);
-        acc = line_op<kOp>(line_op<kOp>(acc, s0), s1);
-        px = qx + ray.dx;
-        py = qy + ray.dy;
-        pz = qz + ray.dz;
-      }
-      if (i == last) acc = line_op<kOp>(acc, sample<kFmt, false>(vv, px, py, pz));
-    }
-  } else if constexpr (kFmt == 7 || kFmt == 11 || kFmt == 13) {
-    const float flast = (float)last;
-    for (float f0 = (float)i; f0 <= flast; f0 = f0 + 1.0f) {
-      acc = line_op<kOp>(acc, sample<kFmt, true>(vv, fmaf(f0, ray.dx, ray.sx), fmaf(f0, ray.dy, ray.sy),
-                                              fmaf(f0, ray.dz, ray.sz)));
+    if (i == last) {
+      acc = line_op<kOp>(acc, sample<kFmt, false>(vv, pos.x, pos.y, pos.z));
+      pos.advance(ray, 1);
     }
   } else {
-    // sample indices as floats (exact: n < 2^24), advanced by float additions
+    // sample indices as floats (exact: n < 2^23), advanced by float additions
     float f0 = (float)i;
     for (; i < last; i += 2) {
       const float f1 = f0 + 1.0f;
       const float s0 = sample<kFmt, true>(vv, fmaf(f0, ray.dx, ray.sx), fmaf(f0, ray.dy, ray.sy),
-                                    fmaf(f0, ray.dz, ray.sz));
+                                          fmaf(f0, ray.dz, ray.sz));
       const float s1 = sample<kFmt, true>(vv, fmaf(f1, ray.dx, ray.sx), fmaf(f1, ray.dy, ray.sy),
-                                    fmaf(f1, ray.dz, ray.sz));
+                                          fmaf(f1, ray.dz, ray.sz));
       acc = line_op<kOp>(line_op<kOp>(acc, s0), s1);
       f0 = f0 + 2.0f;
     }
     if (i == last) {
-      const float f0 = (float)i;
       acc = line_op<kOp>(acc, sample<kFmt, true>(vv, fmaf(f0, ray.dx, ray.sx), fmaf(f0, ray.dy, ray.sy),
-                                              fmaf(f0, ray.dz, ray.sz)));
+                                                 fmaf(f0, ray.dz, ray.sz)));
     }
   }
   return acc;
+}
+
+// Samples [i, last] (i <= last) of one ray, summed segment by segment. `pos`: sample i's position
+// under FP32 set-up; it ends past sample `last`.
+template <int kGeom, int kOp, int kFmt>
+__device__ __forceinline__ float march(const Ray& ray, const VolView& vv, Pos& pos, int i, int last, int seg)
+{
+  if constexpr (is_cell_fmt(kFmt)) {
+    return march_cells<kGeom, kOp, kFmt>(ray, vv, pos, i, last, seg);
+  } else {
+    float tot = line_init<kOp>();
+    for (int end = (seg_of(i, seg) + 1) * seg - 1; i <= last; end += seg) {
+      const int stop = min(end, last);
+      tot = line_op<kOp>(tot, march_samples<kGeom, kOp, kFmt>(ray, vv, pos, i, stop));
+      i = stop + 1;
+    }
+    return tot;
+  }
 }
 
 // The fused NCC epilogue: FP64 sums of m, m^2 and m * zero-mean fixed over the tile, one
@@ -429,7 +506,7 @@ __device__ inline void ncc_epilogue(const DrrItem& it, const TileRef& tr, bool i
     sf = wave_sum_d(sf);
     __shared__ double red[4][3];
     const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
+    if ((threadIdx.x & 63) == 0 && w < 4) {
       red[w][0] = s1;
       red[w][1] = s2;
       red[w][2] = sf;
@@ -463,6 +540,16 @@ __device__ inline void store_pixel(const DrrItem& it, const TileRef& tr, bool in
   ncc_epilogue(it, tr, inside, col, row, pix, ncc_partials, ncc_tiles);
 }
 
+__device__ inline VolView vol_view(const DrrItem& it)
+{
+  VolView vv;
+  vv.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(it.vol), (short)0, (int)it.vol_bytes, 0x00020000);
+  vv.py = it.pitch_y;
+  vv.pz = it.pitch_z;
+  vv.apron = 1u + it.pitch_y + it.pitch_z;
+  return vv;
+}
+
 // One ray of one item: the line integral (SUM) or maximum (MAX) of its samples times the step,
 // or the kernel's initial value when the ray misses the volume. Called by every lane of the
 // wave (`inside` false for lanes past the detector edge), so that the lanes can agree on a
@@ -472,41 +559,421 @@ __device__ inline void store_pixel(const DrrItem& it, const TileRef& tr, bool in
 // nearly the same depth, then fetch the same cells in the same iteration (C2: L1 tag accesses
 // -7.5%, L1 tag-conflict stalls -40%, DRR -2%).
 template <int kGeom, int kOp, int kFmt>
-__device__ inline float cast_ray(const DrrItem& it, int col, int row, bool inside)
+__device__ __forceinline__ float cast_range(const DrrItem& it, const Ray& ray, int i, int last)
 {
-  float acc = (kOp == XRH_LINE_INT_SUM) ? 0.0f : -3.402823466e+38f;
-  Ray ray;
-  ray.n = -1;
-  int i = 0, last = -1;
-  if (inside) {
-    ray = (kGeom == XRH_GEOM_FP32) ? setup_ray_f32(it, (float)col, (float)row) : setup_ray_f64(it, col, row);
-    if (ray.n >= 0) sample_range<kOp, kGeom>(it, ray, i, last);
-  }
+  float acc = line_init<kOp>();
   // wave minimum of the first samples of the lanes with samples (all lanes take part)
   int start = (i <= last) ? i : 0x7fffffff;
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) start = min(start, __shfl_xor(start, off, 64));
   if (ray.n >= 0) {
     if (i <= last) {
-      VolView vv;
-      vv.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(it.vol), (short)0,
-                                                  (int)it.vol_bytes, 0x00020000);
-      vv.py = it.pitch_y;
-      vv.pz = it.pitch_z;
-      vv.apron = 1u + it.pitch_y + it.pitch_z;
-      vv.ce = 0xFFFFFFFFu;
-      acc = march<kGeom, kOp, kFmt>(ray, vv, start, last, acc);
+      Pos pos{ray.sx, ray.sy, ray.sz};
+      if constexpr (kGeom == XRH_GEOM_FP32) pos.advance(ray, start);
+      acc = march<kGeom, kOp, kFmt>(ray, vol_view(it), pos, start, last, seg_len(ray.n));
     }
     acc = acc * it.step;
   }
   return acc;
 }
 
+// Ray set-up and sample range of a pixel ([0, -1] and n = -1 for none).
+template <int kGeom, int kOp>
+__device__ __forceinline__ Ray begin_ray(const DrrItem& it, int col, int row, bool inside, int& first, int& last)
+{
+  Ray ray;
+  ray.n = -1;
+  first = 0;
+  last = -1;
+  if (inside) {
+    ray = (kGeom == XRH_GEOM_FP32) ? setup_ray_f32(it, (float)col, (float)row) : setup_ray_f64(it, col, row);
+    if (ray.n >= 0) sample_range<kOp, kGeom>(it, ray, first, last);
+  }
+  return ray;
+}
+
 template <int kGeom, int kOp, int kFmt>
-__global__ __launch_bounds__(kThreads) void drr_kernel(
+__device__ __forceinline__ float cast_ray(const DrrItem& it, int col, int row, bool inside)
+{
+  int first, last;
+  const Ray ray = begin_ray<kGeom, kOp>(it, col, row, inside, first, last);
+  return cast_range<kGeom, kOp, kFmt>(it, ray, first, last);
+}
+
+// ---------------------------------------------------------------------------------------
+// slab marching. The gathering march is bound by the per-lane fetch path: 16.5 clocks of a CU per
+// 16-byte load, more when its lanes touch more cache lines, and an L1 (32 KB for 32 waves) that
+// holds none of them until the next layer when neighbouring rays are a voxel or more apart (96 x
+// 96 rays over 256 x 256 x 200 voxels: L1 hits 49%, 5 TB/s of fabric traffic, VALU 12%). Here a
+// workgroup moves through the volume slab by slab along the tile's main axis: the box of voxels
+// that its 256 rays can reach in the next few layers is loaded into LDS once, as plain 4-byte
+// voxels (a quarter of the face layout's bytes), 16 bytes per lane straight from the buffer load,
+// and the rays take their cells from there. LDS serves a 64-lane read of two neighbouring voxels
+// in about 5 clocks whatever lines they share, so lanes also need not stay in step.
+//
+// The box comes from the tile's corner rays: the pixel -> position map on a plane across the main
+// axis is projective, so the corners' positions on the slab's two planes bound every ray between
+// them. Slabs end on cell faces, so no cell straddles two. A cell's face coefficients are formed
+// from its voxels by the float operations that built the face layout, and samples pair and
+// segment as in march_cells: the values are the gathering march's bit for bit, and tiles whose box
+// does not fit (rays several voxels apart, oblique tiles) take that march.
+//
+// Measured, FP64 set-up, ns per ray, gathering sample by sample (before) / by cells / slabs: 256 x
+// 256 x 200 voxels at 0.39 voxels between rays 0.412 / 0.355 / 0.330, 0.78: 0.582 / 0.644 / 0.427,
+// 1.55: 1.33 / 1.53 / 1.01; 512 x 512 x 400 voxels at 0.39: 0.942 / 0.748 / 0.554, 0.78: 1.16 / 1.69
+// / 0.746, 1.55: 3.5 / 3.8 / 1.79. Layers per slab:
+// 8 / 12 / 16 at 0.39: 0.386 / 0.351 / 0.353; along x one 64-byte row of 16 voxels.
+constexpr int kSlabDepth = 12, kSlabDepthX = 15;
+
+// One axis of a 3-vector by a uniform index.
+template <class T>
+__device__ inline T pick(int axis, T x, T y, T z)
+{
+  return axis == 0 ? x : (axis == 1 ? y : z);
+}
+
+__device__ inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// v from another lane of the row by a DPP control word
+template <int kCtrl>
+__device__ inline float dpp(float v)
+{
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xf, 0xf, true));
+}
+
+// A box of voxels in LDS: voxel (x, y, z) of the padded grid at x - x0 + sy (y - y0) + sz (z - z0).
+struct Box {
+  int x0, y0, z0, wx, wy, wz;
+  int lpr, rows;  // lanes per row (16 bytes each) and rows per load
+  int sy, sz;
+  __device__ int floats() const { return sz * wz; }
+  __device__ void pitch()
+  {
+    lpr = (wx + 3) >> 2;
+    rows = 64 / lpr;
+    sy = 4 * lpr;
+    sz = sy * wy;
+  }
+};
+
+// Loads the box from the padded voxels (pitches py, pz), 16 bytes per lane straight into LDS, as
+// many rows of one z as fit per instruction (a row's last lane may overhang into its padding).
+__device__ inline void stage_box(__amdgpu_buffer_rsrc_t src, const Box& b, uint32_t py, uint32_t pz, float* lds)
+{
+  const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6);
+  const int sub = lane / b.lpr;
+  const uint32_t lane_off = ((uint32_t)sub * py + (uint32_t)(lane - sub * b.lpr) * 4u) * 4u;
+  const int groups = (b.wy + b.rows - 1) / b.rows;
+  int z = 0, g = wave;
+  while (g >= groups) {
+    g -= groups;
+    ++z;
+  }
+  while (z < b.wz) {
+    const uint32_t row = (uint32_t)(b.z0 + z) * pz + (uint32_t)(b.y0 + g * b.rows) * py + (uint32_t)b.x0;
+    float* dst = lds + z * b.sz + g * b.rows * b.sy;
+    if (sub < min(b.rows, b.wy - g * b.rows)) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)dst, 16,
+                                               (int)(lane_off + row * 4u), 0, 0, 0);
+    }
+    g += kThreads / 64;
+    while (g >= groups) {
+      g -= groups;
+      ++z;
+    }
+  }
+}
+
+struct LdsPair {
+  float a, b;
+};
+// Two consecutive floats at an LDS byte address (one DS_READ2_B32).
+__device__ inline LdsPair lds_pair(int addr)
+{
+  const auto* p = (const __attribute__((address_space(3))) float*)(uintptr_t)(uint32_t)addr;
+  return {p[0], p[1]};
+}
+
+// cast_ray by slabs. Every thread of the block calls it (it synchronises); `lds` holds `budget`
+// floats.
+template <int kGeom, int kOp>
+__device__ __forceinline__ float cast_ray_slab(const DrrItem& it, const TileRef& tr, int col, int row, bool inside,
+                                      float* lds, int budget)
+{
+  __shared__ float corner[4][3];
+  __shared__ float origin[3];
+  __shared__ float reach[3][4];
+
+  int first, last;
+  const Ray ray = begin_ray<kGeom, kOp>(it, col, row, inside, first, last);
+  const int tid = threadIdx.x, lane = tid & 63;
+  if (tid < 4) {
+    // the lines through the tile's corner pixels, padded index frame
+    double det[3], ph[3], dp[3];
+    ind_to_det_d(it.cam, (double)(tr.tx * kTile + (tid & 1) * (kTile - 1)),
+                 (double)(tr.ty * kTile + (tid >> 1) * (kTile - 1)), det);
+    affine_pt_d(it.Md, it.cam.pinhole_d, ph);
+    affine_pt_d(it.Md, det, dp);
+    for (int k = 0; k < 3; ++k) {
+      corner[tid][k] = (float)(dp[k] - ph[k]);
+      if (tid == 0) origin[k] = (float)(ph[k] + 1.0);
+    }
+  }
+  __syncthreads();
+  // main axis of the tile: the largest component of its middle direction
+  const float mx = corner[0][0] + corner[3][0], my = corner[0][1] + corner[3][1], mz = corner[0][2] + corner[3][2];
+  const int A = uni((fabsf(mx) >= fabsf(my) && fabsf(mx) >= fabsf(mz)) ? 0 : (fabsf(my) >= fabsf(mz) ? 1 : 2));
+  const int B = A == 0 ? 1 : 0, C = A == 2 ? 1 : 2;
+  const bool up = uni(pick(A, mx, my, mz) > 0.0f ? 1 : 0) != 0;
+  bool ok = it.raw != nullptr;
+  for (int k = 0; k < 4; ++k) {
+    const float d = up ? corner[k][A] : -corner[k][A];
+    ok = ok && d > 0.0f && 2.0f * d >= fabsf(corner[k][B]) && 2.0f * d >= fabsf(corner[k][C]);
+  }
+  // this lane's line of the hull: corner lane & 3, axis B or C, as position = u + v * (position on A)
+  const int hk = lane & 3, hax = (lane & 8) ? C : B;
+  const float hv = corner[hk][hax] / corner[hk][A], hu = origin[hax] - origin[A] * hv;
+  // the cells along A that the block's samples reach. The margin covers the rounding of the lines
+  // and the samples; under FP32 set-up also the samples' drift, at most one rounding per addition.
+  constexpr float kOff = (kGeom == XRH_GEOM_FP64) ? 0.0f : 1.0f;
+  const float sA = pick(A, ray.sx, ray.sy, ray.sz), dA = pick(A, ray.dx, ray.dy, ray.dz);
+  float lo = 3.0e38f, hi = -3.0e38f, margin = 0.05f;
+  if (first <= last) {
+    if (kGeom == XRH_GEOM_FP32) margin = fmaf((float)last * (float)max(max(it.X, it.Y), it.Z), 6.0e-8f, margin);
+    const float p0 = fmaf((float)first, dA, sA) + kOff, p1 = fmaf((float)last, dA, sA) + kOff;
+    lo = fminf(p0, p1);
+    hi = fmaxf(p0, p1);
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    lo = fminf(lo, __shfl_xor(lo, off, 64));
+    hi = fmaxf(hi, __shfl_xor(hi, off, 64));
+    if (kGeom == XRH_GEOM_FP32) margin = fmaxf(margin, __shfl_xor(margin, off, 64));
+  }
+  if (lane == 0) {
+    reach[0][tid >> 6] = lo;
+    reach[1][tid >> 6] = hi;
+    reach[2][tid >> 6] = margin;
+  }
+  __syncthreads();
+  lo = fminf(fminf(reach[0][0], reach[0][1]), fminf(reach[0][2], reach[0][3]));
+  hi = fmaxf(fmaxf(reach[1][0], reach[1][1]), fmaxf(reach[1][2], reach[1][3]));
+  if (kGeom == XRH_GEOM_FP32) margin = fmaxf(fmaxf(reach[2][0], reach[2][1]), fmaxf(reach[2][2], reach[2][3]));
+  const int nA = pick(A, it.X, it.Y, it.Z), nB = pick(B, it.X, it.Y, it.Z), nC = pick(C, it.X, it.Y, it.Z);
+  const bool any = uni(lo <= hi ? 1 : 0) != 0;
+  const int alo = uni(any ? min(max((int)floorf(lo - margin), 0), nA) : 0);
+  const int ahi = uni(any ? min(max((int)floorf(hi + margin), 0), nA) : -1);
+  const int total = ahi - alo + 1;
+  // the box of cells [a, a + n) along A. `whole`: not cut at the volume's faces (for its size), and
+  // one voxel wider per axis.
+  auto box_of = [&](int a, int n, bool whole) {
+    const float v = fmaf((float)((lane & 4) ? a + n : a), hv, hu);
+    float l = fminf(v, dpp<0xB1>(v)), h = fmaxf(v, dpp<0xB1>(v));  // lanes ^ 1
+    l = fminf(l, dpp<0x4E>(l));                                    // lanes ^ 2
+    h = fmaxf(h, dpp<0x4E>(h));
+    l = fminf(l, dpp<0x141>(l));                                   // the other half of 8 lanes
+    h = fmaxf(h, dpp<0x141>(h));
+    const int il = (int)floorf(__builtin_amdgcn_fmed3f(l - margin, -1.0e6f, 1.0e6f));
+    const int ih = (int)floorf(__builtin_amdgcn_fmed3f(h + margin, -1.0e6f, 1.0e6f)) + 1;
+    const int lb = __builtin_amdgcn_readlane(il, 0), hb = __builtin_amdgcn_readlane(ih, 0);
+    const int lc = __builtin_amdgcn_readlane(il, 8), hc = __builtin_amdgcn_readlane(ih, 8);
+    const int b0 = min(max(lb, 0), nB), b1 = min(max(hb, 1), nB + 1);
+    const int c0 = min(max(lc, 0), nC), c1 = min(max(hc, 1), nC + 1);
+    const int wb = whole ? min(hb - lb + 2, nB + 2) : b1 - b0 + 1, wc = whole ? min(hc - lc + 2, nC + 2) : c1 - c0 + 1;
+    Box b;
+    b.x0 = A == 0 ? a : b0;
+    b.wx = A == 0 ? n + 1 : wb;
+    b.y0 = A == 1 ? a : (A == 0 ? b0 : c0);
+    b.wy = A == 1 ? n + 1 : (A == 0 ? wb : wc);
+    b.z0 = A == 2 ? a : c0;
+    b.wz = A == 2 ? n + 1 : wc;
+    b.wx = max(b.wx, 2);
+    b.wy = max(b.wy, 2);
+    b.wz = max(b.wz, 2);
+    b.pitch();
+    return b;
+  };
+  // the most cells per slab whose box fits at both ends (the uncut widths are convex along A)
+  int depth = 0;
+  if (any && __builtin_amdgcn_readfirstlane(__all(ok && margin < 1.0f) ? 1 : 0)) {
+    for (depth = (A == 0) ? kSlabDepthX : kSlabDepth; depth >= 1; depth = (depth >= 8) ? depth - 1 : depth >> 1) {
+      const int n = min(depth, total);
+      const Box b0 = box_of(alo, n, true), b1 = box_of(ahi + 1 - n, n, true);
+      if (b0.wx <= 256 && b1.wx <= 256 && b0.floats() <= budget && b1.floats() <= budget) break;
+    }
+  }
+  if (depth < 2) return cast_range<kGeom, kOp, 11>(it, ray, first, last);
+
+  const auto src = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(it.raw), (short)0, (int)it.raw_bytes, 0x00020000);
+  const float flast = (float)last, fseg_len = (float)seg_len(ray.n);
+  float f = (first <= last) ? (float)first : flast + 1.0f;
+  float fseg = 0.0f;
+  float tot = line_init<kOp>(), acc = line_init<kOp>();
+  Pos pos{ray.sx, ray.sy, ray.sz};
+  const float qs = up ? sA : -sA, qd = up ? dA : -dA, qr = __builtin_amdgcn_rcpf(qd);
+  const int lds_addr = (int)(uintptr_t)(__attribute__((address_space(3))) float*)lds;
+  float q = fmaf(f, qd, qs);
+  if (first <= last) {
+    const int seg = seg_len(ray.n);
+    fseg = fminf((float)((seg_of(first, seg) + 1) * seg - 1), flast);
+    if constexpr (kGeom == XRH_GEOM_FP32) {
+      pos.advance(ray, first);
+      q = up ? pick(A, pos.x, pos.y, pos.z) : -pick(A, pos.x, pos.y, pos.z);
+    }
+  }
+  for (int t = 0; t < total;) {
+    const int n = min(depth, total - t), a = up ? alo + t : ahi + 1 - t - n;
+    const Box b = box_of(a, n, false);
+    __syncthreads();  // the previous slab has been read
+    stage_box(src, b, it.raw_py, it.raw_pz, lds);
+    asm volatile("s_waitcnt vmcnt(0)");
+    __syncthreads();
+    // samples of the slab: q below its far face, as one comparison
+    const float face = up ? (float)(a + n) - kOff : -((float)a - kOff);
+    const float lim = up ? (face > 0.0f ? __uint_as_float(__float_as_uint(face) - 1u) : -1.0e-30f) : face;
+    float fslab = flast;
+    if constexpr (kGeom == XRH_GEOM_FP64) {
+      // the last of them: an estimate within one sample, corrected with the samples' own positions
+      fslab = floorf((lim - qs) * qr);
+      if (fmaf(fslab + 1.0f, qd, qs) <= lim) fslab = fslab + 1.0f;
+      if (fmaf(fslab, qd, qs) > lim) fslab = fslab - 1.0f;
+      fslab = fminf(fslab, flast);
+    }
+    // LDS byte address of cell (0, 0, 0), row and slice pitch
+    const int py = b.sy * 4, pz = b.sz * 4;
+    int base = lds_addr + (int)kOff * (4 + py + pz) - (b.x0 * 4 + py * b.y0 + pz * b.z0);
+    asm("" : "+s"(base));  // one value: the compiler would subtract x0 per sample
+    for (;;) {
+      const float fstop = fminf(fslab, fseg);
+      while (f <= fstop && (kGeom == XRH_GEOM_FP64 || q <= lim)) {
+        float x, y, z;
+        if constexpr (kGeom == XRH_GEOM_FP32) {
+          x = pos.x;
+          y = pos.y;
+          z = pos.z;
+        } else {
+          x = fmaf(f, ray.dx, ray.sx);
+          y = fmaf(f, ray.dy, ray.sy);
+          z = fmaf(f, ray.dz, ray.sz);
+        }
+        float wx = __builtin_amdgcn_fractf(x), wy = __builtin_amdgcn_fractf(y), wz = __builtin_amdgcn_fractf(z);
+        const int c00 = mad_i24(cvt_floor(z), pz, mad_i24(cvt_floor(y), py, (cvt_floor(x) << 2) + base));
+        const int c10 = c00 + py, c01 = c00 + pz, c11 = c10 + pz;
+        float va[4], vb[4];
+        const LdsPair r00 = lds_pair(c00), r10 = lds_pair(c10), r01 = lds_pair(c01), r11 = lds_pair(c11);
+        va[0] = r00.a;
+        vb[0] = r00.b;
+        va[1] = r10.a - r00.a;
+        vb[1] = r10.b - r00.b;
+        va[2] = r01.a - r00.a;
+        vb[2] = r01.b - r00.b;
+        va[3] = (r11.a - r01.a) - va[1];
+        vb[3] = (r11.b - r01.b) - vb[1];
+        acc = line_op<kOp>(acc, cell_value<11>(va, vb, wx, wy, wz));
+        f = f + 1.0f;
+        if constexpr (kGeom == XRH_GEOM_FP32) {
+          const float bx = x - wx, by = y - wy, bz = z - wz;  // floor
+          pos.advance(ray, 1);
+          q = q + qd;
+          wx = pos.x - bx;
+          wy = pos.y - by;
+          wz = pos.z - bz;
+        } else {
+          wx = wx + ray.dx;
+          wy = wy + ray.dy;
+          wz = wz + ray.dz;
+        }
+        const uint32_t top = max(max(__float_as_uint(wx), __float_as_uint(wy)), __float_as_uint(wz));
+        if (top < 0x3f800000u && f <= fseg) {
+          acc = line_op<kOp>(acc, cell_value<11>(va, vb, wx, wy, wz));
+          f = f + 1.0f;
+          if constexpr (kGeom == XRH_GEOM_FP32) {
+            pos.advance(ray, 1);
+            q = q + qd;
+          }
+        }
+      }
+      // a lane that reached the end of its segment goes on to the next one in this slab
+      const bool roll = f > fseg && f <= flast;
+      if (f > fseg) {
+        tot = line_op<kOp>(tot, acc);
+        acc = line_init<kOp>();
+        fseg = (f > flast) ? 3.0e38f : fminf(fseg + fseg_len, flast);
+      }
+      if (!__any(roll)) break;
+    }
+    t += n;
+  }
+  return (ray.n >= 0) ? tot * it.step : line_init<kOp>();
+}
+
+// The same ray shared by kParts waves of a workgroup of kParts * 256 threads (thread t: pixel
+// t % 256, part t / 256): part p sums segments p, p + kParts, ... and every part adds all
+// segments in order, so the value is cast_ray's bit for bit. The first two parts walk over the
+// empty space from one end each. Every thread of the block calls it (it synchronises).
+template <int kGeom, int kOp, int kFmt, int kParts>
+__device__ __forceinline__ float cast_ray_split(const DrrItem& it, int col, int row, bool inside)
+{
+  static_assert(kParts >= 2 && kSegs % kParts == 0, "segments are dealt evenly");
+  __shared__ float sums[kSegs][kThreads];
+  __shared__ int ends[2][kThreads];
+  const int px = threadIdx.x & (kThreads - 1), part = threadIdx.x / kThreads;
+  Ray ray;
+  ray.n = -1;
+  if (inside) {
+    ray = (kGeom == XRH_GEOM_FP32) ? setup_ray_f32(it, (float)col, (float)row) : setup_ray_f64(it, col, row);
+  }
+  const bool skip = kOp == XRH_LINE_INT_SUM && it.skip;
+  int first = 0, last = ray.n;
+  if (skip) {
+    const float org = (kGeom == XRH_GEOM_FP64) ? 1.0f : 0.0f;
+    if (part == 0) ends[0][px] = (ray.n >= 0) ? skip_empty(it, ray, 0, ray.n, 1, org) : 0;
+    if (part == 1) ends[1][px] = (ray.n >= 0) ? skip_empty(it, ray, ray.n, 0, -1, org) : -1;
+    __syncthreads();
+    first = ends[0][px];
+    last = ends[1][px];
+  }
+  const int seg = seg_len(ray.n);
+  Pos pos{ray.sx, ray.sy, ray.sz};
+  int at = 0;
+#pragma clang loop unroll(disable)
+  for (int k = part; k < kSegs; k += kParts) {
+    const int i = max(first, k * seg), stop = min(last, k * seg + seg - 1);
+    float acc = line_init<kOp>();
+    if (i <= stop) {
+      if constexpr (kGeom == XRH_GEOM_FP32) pos.advance(ray, i - at);
+      acc = march<kGeom, kOp, kFmt>(ray, vol_view(it), pos, i, stop, seg);
+      at = stop + 1;
+    }
+    sums[k][px] = acc;
+  }
+  __syncthreads();
+  float acc = line_init<kOp>();
+  if (ray.n >= 0) {
+#pragma unroll
+    for (int k = 0; k < kSegs; ++k) acc = line_op<kOp>(acc, sums[k][px]);
+    acc = acc * it.step;
+  }
+  __syncthreads();  // the next object's cast reuses the shared arrays
+  return acc;
+}
+
+// kParts: the waves that share a ray, 0 for slab marching with `budget` floats of dynamic LDS.
+template <int kGeom, int kOp, int kFmt, int kParts>
+__device__ __forceinline__ float cast_pixel(const DrrItem& it, const TileRef& tr, int col, int row, bool inside, int budget)
+{
+  if constexpr (kParts == 0) {
+    extern __shared__ __attribute__((aligned(16))) float slab_lds[];
+    return cast_ray_slab<kGeom, kOp>(it, tr, col, row, inside, slab_lds, budget);
+  } else if constexpr (kParts == 1) return cast_ray<kGeom, kOp, kFmt>(it, col, row, inside);
+  else return cast_ray_split<kGeom, kOp, kFmt, kParts>(it, col, row, inside);
+}
+
+template <int kGeom, int kOp, int kFmt, int kParts>
+__global__ __launch_bounds__(kThreads * (kParts > 1 ? kParts : 1), kParts == 0 ? 4 : 8) void drr_kernel(
     const DrrItem* __restrict__ items, const uint32_t* __restrict__ band_start, int64_t num_items,
     int bands, float* __restrict__ out, int accumulate, float fill,
-    double* __restrict__ ncc_partials, int ncc_tiles, int shape)
+    double* __restrict__ ncc_partials, int ncc_tiles, int shape, int budget)
 {
   const TileRef tr = decode_tile(band_start, num_items, bands, items);
   if (!tr.valid) return;
@@ -514,8 +981,10 @@ __global__ __launch_bounds__(kThreads) void drr_kernel(
   int col, row;
   lane_pixel(tr.tx, tr.ty, shape, col, row);
   const bool inside = (col < it.cam.cols) && (row < it.cam.rows);
-  const float acc = cast_ray<kGeom, kOp, kFmt>(it, col, row, inside);
-  store_pixel<kOp>(it, tr, inside, col, row, acc, out, accumulate, fill, ncc_partials, ncc_tiles);
+  const float acc = cast_pixel<kGeom, kOp, kFmt, kParts>(it, tr, col, row, inside, budget);
+  // the first part stores the pixels
+  const bool mine = inside && (kParts <= 1 || threadIdx.x < kThreads);
+  store_pixel<kOp>(it, tr, mine, col, row, acc, out, accumulate, fill, ncc_partials, ncc_tiles);
 }
 
 // Several objects per item (Intensity2D3DRegi::obj_fn with more than one volume,
@@ -524,11 +993,11 @@ __global__ __launch_bounds__(kThreads) void drr_kernel(
 // others added with the line kernel -- per pixel the same float operations as one REPLACE
 // launch followed by ACCUM launches. The item's first entry carries the output offset, the
 // detector and the fused NCC reference.
-template <int kGeom, int kOp, int kFmt>
-__global__ __launch_bounds__(kThreads) void drr_objects_kernel(
+template <int kGeom, int kOp, int kFmt, int kParts>
+__global__ __launch_bounds__(kThreads * (kParts > 1 ? kParts : 1), kParts == 0 ? 4 : 8) void drr_objects_kernel(
     const DrrItem* __restrict__ items, const uint32_t* __restrict__ band_start, int64_t num_items,
     int bands, float* __restrict__ out, float fill, double* __restrict__ ncc_partials, int ncc_tiles,
-    int shape, int objs)
+    int shape, int budget, int objs)
 {
   const TileRef tr = decode_tile(band_start, num_items, bands, items, objs);
   if (!tr.valid) return;
@@ -540,13 +1009,15 @@ __global__ __launch_bounds__(kThreads) void drr_objects_kernel(
   float pix = 0.0f;
   if (inside) pix = it0.bg ? it0.bg[px] : fill;
   for (int k = 0; k < objs; ++k) {
-    const float aa = 0.0f + cast_ray<kGeom, kOp, kFmt>(items[tr.item * objs + k], col, row, inside) * 1.0f;
+    const float aa = 0.0f + cast_pixel<kGeom, kOp, kFmt, kParts>(items[tr.item * objs + k], tr, col, row, inside, budget) * 1.0f;
     if (inside) {
       if constexpr (kOp == XRH_LINE_INT_SUM) pix = pix + aa; else pix = (pix < aa) ? aa : pix;
     }
+    if constexpr (kParts == 0) __syncthreads();  // the next cast reuses the shared arrays
   }
-  if (inside) out[it0.out_off + px] = pix;
-  ncc_epilogue(it0, tr, inside, col, row, pix, ncc_partials, ncc_tiles);
+  const bool mine = inside && (kParts <= 1 || threadIdx.x < kThreads);
+  if (mine) out[it0.out_off + px] = pix;
+  ncc_epilogue(it0, tr, mine, col, row, pix, ncc_partials, ncc_tiles);
 }
 
 template <int kGeom>
@@ -592,38 +1063,60 @@ int device_cus()
   return cache[dev];
 }
 
+// Waves that share a ray in a launch of `tiles` workgroups: the most for which all of them are
+// resident at once (32 waves per CU). A launch of few rays is bound by the longest rays' chain of
+// dependent gathers and by idle CUs, which sharing shortens and fills; one that fills the GPU
+// only pays for the shared set-up (30 items of 256 x 256, two objects: 1.07 ms whole, 1.22 ms by
+// two). One pose, FP64 set-up, DRR kernel: 192 x 192 over 128 x 128 x 96 voxels 30.5
+// whole, 27.2 by two, 21.4 by four; 384 x 384 over 256 x 256 x 200 voxels 102, 80, 90 us.
+int drr_parts(int64_t tiles)
+{
+  const int64_t waves = tiles * (kThreads / 64), room = 32ll * device_cus();
+  return (waves * 4 <= room) ? 4 : (waves * 2 <= room) ? 2 : 1;
+}
+
 template <int kGeom, int kOp>
 void launch_fmt(const DrrLaunch& L, dim3 grid, hipStream_t s, int accumulate, float fill)
 {
-#define XRH_LAUNCH_FMT(F)                                                                      \
-  do {                                                                                         \
-    if (L.objs > 1) {                                                                          \
-      hipLaunchKernelGGL((drr_objects_kernel<kGeom, kOp, F>), grid, dim3(kThreads), 0, s,      \
-                         L.items_dev, L.band_start_dev, L.num_items, L.bands, L.out, fill,     \
-                         L.ncc_partials, L.ncc_tiles_per_item, shape, L.objs);                 \
-    } else {                                                                                   \
-      hipLaunchKernelGGL((drr_kernel<kGeom, kOp, F>), grid, dim3(kThreads), 0, s, L.items_dev, \
-                         L.band_start_dev, L.num_items, L.bands, L.out, accumulate, fill,      \
-                         L.ncc_partials, L.ncc_tiles_per_item, shape);                         \
-    }                                                                                          \
+#define XRH_LAUNCH_PARTS(F, P)                                                                        \
+  do {                                                                                                \
+    const dim3 threads(kThreads * (P > 1 ? P : 1));                                                   \
+    const int lds = (P == 0) ? slab : 0;                                                              \
+    if (L.objs > 1) {                                                                                 \
+      hipLaunchKernelGGL((drr_objects_kernel<kGeom, kOp, F, P>), grid, threads, lds, s, L.items_dev,  \
+                         L.band_start_dev, L.num_items, L.bands, L.out, fill, L.ncc_partials,         \
+                         L.ncc_tiles_per_item, shape, lds / 4, L.objs);                               \
+    } else {                                                                                          \
+      hipLaunchKernelGGL((drr_kernel<kGeom, kOp, F, P>), grid, threads, lds, s, L.items_dev,          \
+                         L.band_start_dev, L.num_items, L.bands, L.out, accumulate, fill,             \
+                         L.ncc_partials, L.ncc_tiles_per_item, shape, lds / 4);                       \
+    }                                                                                                 \
   } while (0)
-  // Cell reuse (one sample per iteration, loads only on cell change) wins when the launch
-  // fills every CU many times over and the kernel is bound by load issue; small launches are
-  // latency-bound and prefer the two-samples-per-iteration kernel. XRH_CELL_REUSE=0 / =1
-  // force either (read per launch, so a process can switch between calls); otherwise a tuned
-  // variant decides, else the launch size.
+#define XRH_LAUNCH_FMT(F)                         \
+  do {                                            \
+    if (parts == 4) XRH_LAUNCH_PARTS(F, 4);       \
+    else if (parts == 2) XRH_LAUNCH_PARTS(F, 2);  \
+    else XRH_LAUNCH_PARTS(F, 1);                  \
+  } while (0)
+  // Waves per ray. XRH_CELL_REUSE=0 / =1 force shared / whole rays (read per launch, so a process
+  // can switch between calls); otherwise a tuned variant decides, else the launch size.
   const char* reuse_env = std::getenv("XRH_CELL_REUSE");
-  const bool reuse = reuse_env ? (std::strcmp(reuse_env, "0") != 0)
-                     : (L.reuse >= 0) ? (L.reuse != 0)
-                                      : ((int64_t)grid.x * grid.y >= 16ll * device_cus());
+  const int reuse = reuse_env ? (std::strcmp(reuse_env, "0") != 0 ? 1 : 0) : L.reuse;
+  const int64_t tiles = (int64_t)grid.x * grid.y;
+  const int parts = (reuse > 0) ? 1 : (reuse == 0) ? std::max(drr_parts(tiles), 2) : drr_parts(tiles);
   const int shape = (L.wave_shape >= 0 && L.wave_shape <= 2) ? L.wave_shape : 0;
   const int fmt = (L.storage == XRH_F32)
-                      ? (L.layout == kLayoutCoef ? (reuse ? 7 : 6)
-                                                 : (L.layout == kLayoutFace ? (reuse ? 11 : 10)
-                                                    : (L.layout == kLayoutBrick ? (reuse ? 13 : 12)
+                      ? (L.layout == kLayoutCoef ? 7
+                                                 : (L.layout == kLayoutFace ? 11
+                                                    : (L.layout == kLayoutBrick ? 13
                                                                                 : (L.layout == kLayoutQuad ? 1 : 0))))
                 : (L.storage == XRH_F16) ? (L.layout == kLayoutOct ? 3 : 2)
                                          : (L.layout == kLayoutOct ? 5 : 4);
+  const int slab = drr_slab_lds(L.ray_spacing, L.geom, L.vol_bytes);
+  if (fmt == 11 && parts == 1 && slab > 0) {
+    XRH_LAUNCH_PARTS(11, 0);
+    return;
+  }
   switch (fmt) {
     case 0: XRH_LAUNCH_FMT(0); break;
     case 1: XRH_LAUNCH_FMT(1); break;
@@ -631,19 +1124,35 @@ void launch_fmt(const DrrLaunch& L, dim3 grid, hipStream_t s, int accumulate, fl
     case 3: XRH_LAUNCH_FMT(3); break;
     case 4: XRH_LAUNCH_FMT(4); break;
     case 5: XRH_LAUNCH_FMT(5); break;
-    case 6: XRH_LAUNCH_FMT(6); break;
     case 7: XRH_LAUNCH_FMT(7); break;
-    case 10: XRH_LAUNCH_FMT(10); break;
-    case 12: XRH_LAUNCH_FMT(12); break;
     case 13: XRH_LAUNCH_FMT(13); break;
     default: XRH_LAUNCH_FMT(11); break;
   }
 #undef XRH_LAUNCH_FMT
+#undef XRH_LAUNCH_PARTS
 }
 
 }  // namespace
 
-bool drr_default_reuse(int64_t workgroups) { return workgroups >= 16ll * device_cus(); }
+// LDS bytes of a slab-marching launch whose rays are `spacing` voxels apart on average (0: not
+// known) and whose largest volume's face layout has `bytes`; 0 to gather. Gathering stays the
+// better march for close rays over a volume that the caches hold (0.39 voxels apart, ns per ray
+// by gathering / slabs: 26 MB of faces 0.190 / 0.197 with FP64 set-up, 0.191 / 0.219 with FP32;
+// 215 MB 0.355 / 0.330 and 0.357 / 0.371; 1.7 GB 0.748 / 0.554 and 0.753 / 0.632). Otherwise eight
+// workgroups per CU (the most) while the boxes are small; four where the rays are about a voxel
+// apart and more, for boxes of several layers; three past the point where most boxes no longer fit
+// and the tiles gather, for which fewer waves per L1 are the better choice. ns per ray with 20 /
+// 40 / 54 KB: 256 x 256 x 200 voxels at 0.58 voxels 0.397 / 0.485 / 0.758, at 0.78 0.440 / 0.516 /
+// 0.828, at 1.16 0.787 / 0.625 / 0.940, at 1.55 1.30 / 1.05 / 1.29, at 2.3 2.22 / 1.91 / 2.28; 512 x
+// 512 x 400 voxels at 3.1 6.06 / 5.66 / 5.32.
+int drr_slab_lds(float spacing, int32_t geom, uint64_t bytes)
+{
+  if (!(spacing > 0.0f)) return 0;
+  if (spacing < 0.5f && bytes < (geom == XRH_GEOM_FP32 ? (256ull << 20) : (64ull << 20))) return 0;
+  return spacing < 0.95f ? 20224 : (spacing < 2.7f ? 40704 : 54272);
+}
+
+bool drr_default_reuse(int64_t workgroups) { return drr_parts(workgroups) == 1; }
 
 std::string drr_tune_key(int32_t storage, int32_t layout, int32_t geom, int32_t kernel, int32_t max_rows,
                          int32_t max_cols, int64_t workgroups)

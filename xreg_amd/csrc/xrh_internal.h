@@ -106,6 +106,9 @@ struct DrrItem {
   CamDev cam;
   const void* vol;   // padded layout base
   uint32_t vol_bytes;
+  uint32_t raw_bytes;
+  const void* raw;   // padded voxels (see VolDesc), or null
+  uint32_t raw_py, raw_pz;
   int32_t X, Y, Z;   // unpadded index extent
   uint32_t pitch_y;  // padded row pitch in elements (X+2)
   uint32_t pitch_z;  // padded slice pitch in elements ((X+2)*(Y+2))
@@ -148,6 +151,11 @@ struct VolDesc {
   // null when skipping is disabled
   const uint8_t* skip;
   int32_t skip_gx, skip_gy, skip_gz, skip_shift;
+  // the padded voxels themselves (kLayoutLinear's arrangement) beside a packed FP32 layout, for
+  // slab marching; null without
+  const void* raw;
+  uint32_t raw_bytes;
+  int32_t pad2_;
 };
 
 // Rejects steps so small that a ray would take millions of samples (keeps kernels short).
@@ -169,8 +177,7 @@ inline void check_step(float step, const VolDesc& v)
 
 namespace xrh {
 // How a DRR launch is laid out (results are identical under every variant):
-//   reuse  1: one sample per loop iteration, loads only when a sample enters a new cell;
-//          0: two samples per iteration, every sample loads; -1: chosen by launch size
+//   reuse  1: one lane marches a whole ray; 0: several waves share it; -1: by launch size
 //   shape  pixels per wave64 inside the 16x16 workgroup tile: 0 = 8x8, 1 = 16x4, 2 = 4x16
 //   bands  detector-row bands of the XCD-aware workgroup order
 struct DrrVariant {
@@ -219,8 +226,11 @@ struct xrh_volume {
   xrh::VolDesc desc{};
   void* data = nullptr;
   void* skip = nullptr;
+  void* raw = nullptr;
   uint64_t bytes = 0;
   int64_t size[3] = {0, 0, 0};
+  double center[3] = {0, 0, 0};  // physical
+  double spacing = 1.0;          // geometric mean of the voxel edges
   // built on first use by an interpolating cast (xrh_line_int_interp), freed with the volume
   xrh::InterpGrid grid[2];
   void* grid_mem[2] = {nullptr, nullptr};
@@ -292,6 +302,9 @@ struct DrrLaunch {
                             // samples of the reference algorithm, [1] = samples evaluated
   int32_t* ray_steps;       // optional with sample_counter: per pixel (at out_off), the last
                             // sample index n of the reference algorithm (-1: the ray misses)
+  float ray_spacing;        // mean distance of neighbouring rays at the volumes' centres (voxels),
+                            // 0 if not known: with vol_bytes, the largest volume's layout bytes,
+  uint64_t vol_bytes;       // it chooses between slab marching and gathering
   int32_t reuse;            // DrrVariant::reuse
   int32_t wave_shape;       // DrrVariant::shape
   int32_t objs;             // objects per item (0 or 1: one); items_dev / poses_dev then hold
@@ -301,9 +314,14 @@ struct DrrLaunch {
 };
 // Key of the tuned-variant table: storage, layout, geometry, line kernel, the largest
 // detector of the launch and its workgroups per CU (rounded down to a power of two).
+// The slab-marching choice of a launch (its dynamic LDS bytes, 0: gathering).
+int drr_slab_lds(float spacing, int32_t geom, uint64_t bytes);
+// Distance (voxels) of neighbouring rays at the volume's centre for a camera and a row-major
+// cam->phys pose.
+float ray_spacing(const xrh_volume* vol, const xrh_camera& cam, const double pose[16]);
 std::string drr_tune_key(int32_t storage, int32_t layout, int32_t geom, int32_t kernel, int32_t max_rows,
                          int32_t max_cols, int64_t workgroups);
-// The cell-reuse choice of an untuned launch of `workgroups` workgroups (reuse = -1).
+// Whether an untuned launch of `workgroups` workgroups marches whole rays (reuse = -1).
 bool drr_default_reuse(int64_t workgroups);
 constexpr int32_t kMaxDrrBands = 16;
 void launch_drr_setup(const DrrLaunch& L, hipStream_t s);

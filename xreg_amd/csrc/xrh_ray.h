@@ -124,7 +124,7 @@ struct Ray {
 
 // Per-ray set-up in float, reference order (xregRayCastLineIntCPU.cpp:204-268).
 // (col, row) is the detector index (a pixel's integer index, or a jittered one).
-__device__ inline Ray setup_ray_f32(const DrrItem& it, float col, float row)
+__device__ __forceinline__ Ray setup_ray_f32(const DrrItem& it, float col, float row)
 {
 #pragma clang fp contract(off)
   Ray ray;
@@ -174,7 +174,7 @@ __device__ inline Ray setup_ray_f32(const DrrItem& it, float col, float row)
 }
 
 // Per-ray set-up in double; samples later placed at start + i*step in float.
-__device__ inline Ray setup_ray_f64(const DrrItem& it, int col, int row)
+__device__ __forceinline__ Ray setup_ray_f64(const DrrItem& it, int col, int row)
 {
   Ray ray;
   ray.n = -1;
@@ -268,7 +268,7 @@ __device__ inline TileRef decode_tile(const uint32_t* band_start, int64_t num_it
 // shape covers the tile's 256 pixels once.
 __device__ inline void lane_pixel(int tx, int ty, int shape, int& col, int& row)
 {
-  const int t = threadIdx.x;
+  const int t = threadIdx.x & (kThreads - 1);
   const int w = t >> 6, l = t & 63;
   if (shape == 1) {
     col = tx * kTile + (l & 15);

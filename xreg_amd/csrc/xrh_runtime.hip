@@ -191,6 +191,15 @@ __device__ inline uint16_t f2bf_bits(float v)
   return (uint16_t)(r >> 16);
 }
 
+// A face's coefficients from its corners, by the float differences that the slab march takes from
+// the voxels themselves.
+__device__ inline float4 face(float v00, float v10, float v01, float v11)
+{
+#pragma clang fp contract(off)
+  const float c1 = v10 - v00;
+  return make_float4(v00, c1, v01 - v00, (v11 - v01) - c1);
+}
+
 // Builds the padded layout from the raw x-fastest volume. One thread per padded voxel.
 __global__ void build_layout_kernel(const float* __restrict__ src, int X, int Y, int Z,
                                     void* __restrict__ dst, int storage, int layout)
@@ -223,16 +232,12 @@ __global__ void build_layout_kernel(const float* __restrict__ src, int X, int Y,
     ((float4*)dst)[i] = q;
   } else if (layout == kLayoutFace) {
     // face normal to x at (a, b, c): corners (b, c), (b+1, c), (b, c+1), (b+1, c+1) over y, z;
-    // bilinear coefficients f(v, w) = c0 + c1 v + c2 w + c3 v w formed in double, rounded once
-    const double v00 = V(a, b, c), v10 = V(a, b + 1, c), v01 = V(a, b, c + 1), v11 = V(a, b + 1, c + 1);
-    ((float4*)dst)[i] = make_float4((float)v00, (float)(v10 - v00), (float)(v01 - v00),
-                                    (float)((v11 - v01) - (v10 - v00)));
+    // bilinear coefficients f(v, w) = c0 + c1 v + c2 w + c3 v w
+    ((float4*)dst)[i] = face(V(a, b, c), V(a, b + 1, c), V(a, b, c + 1), V(a, b + 1, c + 1));
   } else if (layout == kLayoutBrick) {
     // the face of (a, b, c) as in kLayoutFace, written to its brick and, when it is the first
     // x-face of a brick, also as the last x-face of the previous brick in x
-    const double v00 = V(a, b, c), v10 = V(a, b + 1, c), v01 = V(a, b, c + 1), v11 = V(a, b + 1, c + 1);
-    const float4 f = make_float4((float)v00, (float)(v10 - v00), (float)(v01 - v00),
-                                 (float)((v11 - v01) - (v10 - v00)));
+    const float4 f = face(V(a, b, c), V(a, b + 1, c), V(a, b, c + 1), V(a, b + 1, c + 1));
     const int nbx = (int)((Xp - 1 + kBrickEdge - 1) / kBrickEdge);   // bricks of cells 0..X
     const int nby = (int)((Yp + kBrickEdge - 1) / kBrickEdge);
     const int by = b / kBrickEdge, bz = c / kBrickEdge;
@@ -375,6 +380,10 @@ __global__ void hu_to_lin_att_kernel(float* __restrict__ v, int64_t n, double hu
   v[i] = (float)((a < 0.0) ? 0.0 : a);
 }
 
+// Bytes of the plain padded voxels beside a packed layout: 16-byte loads of a row's last voxels may
+// reach past the last one.
+static uint64_t raw_alloc_bytes(int64_t padded) { return (uint64_t)padded * 4 + 64; }
+
 struct HuParams {
   double hu_lower, mu_water, mu_air;
 };
@@ -445,6 +454,13 @@ static void volume_create(xrh_ctx* ctx, const float* vox, const int64_t size[3],
     hipLaunchKernelGGL(build_layout_kernel, dim3((unsigned)blocks), dim3(threads), 0, ctx->stream,
                        (const float*)raw, (int)X, (int)Y, (int)Z, v->data, storage, layout);
     XRH_HIP_CHECK(hipGetLastError());
+    // the plain voxels beside the faces, unless the context's budget is nearly spent
+    if (layout == kLayoutFace && (!ctx->budget || ctx->budget >= ctx->in_use + 4 * raw_alloc_bytes(padded))) {
+      v->raw = ctx_alloc(ctx, raw_alloc_bytes(padded));
+      hipLaunchKernelGGL(build_layout_kernel, dim3((unsigned)blocks), dim3(threads), 0, ctx->stream,
+                         (const float*)raw, (int)X, (int)Y, (int)Z, v->raw, storage, (int)kLayoutLinear);
+      XRH_HIP_CHECK(hipGetLastError());
+    }
     const int SB = 1 << kSkipShift;
     const int64_t sgx = (X + SB - 1) / SB, sgy = (Y + SB - 1) / SB, sgz = (Z + SB - 1) / SB;
     // the walk indexes the map with 24-bit multiply-adds: larger maps go without skipping
@@ -473,6 +489,7 @@ static void volume_create(xrh_ctx* ctx, const float* vox, const int64_t size[3],
     if (raw) ctx_free(ctx, raw);
     if (v->data) ctx_free(ctx, v->data);
     if (v->skip) ctx_free(ctx, v->skip);
+    if (v->raw) ctx_free(ctx, v->raw);
     delete v;
     throw;
   }
@@ -486,6 +503,8 @@ static void volume_create(xrh_ctx* ctx, const float* vox, const int64_t size[3],
   affine_inverse_f32(idx_to_phys, d.p2i);
   affine_inverse_f64(idx_to_phys, d.p2i_d);
   d.data = v->data;
+  d.raw = v->raw;
+  d.raw_bytes = v->raw ? (uint32_t)raw_alloc_bytes(padded) : 0;
   d.bytes = (uint32_t)bytes;
   d.X = (int32_t)X;
   d.Y = (int32_t)Y;
@@ -511,8 +530,31 @@ static void volume_create(xrh_ctx* ctx, const float* vox, const int64_t size[3],
   }
   XRH_REQUIRE(ms > 0.0f && std::isfinite(ms), "idx_to_phys has a zero or non-finite column");
   d.min_spacing = ms;
+  v->spacing = 1.0;
+  for (int c = 0; c < 3; ++c) {
+    double n2 = 0.0;
+    v->center[c] = idx_to_phys[4 * c + 3];
+    for (int r = 0; r < 3; ++r) {
+      n2 += (double)idx_to_phys[4 * r + c] * idx_to_phys[4 * r + c];
+      v->center[c] += idx_to_phys[4 * c + r] * 0.5 * (double)dims[r];
+    }
+    v->spacing *= std::cbrt(std::sqrt(n2));
+  }
   d.max_chord = (float)chord;
   *out = v;
+}
+
+float ray_spacing(const xrh_volume* vol, const xrh_camera& cam, const double pose[16])
+{
+  double d2 = 0.0, px2 = 0.0;
+  for (int r = 0; r < 3; ++r) {
+    double ph = pose[4 * r + 3];
+    for (int c = 0; c < 3; ++c) ph += pose[4 * r + c] * (double)cam.pinhole[c];
+    d2 += (vol->center[r] - ph) * (vol->center[r] - ph);
+    px2 += (double)cam.intrins_inv[3 * r] * cam.intrins_inv[3 * r];  // one column at unit depth
+  }
+  const double s = std::sqrt(px2 * d2) / vol->spacing;
+  return std::isfinite(s) ? (float)s : 0.0f;
 }
 
 // Band-major tile table of num_projs equal detectors into band_start ([bands][num_projs + 1],
@@ -659,6 +701,10 @@ static void line_int_launch(xrh_ctx* ctx, const xrh_volume* vol, const xrh_camer
   L.layout = vol->desc.layout;
   L.out = drr_dev;
   L.sample_counter = samples_out ? (uint64_t*)(dev + off_cnt) : nullptr;
+  double spacing = 0.0;
+  for (int64_t p = 0; p < num_projs; ++p) spacing += ray_spacing(vol, cams[cam_for_proj[p]], pin[p].pose);
+  L.ray_spacing = (float)(spacing / (double)num_projs);
+  L.vol_bytes = vol->bytes;
   L.reuse = var.reuse;
   L.wave_shape = var.shape;
   launch_drr_setup(L, ctx->stream);
@@ -882,6 +928,7 @@ xrh_status xrh_volume_destroy(xrh_volume* vol)
     XRH_HIP_CHECK(hipStreamSynchronize(vol->ctx->stream));
     ctx_free(vol->ctx, vol->data);
     if (vol->skip) ctx_free(vol->ctx, vol->skip);
+    if (vol->raw) ctx_free(vol->ctx, vol->raw);
     for (void* g : vol->grid_mem) {
       if (g) ctx_free(vol->ctx, g);
     }
@@ -891,7 +938,7 @@ xrh_status xrh_volume_destroy(xrh_volume* vol)
 
 uint64_t xrh_volume_bytes(const xrh_volume* vol)
 {
-  return vol ? vol->bytes + vol->grid_bytes[0] + vol->grid_bytes[1] : 0;
+  return vol ? vol->bytes + vol->desc.raw_bytes + vol->grid_bytes[0] + vol->grid_bytes[1] : 0;
 }
 
 xrh_status xrh_volume_info(const xrh_volume* vol, int32_t* storage, int32_t* layout)
