@@ -200,6 +200,10 @@ struct xrh_ctx {
   uint64_t scratch_bytes = 0;
   void* pinned = nullptr;
   uint64_t pinned_bytes = 0;
+  // workspace of the image operations (work_mu held from ctx_work to the end of the work)
+  std::mutex work_mu;
+  void* work = nullptr;
+  uint64_t work_bytes = 0;
   // DRR variants chosen by xrh_batch_autotune, keyed by drr_tune_key
   std::map<std::string, xrh::DrrVariant> tuned;
 };
@@ -248,6 +252,8 @@ void ctx_check_range(xrh_ctx* ctx, const void* p, uint64_t bytes, const char* wh
 // grows ctx->scratch to at least `bytes` (device) and returns it
 void* ctx_scratch(xrh_ctx* ctx, uint64_t bytes);
 void* ctx_pinned(xrh_ctx* ctx, uint64_t bytes);
+// grows ctx->work to at least `bytes` (device) and returns it; the caller holds ctx->work_mu
+void* ctx_work(xrh_ctx* ctx, uint64_t bytes);
 
 // host-side helpers (xrh_runtime.hip)
 CamDev make_cam_dev(const xrh_camera& c);

@@ -20,6 +20,7 @@
 #include "xrh_internal.h"
 
 #include <cmath>
+#include <mutex>
 #include <vector>
 
 namespace xrh {
@@ -102,7 +103,8 @@ __global__ void gauss_x_kernel(const float* __restrict__ img, double* __restrict
   out[(int64_t)r * cols + c] = s;
 }
 
-__global__ void gauss_y_kernel(const double* __restrict__ in, float* __restrict__ out, int rows, int cols,
+// (the filter's float result, as the double that the decomposition starts from)
+__global__ void gauss_y_kernel(const double* __restrict__ in, double* __restrict__ out, int rows, int cols,
                                const double* __restrict__ w, int R)
 {
   const int c = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y;
@@ -112,7 +114,7 @@ __global__ void gauss_y_kernel(const double* __restrict__ in, float* __restrict_
     const int rr = min(max(r + k, 0), rows - 1);
     s += w[k + R] * in[(int64_t)rr * cols + c];
   }
-  out[(int64_t)r * cols + c] = (float)s;
+  out[(int64_t)r * cols + c] = (double)(float)s;
 }
 
 __global__ void to_double_kernel(const float* __restrict__ in, double* __restrict__ out, int64_t n)
@@ -121,54 +123,145 @@ __global__ void to_double_kernel(const float* __restrict__ in, double* __restric
   if (i < n) out[i] = (double)in[i];
 }
 
-// BSplineDecompositionImageFilter::DataToCoefficients1D for the cubic pole, on the line
-// c[0], c[stride], ..., c[(n-1) * stride].
-__device__ void bspline_line(double* c, int n, int64_t stride)
+// BSplineDecompositionImageFilter::DataToCoefficients1D for the cubic pole z = sqrt(3) - 2, cut
+// into chunks. Line by line in one thread the two recursions were a serial chain over global
+// memory (768 x 768: 512 us along the rows, 380 us down the columns). Their memory decays as |z|^k,
+// so a chunk that starts kWarm samples early from zero has the line's own values to |z|^32 =
+// 5e-19, below a double's rounding; only the first and last samples need the mirror-boundary start
+// values. All chunks then run at once: 14 and 17 us.
+constexpr int kWarm = 32;
+constexpr double kPole = 1.7320508075688772 - 2.0;
+constexpr double kGain = (1.0 - kPole) * (1.0 - 1.0 / kPole);
+
+// Start values of a line of n samples (set on the host): terms of the causal start sum when that
+// is shorter than the line, and z^(n-1) for the closed form when it is not.
+struct LineStart {
+  int horizon;
+  double z_n1;
+};
+
+// The first causal coefficient (SetInitialCausalCoefficient) from x(0), x(1), ... (times the gain).
+template <class X>
+__device__ inline double causal_start(int n, const LineStart& ls, X x)
 {
-  if (n == 1) return;
-  const double z = 1.7320508075688772 - 2.0;  // sqrt(3) - 2
-#define C_(i) c[(int64_t)(i) * stride]
-  const double gain = (1.0 - z) * (1.0 - 1.0 / z);
-  for (int i = 0; i < n; ++i) C_(i) *= gain;
-  // initial causal coefficient (SetInitialCausalCoefficient), tolerance 1e-10
-  const int horizon = (int)ceil(log(1.0e-10) / log(fabs(z)));
-  double zn = z;
-  if (horizon < n) {
-    double sum = C_(0);
-    for (int i = 1; i < horizon; ++i) {
-      sum += zn * C_(i);
-      zn *= z;
+  if (ls.horizon < n) {
+    double sum = x(0), zk = kPole;
+    for (int i = 1; i < ls.horizon; ++i) {
+      sum += zk * x(i);
+      zk *= kPole;
     }
-    C_(0) = sum;
-  } else {
-    const double iz = 1.0 / z;
-    double z2n = pow(z, (double)(n - 1));
-    double sum = C_(0) + z2n * C_(n - 1);
-    z2n *= z2n * iz;
-    for (int i = 1; i <= n - 2; ++i) {
-      sum += (zn + z2n) * C_(i);
-      zn *= z;
-      z2n *= iz;
-    }
-    C_(0) = sum / (1.0 - zn * zn);
+    return sum;
   }
-  for (int i = 1; i < n; ++i) C_(i) += z * C_(i - 1);
-  // initial anti-causal coefficient, then the anti-causal recursion
-  C_(n - 1) = (z / (z * z - 1.0)) * (z * C_(n - 2) + C_(n - 1));
-  for (int i = n - 2; i >= 0; --i) C_(i) = z * (C_(i + 1) - C_(i));
-#undef C_
+  const double iz = 1.0 / kPole;
+  double zk = kPole, z2k = ls.z_n1;
+  double sum = x(0) + z2k * x(n - 1);
+  z2k *= z2k * iz;
+  for (int i = 1; i <= n - 2; ++i) {
+    sum += (zk + z2k) * x(i);
+    zk *= kPole;
+    z2k *= iz;
+  }
+  return sum / (1.0 - zk * zk);
 }
 
-__global__ void bspline_rows_kernel(double* __restrict__ coef, int rows, int cols)
+// Rows: one wave per chunk of kRowChunk samples of a row, samples in LDS, each lane a run of them.
+constexpr int kRowChunk = 256;
+__global__ __launch_bounds__(64) void bspline_rows_kernel(const double* __restrict__ in, double* __restrict__ out,
+                                                          int cols, LineStart ls)
 {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < rows) bspline_line(coef + (int64_t)r * cols, cols, 1);
+  __shared__ double x[kRowChunk + 2 * kWarm + 2], y[kRowChunk + kWarm + 2];
+  const double* src = in + (int64_t)blockIdx.y * cols;
+  double* dst = out + (int64_t)blockIdx.y * cols;
+  const int n = cols, s = blockIdx.x * kRowChunk, e = min(s + kRowChunk, n);
+  if (n == 1) {
+    if (threadIdx.x == 0) dst[0] = src[0];
+    return;
+  }
+  const int r0 = max(s - 1, 0), r1 = min(e + kWarm, n), a = max(r0 - kWarm, 0);  // causal values r0..r1
+  for (int i = a + (int)threadIdx.x; i < r1; i += 64) x[i - a] = src[i] * kGain;
+  __syncthreads();
+  {
+    const int m = (r1 - r0 + 63) / 64, p = r0 + (int)threadIdx.x * m, q = min(p + m, r1);
+    if (p < q) {
+      int i = p - kWarm;
+      double c = 0.0;
+      if (i <= 0) {
+        c = causal_start(n, ls, [&](int k) { return x[k]; });  // (a is 0 here)
+        if (p == 0) y[0] = c;
+        i = 1;
+      }
+      for (; i < q; ++i) {
+        c = x[i - a] + kPole * c;
+        if (i >= p) y[i - r0] = c;
+      }
+    }
+  }
+  __syncthreads();
+  const int m = (e - s + 63) / 64, p = s + (int)threadIdx.x * m, q = min(p + m, e);
+  if (p < q) {
+    int j = min(q - 1 + kWarm, n - 1);
+    double c = 0.0;
+    if (j == n - 1) {
+      c = (kPole / (kPole * kPole - 1.0)) * (kPole * y[n - 2 - r0] + y[n - 1 - r0]);
+      if (j < q) dst[j] = c;
+      --j;
+    }
+    for (; j >= p; --j) {
+      c = kPole * (c - y[j - r0]);
+      if (j < q) dst[j] = c;
+    }
+  }
 }
 
-__global__ void bspline_cols_kernel(double* __restrict__ coef, int rows, int cols)
+// Columns: a lane per column, a wave per 64 columns and kColChunk rows; every row is one coalesced
+// read.
+constexpr int kColChunk = 32;
+__global__ __launch_bounds__(64) void bspline_cols_kernel(const double* __restrict__ in, double* __restrict__ out,
+                                                          int rows, int cols, LineStart ls)
 {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < cols) bspline_line(coef + c, rows, cols);
+  __shared__ double y[kColChunk + kWarm + 1][64];
+  const int c0 = blockIdx.x * 64 + (int)threadIdx.x, col = min(c0, cols - 1), l = threadIdx.x;
+  const int n = rows, s = blockIdx.y * kColChunk, e = min(s + kColChunk, n);
+  auto x = [&](int i) { return in[(int64_t)i * cols + col] * kGain; };
+  if (n == 1) {
+    if (c0 < cols) out[col] = in[col];
+    return;
+  }
+  const int r0 = max(s - 1, 0), r1 = min(e + kWarm, n);
+  int i = r0 - kWarm;
+  double c = 0.0;
+  if (i <= 0) {
+    c = causal_start(n, ls, x);
+    if (r0 == 0) y[0][l] = c;
+    i = 1;
+  }
+#pragma unroll 8
+  for (; i < r0; ++i) c = x(i) + kPole * c;
+#pragma unroll 8
+  for (; i < r1; ++i) {
+    c = x(i) + kPole * c;
+    y[i - r0][l] = c;
+  }
+  // (each lane reads back its own column only)
+  int j = min(e - 1 + kWarm, n - 1);
+  c = 0.0;
+  if (j == n - 1) {
+    c = (kPole / (kPole * kPole - 1.0)) * (kPole * y[n - 2 - r0][l] + y[n - 1 - r0][l]);
+    if (j < e && c0 < cols) out[(int64_t)j * cols + col] = c;
+    --j;
+  }
+  for (; j >= s; --j) {
+    c = kPole * (c - y[j - r0][l]);
+    if (j < e && c0 < cols) out[(int64_t)j * cols + col] = c;
+  }
+}
+
+LineStart line_start(int n)
+{
+  LineStart ls;
+  ls.horizon = (int)std::ceil(std::log(1.0e-10) / std::log(std::fabs(kPole)));
+  ls.z_n1 = std::pow(kPole, (double)(n - 1));
+  return ls;
 }
 
 __device__ inline int mirror(int i, int n)
@@ -262,51 +355,50 @@ xrh_status xrh_downsample_image(xrh_ctx* ctx, const float* img, int32_t rows, in
       const double s = (sigma < 0.0) ? 0.5 / factor : sigma;
       w = gaussian_kernel(s * s, 0.01, 32);
     }
-    float* d_img = nullptr;
-    float* d_sm = nullptr;
-    double* d_tmp = nullptr;
-    double* d_w = nullptr;
-    float* d_out = nullptr;
-    auto cleanup = [&] {
-      (void)hipStreamSynchronize(ctx->stream);
-      for (void* p : {(void*)d_img, (void*)d_sm, (void*)d_tmp, (void*)d_w, (void*)d_out})
-        if (p) ctx_free(ctx, p);
-    };
+    auto pad = [](uint64_t x) { return (x + 255) & ~uint64_t(255); };
+    const uint64_t off_a = pad((uint64_t)n * 4), off_b = off_a + pad((uint64_t)n * 8), off_w = off_b + pad((uint64_t)n * 8),
+                   off_out = off_w + pad(w.size() * 8), total = off_out + pad((uint64_t)on * 4);
+    // the context's image workspace while no other thread has it and it stays small, beside its
+    // budget too (allocating and releasing it were a fifth of a 768 x 768 call); else memory of this
+    // call's own
+    std::unique_lock<std::mutex> lk(ctx->work_mu, std::try_to_lock);
+    const bool own = !lk.owns_lock() || total > (64ull << 20) || (ctx->budget && ctx->in_use + 16 * total > ctx->budget);
+    char* mem = (char*)(own ? ctx_alloc(ctx, total) : ctx_work(ctx, total));
+    float* d_img = (float*)mem;
+    double *d_a = (double*)(mem + off_a), *d_b = (double*)(mem + off_b), *d_w = (double*)(mem + off_w);
+    float* d_out = (float*)(mem + off_out);
     try {
-      d_img = (float*)ctx_alloc(ctx, (uint64_t)n * 4);
-      d_sm = (float*)ctx_alloc(ctx, (uint64_t)n * 4);
-      d_tmp = (double*)ctx_alloc(ctx, (uint64_t)n * 8);
-      d_out = (float*)ctx_alloc(ctx, (uint64_t)on * 4);
-      XRH_HIP_CHECK(hipMemcpyAsync(d_img, img, (size_t)n * 4, hipMemcpyHostToDevice, ctx->stream));
-      const float* src = d_img;
+      hipStream_t s = ctx->stream;
+      XRH_HIP_CHECK(hipMemcpyAsync(d_img, img, (size_t)n * 4, hipMemcpyHostToDevice, s));
+      // the (smoothed) float image in double
       if (smooth) {
-        d_w = (double*)ctx_alloc(ctx, w.size() * 8);
-        XRH_HIP_CHECK(hipMemcpyAsync(d_w, w.data(), w.size() * 8, hipMemcpyHostToDevice, ctx->stream));
+        XRH_HIP_CHECK(hipMemcpyAsync(d_w, w.data(), w.size() * 8, hipMemcpyHostToDevice, s));
         const int R = (int)(w.size() / 2);
         const dim3 g((unsigned)((cols + 255) / 256), (unsigned)rows);
-        hipLaunchKernelGGL(gauss_x_kernel, g, dim3(256), 0, ctx->stream, d_img, d_tmp, rows, cols, d_w, R);
-        hipLaunchKernelGGL(gauss_y_kernel, g, dim3(256), 0, ctx->stream, d_tmp, d_sm, rows, cols, d_w, R);
-        XRH_HIP_CHECK(hipGetLastError());
-        src = d_sm;
+        hipLaunchKernelGGL(gauss_x_kernel, g, dim3(256), 0, s, d_img, d_b, rows, cols, d_w, R);
+        hipLaunchKernelGGL(gauss_y_kernel, g, dim3(256), 0, s, d_b, d_a, rows, cols, d_w, R);
+      } else {
+        hipLaunchKernelGGL(to_double_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d_img, d_a, n);
       }
-      // B-spline coefficients of the (smoothed) float image, in double
-      hipLaunchKernelGGL(to_double_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, src, d_tmp,
-                         n);
-      hipLaunchKernelGGL(bspline_rows_kernel, dim3((unsigned)((rows + 63) / 64)), dim3(64), 0, ctx->stream, d_tmp,
-                         rows, cols);
-      hipLaunchKernelGGL(bspline_cols_kernel, dim3((unsigned)((cols + 63) / 64)), dim3(64), 0, ctx->stream, d_tmp,
-                         rows, cols);
-      hipLaunchKernelGGL(resample_kernel, dim3((unsigned)((out_cols + 255) / 256), (unsigned)out_rows), dim3(256), 0,
-                         ctx->stream, d_tmp, rows, cols, d_out, out_rows, out_cols, row_spacing, col_spacing,
-                         row_spacing / factor, col_spacing / factor);
       XRH_HIP_CHECK(hipGetLastError());
-      XRH_HIP_CHECK(hipMemcpyAsync(out, d_out, (size_t)on * 4, hipMemcpyDeviceToHost, ctx->stream));
-      XRH_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+      // its B-spline coefficients
+      hipLaunchKernelGGL(bspline_rows_kernel, dim3((unsigned)((cols + kRowChunk - 1) / kRowChunk), (unsigned)rows),
+                         dim3(64), 0, s, d_a, d_b, cols, line_start(cols));
+      hipLaunchKernelGGL(bspline_cols_kernel,
+                         dim3((unsigned)((cols + 63) / 64), (unsigned)((rows + kColChunk - 1) / kColChunk)), dim3(64), 0,
+                         s, d_b, d_a, rows, cols, line_start(rows));
+      hipLaunchKernelGGL(resample_kernel, dim3((unsigned)((out_cols + 255) / 256), (unsigned)out_rows), dim3(256), 0, s,
+                         d_a, rows, cols, d_out, out_rows, out_cols, row_spacing, col_spacing, row_spacing / factor,
+                         col_spacing / factor);
+      XRH_HIP_CHECK(hipGetLastError());
+      XRH_HIP_CHECK(hipMemcpyAsync(out, d_out, (size_t)on * 4, hipMemcpyDeviceToHost, s));
+      XRH_HIP_CHECK(hipStreamSynchronize(s));
     } catch (...) {
-      cleanup();
+      (void)hipStreamSynchronize(ctx->stream);
+      if (own) ctx_free(ctx, mem);
       throw;
     }
-    cleanup();
+    if (own) ctx_free(ctx, mem);
   });
 }
 

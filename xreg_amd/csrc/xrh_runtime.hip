@@ -88,6 +88,20 @@ void* ctx_scratch(xrh_ctx* ctx, uint64_t bytes)
   return ctx->scratch;
 }
 
+void* ctx_work(xrh_ctx* ctx, uint64_t bytes)
+{
+  if (ctx->work_bytes >= bytes) return ctx->work;
+  if (ctx->work) {
+    void* old = ctx->work;
+    ctx->work = nullptr;
+    ctx->work_bytes = 0;
+    ctx_free(ctx, old);  // (its last user synchronised)
+  }
+  ctx->work = ctx_alloc(ctx, bytes);
+  ctx->work_bytes = bytes;
+  return ctx->work;
+}
+
 void* ctx_pinned(xrh_ctx* ctx, uint64_t bytes)
 {
   // the caller has synchronised the stream before reusing the staging area
