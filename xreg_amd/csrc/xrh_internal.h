@@ -228,10 +228,10 @@ constexpr int kGridBSpline = 1;
 struct xrh_volume {
   xrh_ctx* ctx = nullptr;
   xrh::VolDesc desc{};
-  void* data = nullptr;
+  void* data = nullptr;  // the allocation: the layout, the map and the plain voxels
   void* skip = nullptr;
   void* raw = nullptr;
-  uint64_t bytes = 0;
+  uint64_t bytes = 0;    // of the layout
   int64_t size[3] = {0, 0, 0};
   double center[3] = {0, 0, 0};  // physical
   double spacing = 1.0;          // geometric mean of the voxel edges
