@@ -55,10 +55,12 @@ int sim_tiles(const FixedDev& f);     // tiles of the partial-producing kernel
 int sim_img_tiles(const FixedDev& f); // 16x16 image tiles
 
 // Launch-group key of a fixed image: the metric in the low bits; above kSimKeyShift, for
-// unmasked stride-1 patch metrics whose diameter has a compiled kernel, that diameter (else
-// 0); above kSimKeyBlurShift, the gradient metrics' blur radius (0 for none).
+// stride-1 patch metrics with statistics over every pixel and a compiled kernel for the diameter,
+// that diameter (else 0); above kSimKeyBlurShift, the gradient metrics' blur radius (0 for none);
+// kSimKeyMask, a mask beside a compiled diameter.
 constexpr int kSimKeyShift = 4;
 constexpr int kSimKeyBlurShift = 9;
+constexpr int kSimKeyMask = 1 << 12;
 int sim_group_key(const FixedDev& f);
 
 // Queues the similarity kernels for n_items moving images that all share the group key `key`.

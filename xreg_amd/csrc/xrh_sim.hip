@@ -48,11 +48,12 @@ __device__ inline double wave_sum(double v)
   return v;
 }
 
-// Reduces K per-lane doubles over the 256-lane workgroup; lane 0 writes them to dst.
-template <int K>
+// Reduces K per-lane doubles over the workgroup of kWaves waves; lane 0 writes them to dst.
+template <int K, int kWaves = kThreads / 64>
 __device__ inline void block_reduce_store(double (&v)[K], double* dst)
 {
-  __shared__ double red[4][K];
+  static_assert(kWaves == 2 || kWaves == 4, "two or four waves");
+  __shared__ double red[kWaves][K];
 #pragma unroll
   for (int k = 0; k < K; ++k) v[k] = wave_sum(v[k]);
   const int w = threadIdx.x >> 6;
@@ -63,7 +64,11 @@ __device__ inline void block_reduce_store(double (&v)[K], double* dst)
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) dst[k] = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
+    for (int k = 0; k < K; ++k) {
+      double t = red[0][k] + red[1][k];
+      if constexpr (kWaves == 4) t += red[2][k] + red[3][k];
+      dst[k] = t;
+    }
   }
 }
 
@@ -450,37 +455,71 @@ __global__ __launch_bounds__(kThreads) void patch_kernel(const SimItem* __restri
   block_reduce_store<2>(acc, partials + (it.out_index * ptiles + tile) * 2);
 }
 
-// patch_kernel for the common case -- no mask, stride 1, a compile-time patch diameter kD.
-// Same per-patch closed form; the box sums are formed with sliding windows so that LDS
-// traffic drops about threefold:
+// patch_kernel for the common cases -- stride 1, a compile-time patch diameter kD, every pixel's
+// statistics (kMask: a mask in the correlation and the weights). Same per-patch closed form, with
+// two waves per 16 x 16 patches:
 //  * each direction's window and per-patch fixed statistics are read before the first one is
 //    waited for; the second direction's window is read once the first direction's sums are
 //    done, so that its registers are free during them;
 //  * the window is staged in LDS as float (the values are floats; products are formed in
 //    double);
-//  * horizontal pass: 4 lanes per window row, each forming 4 consecutive d-wide sums -- the
-//    first directly, the next three by adding the entering and removing the leaving column;
-//  * vertical pass: 64 lanes, one per patch column and group of 4 patch rows, slide the same
-//    way down the column and evaluate the closed form for their 4 patches. The row sums are
-//    kept at an odd pitch (17 doubles) so that the horizontal pass's stores spread over the
-//    LDS banks (2-way instead of 8-way conflicts at a pitch of 16).
-// Occupancy: the two-direction form runs at 6 waves per SIMD (78 VGPRs; with the second window
-// read during the first direction's sums it needed 91, 5 waves, and measured 3% slower), the
-// one-direction form at 8 (64 VGPRs).
-// The sums are FP64 throughout; the sliding updates differ from direct sums by a few units in
-// the last place of a double.
-template <bool kTwo, int kD>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kTwo ? 6 : 8)))
+//  * horizontal pass: 4 lanes per window row, each forming 4 neighbouring d-wide sums from their
+//    common columns, the columns left of those added from the right and those right of them from
+//    the left: d + 6 additions for 4 sums, and no column is ever subtracted again, so a NaN or an
+//    infinity reaches exactly the patches that hold it;
+//  * vertical pass: one lane per patch column and pair of patch rows, the same way, then the
+//    closed form for its 2 patches. The row sums are kept at an odd pitch (17 doubles) so that
+//    the horizontal pass's stores spread over the LDS banks (2-way instead of 8-way conflicts
+//    at a pitch of 16).
+// What bounds it: LDS reads and the wait for them between the passes, in blocks of two waves, of which
+// the LDS (16 KB, masked 22 KB at d = 11) lets 10 or 7 stand on a CU. Measured, 20 image pairs of
+// gradients of 384 x 384, d = 11: masked 61 us (174 in patch_kernel, which took them before), 100 pairs
+// unmasked 200 us (247 with sums sliding along and four waves of which at most two had sums to form;
+// with four waves here the masked 20 pairs take 75).
+// The sums are FP64 throughout.
+constexpr int kPatchThreads = 128;
+
+// kN sums of kD neighbours each, k = 0 .. kN - 1 of elements k .. k + kD - 1; add(i, s) adds
+// element i to the sums s (kQ quantities at once), emit(k, s) takes sum k.
+template <int kD, int kN, int kQ, class Add, class Emit>
+__device__ __forceinline__ void box_sums(Add add, Emit emit)
+{
+  static_assert(kD >= kN, "the sums share elements");
+  double l[kN][kQ], r[kQ];
+#pragma unroll
+  for (int q = 0; q < kQ; ++q) l[kN - 1][q] = r[q] = 0.0;
+#pragma unroll
+  for (int i = kN - 1; i < kD; ++i) add(i, l[kN - 1]);
+#pragma unroll
+  for (int k = kN - 2; k >= 0; --k) {
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) l[k][q] = l[k + 1][q];
+    add(k, l[k]);
+  }
+  emit(0, l[0]);
+#pragma unroll
+  for (int k = 1; k < kN; ++k) {
+    add(kD + k - 1, r);
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) l[k][q] += r[q];
+    emit(k, l[k]);
+  }
+}
+
+template <bool kTwo, int kD, bool kMask>
+__global__ __launch_bounds__(kPatchThreads) __attribute__((amdgpu_waves_per_eu(5)))
 void patch_kernel_d(const SimItem* __restrict__ items, double* __restrict__ partials, int ptiles)
 {
   constexpr int kW = (kT - 1) + kD;  // window edge at stride 1
-  constexpr int kRows = (kW + 7) / 8;
+  constexpr int kStep = kPatchThreads / 32;
+  constexpr int kRows = (kW + kStep - 1) / kStep;
   constexpr int kDirs = kTwo ? 2 : 1;
-  constexpr int kSeg = 4;            // sums per lane in the sliding passes
-  constexpr int kSegs = kT / kSeg;   // lanes per window row / per patch column
+  constexpr int kSeg = 4, kSegs = kT / kSeg;                  // sums per lane, lanes per window row
+  constexpr int kVSeg = kT * kT / kPatchThreads;              // patches per lane
   constexpr int kHP = kT + 1;        // row pitch of the double row sums (odd: spreads the banks)
+  constexpr int kQ = kMask ? 4 : 3;  // sum m, m^2, m f and (masked) m over the used pixels
   static_assert(kW <= 32, "one 32-lane column pass per window row");
-  static_assert(kW * kSegs <= kThreads && kT * kSegs <= kThreads, "sliding lanes fit the block");
+  static_assert(kW * kSegs <= kPatchThreads, "horizontal lanes fit the block");
   extern __shared__ double patch_lds[];
   const SimItem it = items[blockIdx.y];
   const ConstFixed fx = (ConstFixed)it.fixed;  // uniform: scalar loads
@@ -491,9 +530,8 @@ void patch_kernel_d(const SimItem* __restrict__ items, double* __restrict__ part
   const int X0 = (tile % TX) * kT, Y0 = (tile / TX) * kT;  // first patch = first pixel
   float* lm = (float*)patch_lds;
   float* lf = lm + kW * kW;
-  double* h1 = (double*)(lf + kW * kW);  // 2 kW^2 floats: a multiple of 8 bytes
-  double* h2 = h1 + kW * kHP;
-  double* hf = h2 + kW * kHP;
+  float* lk = lf + kW * kW;  // masked only: m at the used pixels
+  double* h = (double*)((kMask ? lk : lf) + kW * kW);  // kW is even: a multiple of 8 bytes
   constexpr double kN = (double)(kD * kD);
   constexpr double kInvN = 1.0 / kN, kInvN1 = 1.0 / (kN - 1.0);
   const int lx = threadIdx.x & 31, ly0 = threadIdx.x >> 5;
@@ -502,29 +540,36 @@ void patch_kernel_d(const SimItem* __restrict__ items, double* __restrict__ part
   const int xo = min(X0 + min(lx, kW - 1), cols - 1);
   const int64_t img_bytes = (int64_t)rows * cols * 4;
   const int64_t np = (int64_t)ppr * ppc;
-  // vertical-pass lanes: patch column vc, patch rows vs * kSeg ... + kSeg - 1
-  const bool vlane = threadIdx.x < kT * kSegs;
-  const int vc = threadIdx.x & (kT - 1), vs = (threadIdx.x >> 4) & (kSegs - 1);
+  // vertical-pass lanes: patch column vc, patch rows vs * kVSeg ... + kVSeg - 1
+  const int vc = threadIdx.x & (kT - 1), vs = threadIdx.x / kT;
 
-  // the byte offset of window row r staged by this lane (formed at each read)
-  auto wo = [&](int r) { return (min(Y0 + min(ly0 + 8 * r, kW - 1), rows - 1) * cols + xo) * 4; };
+  // the pixel of window row r staged by this lane (formed at each read)
+  auto wo = [&](int r) { return min(Y0 + min(ly0 + kStep * r, kW - 1), rows - 1) * cols + xo; };
   float vm[kRows], vf[kRows];
+  uint32_t used = 0;  // bit r: the mask of that pixel
   auto load_window = [&](int dir) {
     const auto rm = ro_rsrc((dir == 0) ? (kTwo ? it.gx : it.mov) : it.gy, img_bytes);
     const auto rf = ro_rsrc((dir == 0) ? fx->pf : fx->pfy, img_bytes);
 #pragma unroll
     for (int r = 0; r < kRows; ++r) {
-      const int o = wo(r);
+      const int o = wo(r) * 4;
       vm[r] = ld_f32(rm, o);
       vf[r] = ld_f32(rf, o);
     }
   };
   load_window(0);
-  float mu[kSeg], den[kSeg];
-  double g[kSeg];
-  bool pv[kSeg];
+  if constexpr (kMask) {
+    const auto rk = ro_rsrc(fx->mask, img_bytes / 4);
 #pragma unroll
-  for (int k = 0; k < kSeg; ++k) pv[k] = vlane && (X0 + vc < ppr) && (Y0 + vs * kSeg + k < ppc);
+    for (int r = 0; r < kRows; ++r) {
+      used |= (__builtin_amdgcn_raw_buffer_load_b8(rk, wo(r), 0, 0) ? 1u : 0u) << r;
+    }
+  }
+  float mu[kVSeg], den[kVSeg];
+  double g[kVSeg];
+  bool pv[kVSeg];
+#pragma unroll
+  for (int k = 0; k < kVSeg; ++k) pv[k] = (X0 + vc < ppr) && (Y0 + vs * kVSeg + k < ppc);
   // one direction's per-patch fixed statistics, read when that direction starts (its window
   // staging and horizontal pass cover the reads)
   auto load_stats = [&](int dir) {
@@ -532,8 +577,8 @@ void patch_kernel_d(const SimItem* __restrict__ items, double* __restrict__ part
     const auto rden = ro_rsrc((dir == 0) ? fx->pden : fx->pdeny, np * 4);
     const auto rg = ro_rsrc((dir == 0) ? fx->pg : fx->pgy, np * 8);
 #pragma unroll
-    for (int k = 0; k < kSeg; ++k) {
-      const int p = pv[k] ? (Y0 + vs * kSeg + k) * ppr + X0 + vc : 0;  // invalid: patch 0, discarded
+    for (int k = 0; k < kVSeg; ++k) {
+      const int p = pv[k] ? (Y0 + vs * kVSeg + k) * ppr + X0 + vc : 0;  // invalid: patch 0, discarded
       mu[k] = ld_f32(rmu, p * 4);
       den[k] = ld_f32(rden, p * 4);
       g[k] = ld_f64(rg, p * 8);
@@ -547,10 +592,16 @@ void patch_kernel_d(const SimItem* __restrict__ items, double* __restrict__ part
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kRows; ++r) {
-      const int ly = ly0 + 8 * r;
+      const int ly = ly0 + kStep * r;
       if (col_ok && ly < kW) {
         lm[ly * kW + lx] = vm[r];
-        lf[ly * kW + lx] = vf[r];
+        if constexpr (kMask) {
+          const float k = (used >> r) & 1u ? 1.0f : 0.0f;
+          lf[ly * kW + lx] = vf[r] * k;
+          lk[ly * kW + lx] = vm[r] * k;
+        } else {
+          lf[ly * kW + lx] = vf[r];
+        }
       }
     }
     __syncthreads();
@@ -558,61 +609,40 @@ void patch_kernel_d(const SimItem* __restrict__ items, double* __restrict__ part
       const int row = threadIdx.x / kSegs, c0 = (threadIdx.x % kSegs) * kSeg;
       const float* m = lm + row * kW + c0;
       const float* f = lf + row * kW + c0;
-      double* o1 = h1 + row * kHP + c0;
-      double* o2 = h2 + row * kHP + c0;
-      double* of = hf + row * kHP + c0;
-      double a1 = 0.0, a2 = 0.0, af = 0.0;
+      const float* mk = lk + row * kW + c0;
+      double* o = h + row * kHP + c0;
+      box_sums<kD, kSeg, kQ>(
+          [&](int i, double (&a)[kQ]) {
+            const double dm = (double)m[i];
+            a[0] += dm;
+            a[1] = fma(dm, dm, a[1]);
+            a[2] = fma(dm, (double)f[i], a[2]);
+            if constexpr (kMask) a[3] += (double)mk[i];
+          },
+          [&](int k, double (&a)[kQ]) {
 #pragma unroll
-      for (int xx = 0; xx < kD; ++xx) {
-        const double dm = (double)m[xx];
-        a1 += dm;
-        a2 = fma(dm, dm, a2);
-        af = fma(dm, (double)f[xx], af);
-      }
-      o1[0] = a1;
-      o2[0] = a2;
-      of[0] = af;
-#pragma unroll
-      for (int k = 1; k < kSeg; ++k) {
-        const double mo = (double)m[k - 1], mn = (double)m[k - 1 + kD];
-        a1 = (a1 - mo) + mn;
-        a2 = fma(mn, mn, fma(-mo, mo, a2));
-        af = fma(mn, (double)f[k - 1 + kD], fma(-mo, (double)f[k - 1], af));
-        o1[k] = a1;
-        o2[k] = a2;
-        of[k] = af;
-      }
+            for (int q = 0; q < kQ; ++q) o[q * kW * kHP + k] = a[q];
+          });
     }
     __syncthreads();
-    if (vlane) {
-      const int e0 = vs * kSeg * kHP + vc;
-      double S1 = 0.0, S2 = 0.0, Sf = 0.0;
+    const double* e0 = h + vs * kVSeg * kHP + vc;
+    box_sums<kD, kVSeg, kQ>(
+        [&](int i, double (&a)[kQ]) {
 #pragma unroll
-      for (int yy = 0; yy < kD; ++yy) {
-        S1 += h1[e0 + yy * kHP];
-        S2 += h2[e0 + yy * kHP];
-        Sf += hf[e0 + yy * kHP];
-      }
-#pragma unroll
-      for (int k = 0; k < kSeg; ++k) {
-        if (k > 0) {
-          const int eo = e0 + (k - 1) * kHP, en = e0 + (k - 1 + kD) * kHP;
-          S1 = (S1 - h1[eo]) + h1[en];
-          S2 = (S2 - h2[eo]) + h2[en];
-          Sf = (Sf - hf[eo]) + hf[en];
-        }
-        if (pv[k]) {
-          const double mean = S1 * kInvN;
-          const double var = fmax(S2 - mean * S1, 0.0) * kInvN1;
-          const double sd = fmax((double)1.0e-6f, sqrt(var));
-          const double cross = (Sf - (double)mu[k] * S1) - mean * g[k];
-          acc[dir] += 1.0 - cross / (sd * (double)den[k]);
-        }
-      }
-    }
+          for (int q = 0; q < kQ; ++q) a[q] += e0[q * kW * kHP + i * kHP];
+        },
+        [&](int k, double (&a)[kQ]) {
+          if (pv[k]) {
+            const double mean = a[0] * kInvN;
+            const double var = fmax(a[1] - mean * a[0], 0.0) * kInvN1;
+            const double sd = fmax((double)1.0e-6f, sqrt(var));
+            const double cross = (a[2] - (double)mu[k] * a[kMask ? 3 : 0]) - mean * g[k];
+            acc[dir] += 1.0 - cross / (sd * (double)den[k]);
+          }
+        });
     if (dir + 1 < kDirs) load_window(dir + 1);
   }
-  block_reduce_store<2>(acc, partials + (it.out_index * ptiles + tile) * 2);
+  block_reduce_store<2, kPatchThreads / 64>(acc, partials + (it.out_index * ptiles + tile) * 2);
 }
 
 // fixed-image per-patch statistics (reference float order, ComputePatchMeanStdDev): over the
@@ -836,17 +866,21 @@ int sim_img_tiles(const FixedDev& f) { return ((f.cols + kT - 1) / kT) * ((f.row
 
 int sim_group_key(const FixedDev& f)
 {
+  // Where patch_kernel_d has the diameter it is the faster one throughout (scoring 20 images of 384 x
+  // 384 with Patch-Grad-NCC, us, here / general: d = 5 86 / 145, masked 96 / 168; d = 11 masked 110 /
+  // 219; d = 17 110 / 196, masked 138 / 302). Larger windows would not fit its 32-lane staging;
+  // statistics over the unmasked pixels only need two more sums and the patch's pixel count.
   int d = 0;
   // (the specialised kernel addresses images and patch tables with 32-bit byte offsets)
   const bool small = (int64_t)f.rows * f.cols * 4 < (int64_t)INT32_MAX && f.num_patches * 8 < (int64_t)INT32_MAX;
-  if ((f.metric == XRH_SIM_PATCH_NCC || f.metric == XRH_SIM_PATCH_GRAD_NCC) && !f.mask && f.patch_stride == 1 &&
+  if ((f.metric == XRH_SIM_PATCH_NCC || f.metric == XRH_SIM_PATCH_GRAD_NCC) && !f.pcount && f.patch_stride == 1 &&
       small) {
     const int dd = 2 * f.patch_radius + 1;
-    if (dd == 7 || dd == 9 || dd == 11 || dd == 13 || dd == 15) d = dd;
+    if (dd >= 5 && dd <= 17) d = dd;
   }
   const int rb = (f.metric == XRH_SIM_GRAD_NCC || f.metric == XRH_SIM_PATCH_GRAD_NCC) && f.smooth_ksize > 1
                      ? f.smooth_ksize / 2 : 0;
-  return f.metric | (d << kSimKeyShift) | (rb << kSimKeyBlurShift);
+  return f.metric | (d << kSimKeyShift) | (rb << kSimKeyBlurShift) | ((d && f.mask) ? kSimKeyMask : 0);
 }
 
 #define XRH_BLUR_DISPATCH(rb, KERNEL, ...)                                            \
@@ -863,8 +897,9 @@ int sim_patch_lds_bytes(const FixedDev& f, bool general)
   if (f.metric != XRH_SIM_PATCH_NCC && f.metric != XRH_SIM_PATCH_GRAD_NCC) return 0;
   const int W = patch_lds_edge(f.patch_stride, f.patch_radius);
   if (!general && ((sim_group_key(f) >> kSimKeyShift) & ((1 << (kSimKeyBlurShift - kSimKeyShift)) - 1))) {
-    // patch_kernel_d: float window pair + three double row-sum arrays
-    return 2 * W * W * (int)sizeof(float) + 3 * W * (kT + 1) * (int)sizeof(double);
+    // patch_kernel_d: float windows (moving, fixed, masked moving) + a double row-sum array per quantity
+    const int n = f.mask ? 1 : 0;
+    return (2 + n) * W * W * (int)sizeof(float) + (3 + n) * W * (kT + 1) * (int)sizeof(double);
   }
   return (f.mask ? (3 * W * W + (f.pcount ? 5 : 4) * W * kT) : (2 * W * W + 3 * W * kT)) * (int)sizeof(double);
 }
@@ -877,18 +912,25 @@ int sim_tiles(const FixedDev& f)
   return sim_img_tiles(f);
 }
 
-template <bool kTwo>
+template <bool kTwo, bool kMask>
 static void launch_patch_d(int d, dim3 grid, int lds, hipStream_t s, const SimItem* items, double* partials,
                            int ptiles)
 {
+#define XRH_PATCH_CASE(D)                                                                                            \
+  case D:                                                                                                            \
+    hipLaunchKernelGGL((patch_kernel_d<kTwo, D, kMask>), grid, dim3(kPatchThreads), lds, s, items, partials, ptiles); \
+    break
   switch (d) {
-    case 7: hipLaunchKernelGGL((patch_kernel_d<kTwo, 7>), grid, dim3(kThreads), lds, s, items, partials, ptiles); break;
-    case 9: hipLaunchKernelGGL((patch_kernel_d<kTwo, 9>), grid, dim3(kThreads), lds, s, items, partials, ptiles); break;
-    case 11: hipLaunchKernelGGL((patch_kernel_d<kTwo, 11>), grid, dim3(kThreads), lds, s, items, partials, ptiles); break;
-    case 13: hipLaunchKernelGGL((patch_kernel_d<kTwo, 13>), grid, dim3(kThreads), lds, s, items, partials, ptiles); break;
-    case 15: hipLaunchKernelGGL((patch_kernel_d<kTwo, 15>), grid, dim3(kThreads), lds, s, items, partials, ptiles); break;
+    XRH_PATCH_CASE(5);
+    XRH_PATCH_CASE(7);
+    XRH_PATCH_CASE(9);
+    XRH_PATCH_CASE(11);
+    XRH_PATCH_CASE(13);
+    XRH_PATCH_CASE(15);
+    XRH_PATCH_CASE(17);
     default: fail(XRH_ERR_INVALID, "no specialised patch kernel for this diameter");
   }
+#undef XRH_PATCH_CASE
 }
 
 void launch_sim(int key, const SimItem* items_dev, int64_t n_items, int max_img_tiles,
@@ -899,7 +941,8 @@ void launch_sim(int key, const SimItem* items_dev, int64_t n_items, int max_img_
   const int metric = key & ((1 << kSimKeyShift) - 1);
   // compile-time patch diameter (0: the general patch kernel) and blur radius of the group
   const int dfix = (key >> kSimKeyShift) & ((1 << (kSimKeyBlurShift - kSimKeyShift)) - 1);
-  const int rb = key >> kSimKeyBlurShift;
+  const int rb = (key & ~kSimKeyMask) >> kSimKeyBlurShift;
+  const bool masked = (key & kSimKeyMask) != 0;
   XRH_REQUIRE(n_items < 65536, "too many moving images in one similarity launch");
   const bool patch = (metric == XRH_SIM_PATCH_NCC || metric == XRH_SIM_PATCH_GRAD_NCC);
   const int ptiles = patch ? max_patch_tiles : max_img_tiles;
@@ -914,7 +957,8 @@ void launch_sim(int key, const SimItem* items_dev, int64_t n_items, int max_img_
       break;
     case XRH_SIM_PATCH_NCC:
       if (dfix) {
-        launch_patch_d<false>(dfix, grid, patch_lds_bytes, s, items_dev, partials, ptiles);
+        auto* launch = masked ? launch_patch_d<false, true> : launch_patch_d<false, false>;
+        launch(dfix, grid, patch_lds_bytes, s, items_dev, partials, ptiles);
       } else {
         hipLaunchKernelGGL(patch_kernel<false>, grid, dim3(kThreads), patch_lds_bytes, s, items_dev, partials, ptiles);
       }
@@ -923,7 +967,8 @@ void launch_sim(int key, const SimItem* items_dev, int64_t n_items, int max_img_
       XRH_BLUR_DISPATCH(rb, grad_images_kernel, dim3(xcd_grid_x(max_img_tiles), (unsigned)n_items), dim3(kThreads), 0,
                         s, items_dev);
       if (dfix) {
-        launch_patch_d<true>(dfix, grid, patch_lds_bytes, s, items_dev, partials, ptiles);
+        auto* launch = masked ? launch_patch_d<true, true> : launch_patch_d<true, false>;
+        launch(dfix, grid, patch_lds_bytes, s, items_dev, partials, ptiles);
       } else {
         hipLaunchKernelGGL(patch_kernel<true>, grid, dim3(kThreads), patch_lds_bytes, s, items_dev, partials, ptiles);
       }
@@ -1262,7 +1307,7 @@ static void sim_compute(xrh_ctx* ctx, const xrh_fixed* fixed, const float* mov_d
   if (scores_host_out) {
     // the general patch kernel writes the per-patch scores: clear the group key's diameter
     const int dmask = ((1 << (kSimKeyBlurShift - kSimKeyShift)) - 1) << kSimKeyShift;
-    key &= ~dmask;
+    key &= ~(dmask | kSimKeyMask);
   }
   launch_sim(key, (const SimItem*)(dev + off_items), num_mov, img_tiles, ptiles, (double*)(dev + off_part), sims,
              false, sim_patch_lds_bytes(h, scores_host_out != nullptr), ctx->stream);
