@@ -239,13 +239,14 @@ struct TileRef {
   bool valid;
 };
 
+// `split`: consecutive workgroups of a band that share a tile.
 __device__ inline TileRef decode_tile(const uint32_t* band_start, int64_t num_items, int bands,
-                                      const DrrItem* items, int stride = 1)
+                                      const DrrItem* items, int stride = 1, int split = 1)
 {
   TileRef t;
   const uint32_t b = blockIdx.x;
   const int band = (int)(b % (uint32_t)bands);
-  const uint32_t j = b / (uint32_t)bands;
+  const uint32_t j = b / (uint32_t)bands / (uint32_t)split;
   const uint32_t* bs = band_start + (int64_t)band * (num_items + 1);
   t.valid = j < bs[num_items];
   if (!t.valid) return t;
