@@ -249,14 +249,48 @@ __device__ inline double wave_sum_d(double v)
 // ---------------------------------------------------------------------------------------
 // kernels
 
-__global__ void drr_setup_kernel(const PoseIn* __restrict__ poses, const VolDesc* __restrict__ vols,
-                                 const CamDev* __restrict__ cams, DrrItem* __restrict__ items,
-                                 int64_t n)
+constexpr int kSetupItems = 8, kSetupThreads = 64, kSetupCopy = 256;  // items, lanes, words copied per workgroup
+
+__global__ __launch_bounds__(kSetupThreads) void drr_setup_kernel(const PoseIn* __restrict__ poses,
+                                                                  const VolDesc* __restrict__ vols,
+                                                                  const CamDev* __restrict__ cams,
+                                                                  DrrItem* __restrict__ items, int64_t n,
+                                                                  int item_blocks, SetupCopy copy)
 {
 #pragma clang fp contract(off)
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const PoseIn& p = poses[i];
+  constexpr int kWords = (int)sizeof(PoseIn) / 8, kLoads = (kSetupItems * kWords + kSetupThreads - 1) / kSetupThreads;
+  static_assert(sizeof(PoseIn) % 8 == 0, "poses are read in 8-byte words");
+  const int tid = threadIdx.x;
+  if ((int)blockIdx.x >= item_blocks) {
+    const uint64_t w0 = (uint64_t)(blockIdx.x - item_blocks) * kSetupCopy;
+#pragma unroll
+    for (int k = 0; k < kSetupCopy / kSetupThreads; ++k) {
+      const uint64_t w = w0 + (uint64_t)(k * kSetupThreads + tid);
+      if (w < copy.words[0]) copy.dst[0][w] = copy.src[0][w];
+      else if (w - copy.words[0] < copy.words[1]) copy.dst[1][w - copy.words[0]] = copy.src[1][w - copy.words[0]];
+    }
+    return;
+  }
+  // the workgroup's poses, read together: they may be in host memory
+  __shared__ uint64_t words[kSetupItems * kWords];
+  const int64_t i0 = (int64_t)blockIdx.x * kSetupItems;
+  const int m = (int)min((int64_t)kSetupItems, n - i0);
+  uint64_t buf[kLoads];
+#pragma unroll
+  for (int k = 0; k < kLoads; ++k) {
+    const int w = k * kSetupThreads + tid;
+    buf[k] = (w < m * kWords) ? ((const uint64_t*)(poses + i0))[w] : 0;
+  }
+#pragma unroll
+  for (int k = 0; k < kLoads; ++k) {
+    const int w = k * kSetupThreads + tid;
+    if (w < m * kWords) words[w] = buf[k];
+  }
+  __syncthreads();
+  if (tid >= m) return;
+  const int64_t i = i0 + tid;
+  PoseIn p;
+  __builtin_memcpy(&p, &words[tid * kWords], sizeof(PoseIn));
   const VolDesc& v = vols[p.vol];
   DrrItem it;
   // phys->idx * cam->phys: Affine*Affine product (xregRayCastLineIntCPU.cpp:207-208), float
@@ -1186,14 +1220,14 @@ TilePlan build_tiles(const std::vector<int32_t>& rows, const std::vector<int32_t
   return p;
 }
 
-void launch_drr_setup(const DrrLaunch& L, hipStream_t s)
+void launch_drr_setup(const DrrLaunch& L, hipStream_t s, const SetupCopy& copy)
 {
   if (L.num_items <= 0) return;
   const int64_t entries = L.num_items * (L.objs > 1 ? L.objs : 1);
-  const int threads = 64;
-  const int blocks = (int)((entries + threads - 1) / threads);
-  hipLaunchKernelGGL(drr_setup_kernel, dim3(blocks), dim3(threads), 0, s, L.poses_dev, L.vols_dev,
-                     L.cams_dev, L.items_dev, entries);
+  const int64_t item_blocks = (entries + kSetupItems - 1) / kSetupItems;
+  const int64_t copy_blocks = (int64_t)((copy.words[0] + copy.words[1] + kSetupCopy - 1) / kSetupCopy);
+  hipLaunchKernelGGL(drr_setup_kernel, dim3((unsigned)(item_blocks + copy_blocks)), dim3(kSetupThreads), 0, s,
+                     L.poses_dev, L.vols_dev, L.cams_dev, L.items_dev, entries, (int)item_blocks, copy);
   XRH_HIP_CHECK(hipGetLastError());
 }
 

@@ -330,7 +330,14 @@ std::string drr_tune_key(int32_t storage, int32_t layout, int32_t geom, int32_t 
 // Whether an untuned launch of `workgroups` workgroups marches whole rays (reuse = -1).
 bool drr_default_reuse(int64_t workgroups);
 constexpr int32_t kMaxDrrBands = 16;
-void launch_drr_setup(const DrrLaunch& L, hipStream_t s);
+// Words copied beside the set-up, from pinned host memory into device memory.
+struct SetupCopy {
+  const uint64_t* src[2] = {};
+  uint64_t* dst[2] = {};
+  uint64_t words[2] = {};
+};
+// `poses_dev` may be pinned host memory that the device can read.
+void launch_drr_setup(const DrrLaunch& L, hipStream_t s, const SetupCopy& copy = SetupCopy());
 void launch_drr(const DrrLaunch& L, hipStream_t s);
 // Casts with RayCasterLineIntCPU's sampling options (xrh_interp.hip). interp_prepare builds the
 // grid `interp` reads, once per volume (synchronous; allocates from the volume's context; the

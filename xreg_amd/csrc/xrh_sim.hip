@@ -805,48 +805,63 @@ __device__ inline double ncc_from_sums(double s1, double s2, double sf, double n
   return (1.0 - ncc) * 0.5;
 }
 
-// finish: one wave per item sums the tile records in a fixed order
-__global__ void finish_kernel(const SimItem* __restrict__ items, const double* __restrict__ partials,
-                              int ptiles, int stride_rec, float* __restrict__ sim_out, int64_t n_items)
+// finish: a workgroup per item sums the tile records (kRec doubles each, kSums of them used) in a
+// fixed order and writes the image's similarity, which may be in host memory. A single image is all
+// latency: four waves and records read as whole 16-byte pairs, with the loop unrolled, took 576 patch
+// tiles from 6.5 to 4.0 us.
+constexpr int kFinishThreads = 256;
+
+template <int kRec, int kSums>
+__global__ __launch_bounds__(kFinishThreads) void finish_kernel(const SimItem* __restrict__ items,
+                                                                const double* __restrict__ partials, int ptiles,
+                                                                float* __restrict__ sim_out, int64_t n_items)
 {
+  constexpr int kPairs = (kSums + 1) / 2, kWaves = kFinishThreads / 64;
   const int64_t item = blockIdx.x;
   if (item >= n_items) return;
   const SimItem it = items[item];
   const FixedDev& fx = *it.fixed;
-  int ntiles;
-  if (fx.metric == XRH_SIM_PATCH_NCC || fx.metric == XRH_SIM_PATCH_GRAD_NCC) {
-    ntiles = ((fx.ppr + kT - 1) / kT) * ((fx.ppc + kT - 1) / kT);
-  } else {
-    ntiles = ((fx.cols + kT - 1) / kT) * ((fx.rows + kT - 1) / kT);
+  const int ntiles = (kRec == 2) ? ((fx.ppr + kT - 1) / kT) * ((fx.ppc + kT - 1) / kT)
+                                 : ((fx.cols + kT - 1) / kT) * ((fx.rows + kT - 1) / kT);
+  double acc[2 * kPairs] = {};
+  const double2* base = (const double2*)(partials + it.out_index * ptiles * kRec);
+#pragma unroll 4
+  for (int t = threadIdx.x; t < ntiles; t += kFinishThreads) {
+#pragma unroll
+    for (int k = 0; k < kPairs; ++k) {
+      const double2 v = base[(int64_t)t * (kRec / 2) + k];
+      acc[2 * k] += v.x;
+      acc[2 * k + 1] += v.y;
+    }
   }
-  double acc[6] = {0, 0, 0, 0, 0, 0};
-  const double* base = partials + it.out_index * ptiles * stride_rec;
-  for (int t = threadIdx.x; t < ntiles; t += 64) {
-    for (int k = 0; k < 6 && k < stride_rec; ++k) acc[k] += base[(int64_t)t * stride_rec + k];
+  __shared__ double red[kWaves][kSums];
+#pragma unroll
+  for (int k = 0; k < kSums; ++k) {
+    const double w = wave_sum(acc[k]);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = w;
   }
-  for (int k = 0; k < 6; ++k) acc[k] = wave_sum(acc[k]);
+  __syncthreads();
   if (threadIdx.x != 0) return;
+#pragma unroll
+  for (int k = 0; k < kSums; ++k) {
+    acc[k] = 0.0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) acc[k] += red[w][k];
+  }
   double sim = 0.0;
   const double n = (double)fx.count;
-  switch (fx.metric) {
-    case XRH_SIM_NCC:
-      sim = ncc_from_sums(acc[0], acc[1], acc[2], n, fx.sum_zf, fx.std_f);
-      break;
-    case XRH_SIM_GRAD_NCC: {
-      const float sx = (float)ncc_from_sums(acc[0], acc[1], acc[2], n, fx.sum_zf, fx.std_f);
-      const float sy = (float)ncc_from_sums(acc[3], acc[4], acc[5], n, fx.sum_zfy, fx.std_fy);
-      sim = 0.5 * (double)(sx + sy);
-      break;
-    }
-    case XRH_SIM_PATCH_NCC:
-      sim = (acc[0] + fx.patch_offset[0]) / fx.patch_norm[0];
-      break;
-    default: {
-      const float sx = (float)((acc[0] + fx.patch_offset[0]) / fx.patch_norm[0]);
-      const float sy = (float)((acc[1] + fx.patch_offset[1]) / fx.patch_norm[1]);
-      sim = 0.5 * (double)(sx + sy);
-      break;
-    }
+  if constexpr (kRec == 4) {
+    sim = ncc_from_sums(acc[0], acc[1], acc[2], n, fx.sum_zf, fx.std_f);
+  } else if constexpr (kRec == 8) {
+    const float sx = (float)ncc_from_sums(acc[0], acc[1], acc[2], n, fx.sum_zf, fx.std_f);
+    const float sy = (float)ncc_from_sums(acc[3], acc[4], acc[5], n, fx.sum_zfy, fx.std_fy);
+    sim = 0.5 * (double)(sx + sy);
+  } else if (fx.metric == XRH_SIM_PATCH_NCC) {
+    sim = (acc[0] + fx.patch_offset[0]) / fx.patch_norm[0];
+  } else {
+    const float sx = (float)((acc[0] + fx.patch_offset[0]) / fx.patch_norm[0]);
+    const float sy = (float)((acc[1] + fx.patch_offset[1]) / fx.patch_norm[1]);
+    sim = 0.5 * (double)(sx + sy);
   }
   sim_out[it.out_index] = (float)sim;
 }
@@ -947,7 +962,6 @@ void launch_sim(int key, const SimItem* items_dev, int64_t n_items, int max_img_
   const bool patch = (metric == XRH_SIM_PATCH_NCC || metric == XRH_SIM_PATCH_GRAD_NCC);
   const int ptiles = patch ? max_patch_tiles : max_img_tiles;
   const dim3 grid(xcd_grid_x(ptiles), (unsigned)n_items);
-  const int rec = sim_record_stride(metric);
   switch (metric) {
     case XRH_SIM_NCC:
       if (!fused_ncc_done) hipLaunchKernelGGL(ncc_sums_kernel, grid, dim3(kThreads), 0, s, items_dev, partials, ptiles);
@@ -977,7 +991,9 @@ void launch_sim(int key, const SimItem* items_dev, int64_t n_items, int max_img_
       fail(XRH_ERR_INVALID, "unknown similarity metric");
   }
   XRH_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(finish_kernel, dim3((unsigned)n_items), dim3(64), 0, s, items_dev, partials, ptiles, rec,
+  auto* finish = (metric == XRH_SIM_NCC) ? finish_kernel<4, 3>
+                 : (metric == XRH_SIM_GRAD_NCC) ? finish_kernel<8, 6> : finish_kernel<2, 2>;
+  hipLaunchKernelGGL(finish, dim3((unsigned)n_items), dim3(kFinishThreads), 0, s, items_dev, partials, ptiles,
                      sim_out_dev, n_items);
   XRH_HIP_CHECK(hipGetLastError());
 }
