@@ -399,7 +399,7 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
   D.ncc_tiles_per_item = b->max_img_tiles;
   D.ray_spacing = (float)(spacing / (double)(n * objs));
   D.vol_bytes = vol_bytes;
-  b->last_slab = drr_slab_lds(D.ray_spacing, b->geom, vol_bytes);
+  b->last_slab = drr_slab_lds(D.ray_spacing, b->geom, vol_bytes, b->storage);
   D.reuse = var.reuse;
   D.wave_shape = var.shape;
   D.objs = objs;

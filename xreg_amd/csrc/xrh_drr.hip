@@ -37,7 +37,8 @@ namespace {
 // ---------------------------------------------------------------------------------------
 // trilinear sampling per layout. Formats: 0 f32 linear, 1 f32 quad, 2 f16 linear, 3 f16 oct,
 // 4 bf16 linear, 5 bf16 oct, sampled one by one; 7 f32 coefficients, 11 f32 x-faces, 13 f32
-// x-faces in bricks, fetched cell by cell (two 16-byte loads) and marched with march_cells.
+// x-faces in bricks, fetched cell by cell (two 16-byte loads) and marched with march_cells. (16-bit oct
+// cells, one load each, are faster sample by sample: 0.315 ns per ray against 0.353 by cells.)
 constexpr bool is_cell_fmt(int fmt) { return fmt == 7 || fmt == 11 || fmt == 13; }
 
 struct VolView {
@@ -65,6 +66,32 @@ __device__ inline float tri(float v000, float v100, float v010, float v110, floa
   return lerp(xx0, xx1, wz);
 }
 
+// The same for corners of 16-bit storage: their differences along x are exact in FP32 (11 or 8 bits of
+// significand, unless one is over 2^13 times the other), so a + w (b - a) is rounded once. Two samples
+// of one cell share them.
+__device__ inline float tri16_x(float v000, float d00, float v010, float d10, float v001, float d01, float v011,
+                                float d11, float wx, float wy, float wz)
+{
+  const float xx0 = lerp(fmaf(wx, d00, v000), fmaf(wx, d10, v010), wy);
+  const float xx1 = lerp(fmaf(wx, d01, v001), fmaf(wx, d11, v011), wy);
+  return lerp(xx0, xx1, wz);
+}
+
+__device__ inline float tri16(float v000, float v100, float v010, float v110, float v001,
+                              float v101, float v011, float v111, float wx, float wy, float wz)
+{
+  return tri16_x(v000, v100 - v000, v010, v110 - v010, v001, v101 - v001, v011, v111 - v011, wx, wy, wz);
+}
+
+// The high minus the low half of a word, both f16, in FP32 (V_FMA_MIX_F32 converts its operands; from
+// two conversions and a subtraction the compiler does not form it, and the gathering march over 256 x
+// 256 x 200 f16 voxels takes 0.402 instead of 0.315 ns per ray).
+__device__ inline float half_diff(uint32_t w)
+{
+  float d;
+  asm("v_fma_mix_f32 %0, %1, 1.0, -%1 op_sel:[1,0,0] op_sel_hi:[1,0,1]" : "=v"(d) : "v"(w));
+  return d;
+}
 
 // floor(x) converted to int in one instruction (V_CVT_FLR_I32_F32). Inline asm counts as
 // convergent, so the sample loops below are unrolled by hand.
@@ -158,18 +185,22 @@ __device__ inline float sample(const VolView& v, float x, float y, float z)
     float f[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) f[i] = (kFmt == 2) ? h2f(r[i]) : bf2f(r[i]);
-    return tri(f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7], wx, wy, wz);
+    return tri16(f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7], wx, wy, wz);
   } else {
     const int o = (int)(e * 16u);
     const auto q = __builtin_amdgcn_raw_buffer_load_b128(v.rsrc, o, 0, 0);
-    float f[8];
+    float f[4], d[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint32_t lo = q[i] & 0xffffu, hi = q[i] >> 16;
-      f[2 * i] = (kFmt == 3) ? h2f(lo) : bf2f(lo);
-      f[2 * i + 1] = (kFmt == 3) ? h2f(hi) : bf2f(hi);
+      if constexpr (kFmt == 3) {
+        f[i] = h2f(q[i] & 0xffffu);
+        d[i] = half_diff(q[i]);
+      } else {
+        f[i] = bf2f(q[i] & 0xffffu);
+        d[i] = bf2f(q[i] >> 16) - f[i];
+      }
     }
-    return tri(f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7], wx, wy, wz);
+    return tri16_x(f[0], d[0], f[1], d[1], f[2], d[2], f[3], d[3], wx, wy, wz);
   }
 }
 
@@ -648,8 +679,9 @@ __device__ __forceinline__ float cast_ray(const DrrItem& it, int col, int row, b
 // The box comes from the tile's corner rays: the pixel -> position map on a plane across the main
 // axis is projective, so the corners' positions on the slab's two planes bound every ray between
 // them. Slabs end on cell faces, so no cell straddles two. A cell's face coefficients are formed
-// from its voxels by the float operations that built the face layout, and samples pair and
-// segment as in march_cells: the values are the gathering march's bit for bit, and tiles whose box
+// from its voxels by the float operations that built the face layout (16-bit storage: the gathering
+// march's lerps, from voxels kept as floats), and samples segment as there: the values are the
+// gathering march's bit for bit, and tiles whose box
 // does not fit (rays several voxels apart, oblique tiles) take that march.
 //
 // Measured, FP64 set-up, ns per ray, gathering sample by sample (before) / by cells / slabs: 256 x
@@ -730,7 +762,7 @@ __device__ inline LdsPair lds_pair(int addr)
 
 // cast_ray by slabs. Every thread of the block calls it (it synchronises); `lds` holds `budget`
 // floats.
-template <int kGeom, int kOp>
+template <int kGeom, int kOp, int kFmt>
 __device__ __forceinline__ float cast_ray_slab(const DrrItem& it, const TileRef& tr, int col, int row, bool inside,
                                       float* lds, int budget)
 {
@@ -836,7 +868,7 @@ __device__ __forceinline__ float cast_ray_slab(const DrrItem& it, const TileRef&
       if (b0.wx <= 256 && b1.wx <= 256 && b0.floats() <= budget && b1.floats() <= budget) break;
     }
   }
-  if (depth < 2) return cast_range<kGeom, kOp, 11>(it, ray, first, last);
+  if (depth < 2) return cast_range<kGeom, kOp, kFmt>(it, ray, first, last);
 
   const auto src = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(it.raw), (short)0, (int)it.raw_bytes, 0x00020000);
   const float flast = (float)last, fseg_len = (float)seg_len(ray.n);
@@ -895,15 +927,26 @@ __device__ __forceinline__ float cast_ray_slab(const DrrItem& it, const TileRef&
         const int c10 = c00 + py, c01 = c00 + pz, c11 = c10 + pz;
         float va[4], vb[4];
         const LdsPair r00 = lds_pair(c00), r10 = lds_pair(c10), r01 = lds_pair(c01), r11 = lds_pair(c11);
-        va[0] = r00.a;
-        vb[0] = r00.b;
-        va[1] = r10.a - r00.a;
-        vb[1] = r10.b - r00.b;
-        va[2] = r01.a - r00.a;
-        vb[2] = r01.b - r00.b;
-        va[3] = (r11.a - r01.a) - va[1];
-        vb[3] = (r11.b - r01.b) - vb[1];
-        acc = line_op<kOp>(acc, cell_value<11>(va, vb, wx, wy, wz));
+        if constexpr (kFmt == 11) {
+          va[0] = r00.a;
+          vb[0] = r00.b;
+          va[1] = r10.a - r00.a;
+          vb[1] = r10.b - r00.b;
+          va[2] = r01.a - r00.a;
+          vb[2] = r01.b - r00.b;
+          va[3] = (r11.a - r01.a) - va[1];
+          vb[3] = (r11.b - r01.b) - vb[1];
+        } else {
+          va[0] = r00.b - r00.a;
+          va[1] = r10.b - r10.a;
+          va[2] = r01.b - r01.a;
+          va[3] = r11.b - r11.a;
+        }
+        auto value = [&] {
+          if constexpr (kFmt == 11) return cell_value<11>(va, vb, wx, wy, wz);
+          else return tri16_x(r00.a, va[0], r10.a, va[1], r01.a, va[2], r11.a, va[3], wx, wy, wz);
+        };
+        acc = line_op<kOp>(acc, value());
         f = f + 1.0f;
         if constexpr (kGeom == XRH_GEOM_FP32) {
           const float bx = x - wx, by = y - wy, bz = z - wz;  // floor
@@ -912,6 +955,11 @@ __device__ __forceinline__ float cast_ray_slab(const DrrItem& it, const TileRef&
           wx = pos.x - bx;
           wy = pos.y - by;
           wz = pos.z - bz;
+        } else if constexpr (kFmt != 11) {
+          // as the gathering march of these formats, from the sample's own position
+          wx = fmaf(f, ray.dx, ray.sx) - (x - wx);
+          wy = fmaf(f, ray.dy, ray.sy) - (y - wy);
+          wz = fmaf(f, ray.dz, ray.sz) - (z - wz);
         } else {
           wx = wx + ray.dx;
           wy = wy + ray.dy;
@@ -919,7 +967,7 @@ __device__ __forceinline__ float cast_ray_slab(const DrrItem& it, const TileRef&
         }
         const uint32_t top = max(max(__float_as_uint(wx), __float_as_uint(wy)), __float_as_uint(wz));
         if (top < 0x3f800000u && f <= fseg) {
-          acc = line_op<kOp>(acc, cell_value<11>(va, vb, wx, wy, wz));
+          acc = line_op<kOp>(acc, value());
           f = f + 1.0f;
           if constexpr (kGeom == XRH_GEOM_FP32) {
             pos.advance(ray, 1);
@@ -998,7 +1046,7 @@ __device__ __forceinline__ float cast_pixel(const DrrItem& it, const TileRef& tr
 {
   if constexpr (kParts == 0) {
     extern __shared__ __attribute__((aligned(16))) float slab_lds[];
-    return cast_ray_slab<kGeom, kOp>(it, tr, col, row, inside, slab_lds, budget);
+    return cast_ray_slab<kGeom, kOp, kFmt>(it, tr, col, row, inside, slab_lds, budget);
   } else if constexpr (kParts == 1) return cast_ray<kGeom, kOp, kFmt>(it, col, row, inside);
   else return cast_ray_split<kGeom, kOp, kFmt, kParts>(it, col, row, inside);
 }
@@ -1146,9 +1194,11 @@ void launch_fmt(const DrrLaunch& L, dim3 grid, hipStream_t s, int accumulate, fl
                                                                                 : (L.layout == kLayoutQuad ? 1 : 0))))
                 : (L.storage == XRH_F16) ? (L.layout == kLayoutOct ? 3 : 2)
                                          : (L.layout == kLayoutOct ? 5 : 4);
-  const int slab = drr_slab_lds(L.ray_spacing, L.geom, L.vol_bytes);
-  if (fmt == 11 && parts == 1 && slab > 0) {
-    XRH_LAUNCH_PARTS(11, 0);
+  const int slab = drr_slab_lds(L.ray_spacing, L.geom, L.vol_bytes, L.storage);
+  if (parts == 1 && slab > 0 && (fmt == 11 || fmt == 3 || fmt == 5)) {
+    if (fmt == 11) XRH_LAUNCH_PARTS(11, 0);
+    else if (fmt == 3) XRH_LAUNCH_PARTS(3, 0);
+    else XRH_LAUNCH_PARTS(5, 0);
     return;
   }
   switch (fmt) {
@@ -1179,10 +1229,23 @@ void launch_fmt(const DrrLaunch& L, dim3 grid, hipStream_t s, int accumulate, fl
 // 40 / 54 KB: 256 x 256 x 200 voxels at 0.58 voxels 0.397 / 0.485 / 0.758, at 0.78 0.440 / 0.516 /
 // 0.828, at 1.16 0.787 / 0.625 / 0.940, at 1.55 1.30 / 1.05 / 1.29, at 2.3 2.22 / 1.91 / 2.28; 512 x
 // 512 x 400 voxels at 3.1 6.06 / 5.66 / 5.32.
-int drr_slab_lds(float spacing, int32_t geom, uint64_t bytes)
+//
+// With 16-bit storage a gathered sample is one load instead of an FP32 cell's two, so slabs pay later
+// (ns per ray by gathering / slabs, f16): 215 MB, FP64 set-up, at 0.19 voxels 0.315 / 0.316, 0.39 0.348 /
+// 0.360, 0.58 0.364 / 0.401, 0.78 0.495 / 0.440, 1.55 1.31 / 1.02; FP32 set-up 0.39 0.32 / 0.38, 0.78
+// 0.49 / 0.45, 1.55 1.29 / 1.05. 1.7 GB, FP64: 0.39 0.65 / 0.60, 0.78 1.13 / 0.80, 1.55 3.1 / 1.8. 26
+// MB: 0.39 0.209 / 0.219, 0.78 0.233 / 0.279, 1.55 0.47 / 0.62.
+int drr_slab_lds(float spacing, int32_t geom, uint64_t bytes, int32_t storage)
 {
   if (!(spacing > 0.0f)) return 0;
-  if (spacing < 0.5f && bytes < (geom == XRH_GEOM_FP32 ? (256ull << 20) : (64ull << 20))) return 0;
+  const bool fp32 = geom == XRH_GEOM_FP32;
+  if (storage == XRH_F32) {
+    if (spacing < 0.5f && bytes < (fp32 ? (256ull << 20) : (64ull << 20))) return 0;
+  } else if (bytes < (64ull << 20)) {
+    return 0;
+  } else if (spacing < 0.7f && (fp32 || bytes < (512ull << 20))) {
+    return 0;
+  }
   return spacing < 0.95f ? 20224 : (spacing < 2.7f ? 40704 : 54272);
 }
 

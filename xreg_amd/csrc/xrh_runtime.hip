@@ -1,5 +1,6 @@
 // xrh_runtime.hip -- context, budgeted device memory, resident volumes and xrh_line_int.
 #include "xrh_internal.h"
+#include "xrh_ray.h"
 
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
@@ -214,7 +215,10 @@ __device__ inline float4 face(float v00, float v10, float v01, float v11)
   return make_float4(v00, c1, v01 - v00, (v11 - v01) - c1);
 }
 
-// Builds the padded layout from the raw x-fastest volume. One thread per padded voxel.
+// Builds the padded layout from the raw x-fastest volume. One thread per padded voxel. kLayoutPlain:
+// the values that the storage type holds, as floats.
+constexpr int kLayoutPlain = -1;
+
 __global__ void build_layout_kernel(const float* __restrict__ src, int X, int Y, int Z,
                                     void* __restrict__ dst, int storage, int layout)
 {
@@ -232,7 +236,10 @@ __global__ void build_layout_kernel(const float* __restrict__ src, int X, int Y,
     int z = min(max(cc - 1, 0), Z - 1);
     return src[(int64_t)x + (int64_t)X * ((int64_t)y + (int64_t)Y * z)];
   };
-  if (layout == kLayoutLinear) {
+  if (layout == kLayoutPlain) {
+    const float v = V(a, b, c);
+    ((float*)dst)[i] = (storage == XRH_F32) ? v : (storage == XRH_F16) ? h2f(f2h_bits(v)) : bf2f(f2bf_bits(v));
+  } else if (layout == kLayoutLinear) {
     const float v = V(a, b, c);
     if (storage == XRH_F32) ((float*)dst)[i] = v;
     else if (storage == XRH_F16) ((uint16_t*)dst)[i] = f2h_bits(v);
@@ -456,10 +463,10 @@ static void volume_create(xrh_ctx* ctx, const float* vox, const int64_t size[3],
   const int64_t sgx = (X + SB - 1) / SB, sgy = (Y + SB - 1) / SB, sgz = (Z + SB - 1) / SB, nb = sgx * sgy * sgz;
   // the walk indexes the map with 24-bit multiply-adds: larger maps go without skipping
   const bool skip = skip_enabled() && nb < (int64_t(1) << 24) && sgy * sgz < (int64_t(1) << 24);
-  // one allocation: the layout, the empty-space map and the plain voxels beside the faces. A context
+  // one allocation: the layout, the empty-space map and the plain voxels beside the packed layout. A context
   // with a budget goes without the plain voxels (4 bytes a voxel more, used by the slabs only), so
   // what fitted a budget without them fits it still
-  bool plain = layout == kLayoutFace && !ctx->budget;
+  bool plain = (layout == kLayoutFace || layout == kLayoutOct) && !ctx->budget;
   auto pad = [](uint64_t x) { return (x + 255) & ~uint64_t(255); };
   const uint64_t map_end = bytes + (skip ? (uint64_t)nb : 0), off_plain = pad(map_end);
   try {
@@ -514,7 +521,7 @@ static void volume_create(xrh_ctx* ctx, const float* vox, const int64_t size[3],
     XRH_HIP_CHECK(hipGetLastError());
     if (plain) {
       hipLaunchKernelGGL(build_layout_kernel, grid(padded), dim3(threads), 0, ctx->stream, (const float*)raw, (int)X,
-                         (int)Y, (int)Z, v->raw, storage, (int)kLayoutLinear);
+                         (int)Y, (int)Z, v->raw, storage, kLayoutPlain);
       XRH_HIP_CHECK(hipGetLastError());
     }
     XRH_HIP_CHECK(hipStreamSynchronize(ctx->stream));
