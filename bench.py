@@ -629,17 +629,17 @@ def main():
 
     # ---- roofline of the DRR kernel (the dominant kernel) ----
     # The DRR's gathers are served mostly by L1/L2/Infinity Cache (the C2 volume is cache
-    # resident), so the algorithmic gather bytes of the reference algorithm exceed what HBM
-    # moves; the bound that the counters show is vector-ALU issue. `achieved` is the kernel's
+    # resident) and LDS, so the algorithmic gather bytes of the reference algorithm exceed what HBM
+    # moves; the bound that the counters show is vector-ALU issue, with LDS reads close behind. `achieved` is the kernel's
     # VALU wave-instructions per launch (SQ_INSTS_VALU, rocprofv3, same configuration and kernel
-    # source) over its live-measured duration; `peak` is one VALU wave-instruction per CU per
-    # clock at the 2.4 GHz peak engine clock. `hbm_frac` is the measured HBM-side traffic
+    # source) over its live-measured duration; `peak` is two FP32 VALU wave-instructions per CU per
+    # clock (157 TFLOP/s as FMAs) at the 2.4 GHz peak engine clock. `hbm_frac` is the measured HBM-side traffic
     # (FETCH_SIZE + WRITE_SIZE, calibrated) over the same duration against 8 TB/s.
     key = (f"workload={workload} storage={args.storage} geometry={args.geom} skip={0 if args.no_skip else 1} "
            f"smooth={args.smooth} src={kernel_source_key()}")
     prof = profiled(key)
     cus = device_cus()
-    valu_peak = cus * PEAK_CLOCK_GHZ  # G wave-instructions / s
+    valu_peak = 2 * cus * PEAK_CLOCK_GHZ  # G wave-instructions / s
     valu_rate = prof["valu_insts"] / (drr_ms_avg * 1e-3) / 1e9 if "valu_insts" in prof else None
     traffic = prof.get("traffic_bytes")
     roofline = {"bound": "valu", "achieved": round(valu_rate, 1) if valu_rate else None, "peak": valu_peak,

@@ -176,7 +176,8 @@ xrh_status xrh_volume_create_layout(xrh_ctx* ctx, const float* vox, const int64_
 xrh_status xrh_volume_create_hu(xrh_ctx* ctx, const float* vox_hu, const int64_t size[3],
                                 const float idx_to_phys[16], int32_t storage, int32_t layout,
                                 double hu_lower, double mu_water, double mu_air, xrh_volume** out);
-/* Device bytes held by the volume (its layout, empty-space map and any interpolation grids). */
+/* Device bytes held by the volume: its layout, the plain voxels kept beside it (4 bytes per padded
+ * voxel of the default layouts; none in a context with an HBM budget) and any interpolation grids. */
 uint64_t xrh_volume_bytes(const xrh_volume* vol);
 /* Storage type and HBM layout a volume was built with (the automatic choice included: a
  * volume whose packed layout would pass 4 GiB is kept linear). Volumes batched together must

@@ -17,7 +17,10 @@
 //   - the volume sits in HBM in an edge-padded layout read through buffer loads
 //     (hardware range check: a stray offset returns 0, it can never fault); the quad (f32)
 //     and oct (f16/bf16) layouts pre-pack interpolation corners so a sample costs 2 or 1
-//     16-byte loads instead of 8 scalar gathers;
+//     16-byte loads instead of 8 scalar gathers, the face layout (f32, the default) two loads
+//     per cell;
+//   - large launches march by slabs of the volume staged in LDS where that is the faster way
+//     (drr_slab_lds); in small ones two or four waves share a ray (drr_parts);
 //   - trilinear weights and lerps are FP32 in software: HIP's image/texture API is not
 //     available for gfx950 (hipcc rejects tex3D for this target), so there is no hardware
 //     filtering to fall back on.

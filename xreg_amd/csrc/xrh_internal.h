@@ -151,8 +151,8 @@ struct VolDesc {
   // null when skipping is disabled
   const uint8_t* skip;
   int32_t skip_gx, skip_gy, skip_gz, skip_shift;
-  // the padded voxels themselves (kLayoutLinear's arrangement) beside a packed FP32 layout, for
-  // slab marching; null without
+  // the padded voxels themselves as floats (of 16-bit storage, the rounded values; kLayoutLinear's
+  // arrangement) beside the face or oct layout, for slab marching; null without
   const void* raw;
   uint32_t raw_bytes;
   int32_t pad2_;
