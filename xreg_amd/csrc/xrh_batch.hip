@@ -70,7 +70,7 @@ struct xrh_batch {
   bool variant_set = false;
   DrrVariant variant;
   DrrVariant last_variant;         // the variant of the last staged launch
-  int32_t last_slab = 0;           // and its slab-marching choice
+  int64_t last_plan = 0;           // and its default way of marching
 };
 
 namespace {
@@ -399,7 +399,7 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
   D.ncc_tiles_per_item = b->max_img_tiles;
   D.ray_spacing = (float)(spacing / (double)(n * objs));
   D.vol_bytes = vol_bytes;
-  b->last_slab = drr_slab_lds(D.ray_spacing, b->geom, vol_bytes, b->storage);
+  b->last_plan = drr_launch_plan(D);
   D.reuse = var.reuse;
   D.wave_shape = var.shape;
   D.objs = objs;
@@ -454,7 +454,7 @@ std::string signature(const xrh_batch* b, const int32_t* item_view, int64_t n, c
   key.append((const char*)&drr_out, sizeof(drr_out));
   key.append((const char*)&b->version, sizeof(b->version));
   key.append((const char*)&b->last_variant, sizeof(b->last_variant));
-  key.append((const char*)&b->last_slab, sizeof(b->last_slab));
+  key.append((const char*)&b->last_plan, sizeof(b->last_plan));
   return key;
 }
 

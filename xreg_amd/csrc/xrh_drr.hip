@@ -1048,8 +1048,8 @@ template <int kGeom, int kOp, int kFmt, int kParts>
 __device__ __forceinline__ float cast_pixel(const DrrItem& it, const TileRef& tr, int col, int row, bool inside, int budget)
 {
   if constexpr (kParts == 0) {
-    extern __shared__ __attribute__((aligned(16))) float slab_lds[];
-    return cast_ray_slab<kGeom, kOp, kFmt>(it, tr, col, row, inside, slab_lds, budget);
+    extern __shared__ __attribute__((aligned(16))) float box_lds[];
+    return cast_ray_slab<kGeom, kOp, kFmt>(it, tr, col, row, inside, box_lds, budget);
   } else if constexpr (kParts == 1) return cast_ray<kGeom, kOp, kFmt>(it, col, row, inside);
   else return cast_ray_split<kGeom, kOp, kFmt, kParts>(it, col, row, inside);
 }
@@ -1154,11 +1154,37 @@ int device_cus()
 // only pays for the shared set-up (30 items of 256 x 256, two objects: 1.07 ms whole, 1.22 ms by
 // two). One pose, FP64 set-up, DRR kernel: 192 x 192 over 128 x 128 x 96 voxels 30.5
 // whole, 27.2 by two, 21.4 by four; 384 x 384 over 256 x 256 x 200 voxels 102, 80, 90 us.
-int drr_parts(int64_t tiles)
+//
+// Rays `spacing` voxels apart (0: not known) share no cache lines, and waves at several depths of the
+// same rays then evict each other's: from 1.75 voxels on, and by two from 0.95 on, a wave takes whole
+// rays (us, shared / whole: 546 tiles at 1.94 voxels 478 / 386, 686 at 2.26 1037 / 790, 560 at 2.62 654 /
+// 500, 624 at 1.0 510 / 387; but 98 at 1.64 128 / 172, 324 at 1.16 180 / 226, 442 at 0.80 105 / 142).
+// Where rays are close and gather, sharing by two pays up to twice as many tiles (16-bit, whole / shared:
+// 1392 at 0.39 345 / 321, 1440 at 0.31 207 / 178, 1736 at 0.36 162 / 146, 1596 at 0.45 217 / 203).
+int drr_parts(int64_t tiles, float spacing, int slab)
 {
   const int64_t waves = tiles * (kThreads / 64), room = 32ll * device_cus();
-  return (waves * 4 <= room) ? 4 : (waves * 2 <= room) ? 2 : 1;
+  if (waves * 4 <= room) return spacing < 1.75f ? 4 : 1;
+  if (slab == 0 && spacing > 0.0f && spacing < 0.75f && waves <= room) return 2;
+  return (waves * 2 <= room && spacing < 0.95f) ? 2 : 1;
 }
+
+// LDS bytes of a workgroup's boxes for rays `spacing` voxels apart.
+int slab_lds(float spacing)
+{
+  return !(spacing > 0.0f) ? 0 : (spacing < 0.95f ? 20224 : (spacing < 2.7f ? 40704 : 54272));
+}
+
+}  // namespace
+
+int64_t drr_launch_plan(const DrrLaunch& L)
+{
+  const int64_t tiles = L.max_band_tiles * L.bands;
+  const int slab = drr_slab_lds(L.ray_spacing, L.geom, L.vol_bytes, L.storage, tiles);
+  return (int64_t)slab * 8 + drr_parts(tiles, L.ray_spacing, slab);
+}
+
+namespace {
 
 template <int kGeom, int kOp>
 void launch_fmt(const DrrLaunch& L, dim3 grid, hipStream_t s, int accumulate, float fill)
@@ -1183,12 +1209,11 @@ void launch_fmt(const DrrLaunch& L, dim3 grid, hipStream_t s, int accumulate, fl
     else if (parts == 2) XRH_LAUNCH_PARTS(F, 2);  \
     else XRH_LAUNCH_PARTS(F, 1);                  \
   } while (0)
-  // Waves per ray. XRH_CELL_REUSE=0 / =1 force shared / whole rays (read per launch, so a process
+  // Waves per ray. XRH_CELL_REUSE=0 / =1 force shared rays / slabs (read per launch, so a process
   // can switch between calls); otherwise a tuned variant decides, else the launch size.
   const char* reuse_env = std::getenv("XRH_CELL_REUSE");
   const int reuse = reuse_env ? (std::strcmp(reuse_env, "0") != 0 ? 1 : 0) : L.reuse;
   const int64_t tiles = (int64_t)grid.x * grid.y;
-  const int parts = (reuse > 0) ? 1 : (reuse == 0) ? std::max(drr_parts(tiles), 2) : drr_parts(tiles);
   const int shape = (L.wave_shape >= 0 && L.wave_shape <= 2) ? L.wave_shape : 0;
   const int fmt = (L.storage == XRH_F32)
                       ? (L.layout == kLayoutCoef ? 7
@@ -1197,7 +1222,11 @@ void launch_fmt(const DrrLaunch& L, dim3 grid, hipStream_t s, int accumulate, fl
                                                                                 : (L.layout == kLayoutQuad ? 1 : 0))))
                 : (L.storage == XRH_F16) ? (L.layout == kLayoutOct ? 3 : 2)
                                          : (L.layout == kLayoutOct ? 5 : 4);
-  const int slab = drr_slab_lds(L.ray_spacing, L.geom, L.vol_bytes, L.storage);
+  // (forced whole rays go by slabs whatever the sizes)
+  const int slab = (reuse_env && reuse > 0) ? slab_lds(L.ray_spacing)
+                                            : drr_slab_lds(L.ray_spacing, L.geom, L.vol_bytes, L.storage, tiles);
+  const int parts = (reuse > 0) ? 1 : (reuse == 0) ? std::max(drr_parts(tiles, 0.0f, 0), 2)
+                                                   : drr_parts(tiles, L.ray_spacing, slab);
   if (parts == 1 && slab > 0 && (fmt == 11 || fmt == 3 || fmt == 5)) {
     if (fmt == 11) XRH_LAUNCH_PARTS(11, 0);
     else if (fmt == 3) XRH_LAUNCH_PARTS(3, 0);
@@ -1233,26 +1262,30 @@ void launch_fmt(const DrrLaunch& L, dim3 grid, hipStream_t s, int accumulate, fl
 // 0.828, at 1.16 0.787 / 0.625 / 0.940, at 1.55 1.30 / 1.05 / 1.29, at 2.3 2.22 / 1.91 / 2.28; 512 x
 // 512 x 400 voxels at 3.1 6.06 / 5.66 / 5.32.
 //
+// Volumes of under 64 MB gather at any distance (40 MB, 2016 tiles at 0.70 voxels: 179 / 211 us).
 // With 16-bit storage a gathered sample is one load instead of an FP32 cell's two, so slabs pay later
 // (ns per ray by gathering / slabs, f16): 215 MB, FP64 set-up, at 0.19 voxels 0.315 / 0.316, 0.39 0.348 /
 // 0.360, 0.58 0.364 / 0.401, 0.78 0.495 / 0.440, 1.55 1.31 / 1.02; FP32 set-up 0.39 0.32 / 0.38, 0.78
 // 0.49 / 0.45, 1.55 1.29 / 1.05. 1.7 GB, FP64: 0.39 0.65 / 0.60, 0.78 1.13 / 0.80, 1.55 3.1 / 1.8. 26
-// MB: 0.39 0.209 / 0.219, 0.78 0.233 / 0.279, 1.55 0.47 / 0.62.
-int drr_slab_lds(float spacing, int32_t geom, uint64_t bytes, int32_t storage)
+// MB: 0.39 0.209 / 0.219, 0.78 0.233 / 0.279, 1.55 0.47 / 0.62. They also need more tiles, for the four
+// workgroups per CU that their boxes leave room for: 112 MB, 2360 tiles at 1.71 428 / 592 us; 289 MB,
+// 2430 at 0.84 339 / 382; 556 MB, 2112 at 1.60 1019 / 937.
+int drr_slab_lds(float spacing, int32_t geom, uint64_t bytes, int32_t storage, int64_t tiles)
 {
-  if (!(spacing > 0.0f)) return 0;
+  if (!(spacing > 0.0f) || bytes < (64ull << 20)) return 0;
   const bool fp32 = geom == XRH_GEOM_FP32;
   if (storage == XRH_F32) {
-    if (spacing < 0.5f && bytes < (fp32 ? (256ull << 20) : (64ull << 20))) return 0;
-  } else if (bytes < (64ull << 20)) {
-    return 0;
-  } else if (spacing < 0.7f && (fp32 || bytes < (512ull << 20))) {
-    return 0;
+    if (fp32 && spacing < 0.5f && bytes < (256ull << 20)) return 0;
+  } else {
+    const bool large = bytes >= (512ull << 20);
+    const int64_t cus = device_cus();
+    if (spacing < 0.7f && (fp32 || !large)) return 0;
+    if (tiles < (large ? 8 : 16) * cus || bytes < (128ull << 20)) return 0;
   }
-  return spacing < 0.95f ? 20224 : (spacing < 2.7f ? 40704 : 54272);
+  return slab_lds(spacing);
 }
 
-bool drr_default_reuse(int64_t workgroups) { return drr_parts(workgroups) == 1; }
+bool drr_default_reuse(int64_t workgroups) { return drr_parts(workgroups, 0.0f, 0) == 1; }
 
 std::string drr_tune_key(int32_t storage, int32_t layout, int32_t geom, int32_t kernel, int32_t max_rows,
                          int32_t max_cols, int64_t workgroups)

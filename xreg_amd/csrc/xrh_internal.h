@@ -321,7 +321,9 @@ struct DrrLaunch {
 // Key of the tuned-variant table: storage, layout, geometry, line kernel, the largest
 // detector of the launch and its workgroups per CU (rounded down to a power of two).
 // The slab-marching choice of a launch (its dynamic LDS bytes, 0: gathering).
-int drr_slab_lds(float spacing, int32_t geom, uint64_t bytes, int32_t storage);
+int drr_slab_lds(float spacing, int32_t geom, uint64_t bytes, int32_t storage, int64_t tiles);
+// The default way a launch marches, as one number (captured launches are kept by it).
+int64_t drr_launch_plan(const DrrLaunch& L);
 // Distance (voxels) of neighbouring rays at the volume's centre for a camera and a row-major
 // cam->phys pose.
 float ray_spacing(const xrh_volume* vol, const xrh_camera& cam, const double pose[16]);
