@@ -1156,15 +1156,22 @@ int device_cus()
 // whole, 27.2 by two, 21.4 by four; 384 x 384 over 256 x 256 x 200 voxels 102, 80, 90 us.
 //
 // Rays `spacing` voxels apart (0: not known) share no cache lines, and waves at several depths of the
-// same rays then evict each other's: from 1.75 voxels on, and by two from 0.95 on, a wave takes whole
-// rays (us, shared / whole: 546 tiles at 1.94 voxels 478 / 386, 686 at 2.26 1037 / 790, 560 at 2.62 654 /
-// 500, 624 at 1.0 510 / 387; but 98 at 1.64 128 / 172, 324 at 1.16 180 / 226, 442 at 0.80 105 / 142).
+// same rays then evict each other's: over 512 tiles a wave takes whole rays from 0.95 voxels on (us,
+// shared by two / whole: 546 tiles at 1.94 voxels 478 / 386, 686 at 2.26 1037 / 790, 624 at 1.0 510 /
+// 387); up to 512 FP32 rays are shared by four while there are few or they are close, else by two (four /
+// two: 252 tiles at 1.03 80 / 95, 98 at 1.64 129 / 132, 507 at 1.01 177 / 161; whole / two: 72 at 2.77 427 /
+// 260, 100 at 3.55 427 / 374, 200 at 2.66 339 / 275), and 16-bit rays, with half the loads, by four up to
+// 1.75 voxels (210 tiles at 1.67 four / two 111 / 117), from there by two only up to 128 tiles (whole / two:
+// 50 at 3.76 286 / 263, 280 at 3.22 267 / 281, 440 at 1.82 181 / 199).
 // Where rays are close and gather, sharing by two pays up to twice as many tiles (16-bit, whole / shared:
 // 1392 at 0.39 345 / 321, 1440 at 0.31 207 / 178, 1736 at 0.36 162 / 146, 1596 at 0.45 217 / 203).
-int drr_parts(int64_t tiles, float spacing, int slab)
+int drr_parts(int64_t tiles, float spacing, int slab, int32_t storage)
 {
   const int64_t waves = tiles * (kThreads / 64), room = 32ll * device_cus();
-  if (waves * 4 <= room) return spacing < 1.75f ? 4 : 1;
+  if (waves * 4 <= room) {
+    if (storage != XRH_F32) return spacing < 1.75f ? 4 : (waves * 16 <= room ? 2 : 1);
+    return (spacing < 0.95f || (spacing < 1.65f && waves * 8 <= room)) ? 4 : 2;
+  }
   if (slab == 0 && spacing > 0.0f && spacing < 0.75f && waves <= room) return 2;
   return (waves * 2 <= room && spacing < 0.95f) ? 2 : 1;
 }
@@ -1181,7 +1188,7 @@ int64_t drr_launch_plan(const DrrLaunch& L)
 {
   const int64_t tiles = L.max_band_tiles * L.bands;
   const int slab = drr_slab_lds(L.ray_spacing, L.geom, L.vol_bytes, L.storage, tiles);
-  return (int64_t)slab * 8 + drr_parts(tiles, L.ray_spacing, slab);
+  return (int64_t)slab * 8 + drr_parts(tiles, L.ray_spacing, slab, L.storage);
 }
 
 namespace {
@@ -1225,8 +1232,8 @@ void launch_fmt(const DrrLaunch& L, dim3 grid, hipStream_t s, int accumulate, fl
   // (forced whole rays go by slabs whatever the sizes)
   const int slab = (reuse_env && reuse > 0) ? slab_lds(L.ray_spacing)
                                             : drr_slab_lds(L.ray_spacing, L.geom, L.vol_bytes, L.storage, tiles);
-  const int parts = (reuse > 0) ? 1 : (reuse == 0) ? std::max(drr_parts(tiles, 0.0f, 0), 2)
-                                                   : drr_parts(tiles, L.ray_spacing, slab);
+  const int parts = (reuse > 0) ? 1 : (reuse == 0) ? std::max(drr_parts(tiles, 0.0f, 0, L.storage), 2)
+                                                   : drr_parts(tiles, L.ray_spacing, slab, L.storage);
   if (parts == 1 && slab > 0 && (fmt == 11 || fmt == 3 || fmt == 5)) {
     if (fmt == 11) XRH_LAUNCH_PARTS(11, 0);
     else if (fmt == 3) XRH_LAUNCH_PARTS(3, 0);
@@ -1285,7 +1292,7 @@ int drr_slab_lds(float spacing, int32_t geom, uint64_t bytes, int32_t storage, i
   return slab_lds(spacing);
 }
 
-bool drr_default_reuse(int64_t workgroups) { return drr_parts(workgroups, 0.0f, 0) == 1; }
+bool drr_default_reuse(int64_t workgroups) { return drr_parts(workgroups, 0.0f, 0, XRH_F32) == 1; }
 
 std::string drr_tune_key(int32_t storage, int32_t layout, int32_t geom, int32_t kernel, int32_t max_rows,
                          int32_t max_cols, int64_t workgroups)
