@@ -895,7 +895,7 @@ __device__ __forceinline__ float cast_ray_slab(const DrrItem& it, const TileRef&
     const Box b = box_of(a, n, false);
     __syncthreads();  // the previous slab has been read
     stage_box(src, b, it.raw_py, it.raw_pz, lds);
-    asm volatile("s_waitcnt vmcnt(0)");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the clobber: no read of the box above the wait)
     __syncthreads();
     // samples of the slab: q below its far face, as one comparison
     const float face = up ? (float)(a + n) - kOff : -((float)a - kOff);

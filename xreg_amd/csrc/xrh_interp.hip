@@ -423,7 +423,7 @@ __device__ __forceinline__ float cast_taps(const GridView& g, const Ray& ray, bo
                                                      16, (int)(lane_off + at * (uint32_t)sizeof(E)), 0, 0, 0);
           }
         }
-      asm volatile("s_waitcnt vmcnt(0)");
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the clobber: no read of the box above the wait)
       __syncthreads();
     }
     const int org = lo[0] + sy * lo[1] + sz * lo[2] - (1 + sy + sz);
