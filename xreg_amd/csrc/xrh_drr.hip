@@ -763,52 +763,103 @@ __device__ inline LdsPair lds_pair(int addr)
   return {p[0], p[1]};
 }
 
+// Margin of the boxes around the corner rays (voxels). A sample lies off its exact line by the rounding
+// of its start, step and position: in all at most some 5e-7 of the volume's largest edge across the main
+// axis, with what its offset along that axis moves the line there (slopes up to 2) and the lines' own
+// rounding to float, kept at 1e-6. FP32 set-up carries the detector point through 13 rounded operations
+// and the start of the samples through three more, 6e-8 of the largest intermediate (tile_corner's size) each:
+// 1e-6 of it per axis, 3e-6 with the offset along the main axis.
+constexpr float kSlabMargin = 0.05f, kSlabMarginEdge = 1.0e-6f, kSlabMarginSetup = 3.0e-6f;
+
+// Source and detector point of the pixel (col, row) in the index frame, in double and from the parameters
+// that the rays' set-up uses. `size` (FP32 set-up): with the absolute value of every product and term, so
+// the points' sum bounds what the set-up's operations meet.
+template <int kGeom>
+__device__ __forceinline__ void tile_corner(const DrrItem& it, double col, double row, bool size, double ph[3],
+                                            double dp[3])
+{
+  if constexpr (kGeom == XRH_GEOM_FP64) {
+    double det[3];
+    ind_to_det_d(it.cam, col, row, det);
+    affine_pt_d(it.Md, it.cam.pinhole_d, ph);
+    affine_pt_d(it.Md, det, dp);
+  } else {
+    auto term = [&](float a, double b) {
+      const double t = (double)a * b;
+      return size ? fabs(t) : t;
+    };
+    auto rowd = [&](const float* m, const double (&p)[3]) { return (term(m[0], p[0]) + term(m[1], p[1])) + term(m[2], p[2]); };
+    const double q[3] = {(double)it.cam.det_z * col, (double)it.cam.det_z * row, (double)it.cam.det_z};
+    const double r[3] = {rowd(&it.cam.kinv[0], q), rowd(&it.cam.kinv[3], q), rowd(&it.cam.kinv[6], q) + term(it.cam.z_adj, 1.0)};
+    double det[3], pin[3];
+    for (int k = 0; k < 3; ++k) {
+      det[k] = rowd(&it.cam.einv[4 * k], r) + term(it.cam.einv[4 * k + 3], 1.0);
+      pin[k] = term(it.cam.pinhole[k], 1.0);
+    }
+    for (int k = 0; k < 3; ++k) {
+      const double t = term(it.M[4 * k + 3], 1.0);
+      ph[k] = rowd(&it.M[4 * k], pin) + t;
+      dp[k] = rowd(&it.M[4 * k], det) + t;
+    }
+  }
+}
+
 // cast_ray by slabs. Every thread of the block calls it (it synchronises); `lds` holds `budget`
 // floats.
 template <int kGeom, int kOp, int kFmt>
 __device__ __forceinline__ float cast_ray_slab(const DrrItem& it, const TileRef& tr, int col, int row, bool inside,
                                       float* lds, int budget)
 {
-  __shared__ float corner[4][3];
-  __shared__ float origin[3];
+  __shared__ double corner[4][3];
+  __shared__ double origin[3];
   __shared__ float reach[3][4];
+  __shared__ float setup_size;
 
   int first, last;
   const Ray ray = begin_ray<kGeom, kOp>(it, col, row, inside, first, last);
   const int tid = threadIdx.x, lane = tid & 63;
-  if (tid < 4) {
+  if (tid < (kGeom == XRH_GEOM_FP32 ? 8 : 4)) {
     // the lines through the tile's corner pixels, padded index frame
-    double det[3], ph[3], dp[3];
-    ind_to_det_d(it.cam, (double)(tr.tx * kTile + (tid & 1) * (kTile - 1)),
-                 (double)(tr.ty * kTile + (tid >> 1) * (kTile - 1)), det);
-    affine_pt_d(it.Md, it.cam.pinhole_d, ph);
-    affine_pt_d(it.Md, det, dp);
-    for (int k = 0; k < 3; ++k) {
-      corner[tid][k] = (float)(dp[k] - ph[k]);
-      if (tid == 0) origin[k] = (float)(ph[k] + 1.0);
+    const bool size = tid >= 4;
+    double ph[3], dp[3];
+    tile_corner<kGeom>(it, (double)(tr.tx * kTile + (tid & 1) * (kTile - 1)),
+                       (double)(tr.ty * kTile + ((tid >> 1) & 1) * (kTile - 1)), size, ph, dp);
+    if (!size) {
+      for (int k = 0; k < 3; ++k) {
+        corner[tid][k] = dp[k] - ph[k];
+        if (tid == 0) origin[k] = ph[k] + 1.0;
+      }
+    } else if (tid == 7) {  // (the largest column and row)
+      setup_size = (float)fmax(fmax(ph[0] + dp[0], ph[1] + dp[1]), ph[2] + dp[2]);
     }
   }
   __syncthreads();
   // main axis of the tile: the largest component of its middle direction
-  const float mx = corner[0][0] + corner[3][0], my = corner[0][1] + corner[3][1], mz = corner[0][2] + corner[3][2];
+  const float mx = (float)(corner[0][0] + corner[3][0]), my = (float)(corner[0][1] + corner[3][1]),
+              mz = (float)(corner[0][2] + corner[3][2]);
   const int A = uni((fabsf(mx) >= fabsf(my) && fabsf(mx) >= fabsf(mz)) ? 0 : (fabsf(my) >= fabsf(mz) ? 1 : 2));
   const int B = A == 0 ? 1 : 0, C = A == 2 ? 1 : 2;
   const bool up = uni(pick(A, mx, my, mz) > 0.0f ? 1 : 0) != 0;
   bool ok = it.raw != nullptr;
   for (int k = 0; k < 4; ++k) {
-    const float d = up ? corner[k][A] : -corner[k][A];
-    ok = ok && d > 0.0f && 2.0f * d >= fabsf(corner[k][B]) && 2.0f * d >= fabsf(corner[k][C]);
+    const double d = up ? corner[k][A] : -corner[k][A];
+    ok = ok && d > 0.0 && 2.0 * d >= fabs(corner[k][B]) && 2.0 * d >= fabs(corner[k][C]);
   }
-  // this lane's line of the hull: corner lane & 3, axis B or C, as position = u + v * (position on A)
+  // this lane's line of the hull: corner lane & 3, axis B or C, as position = u + v * (position on A).
+  // (u in double: a source far from the volume is a large number, of which little remains)
   const int hk = lane & 3, hax = (lane & 8) ? C : B;
-  const float hv = corner[hk][hax] / corner[hk][A], hu = origin[hax] - origin[A] * hv;
+  const double hvd = corner[hk][hax] / corner[hk][A];
+  const float hv = (float)hvd, hu = (float)(origin[hax] - origin[A] * hvd);
   // the cells along A that the block's samples reach. The margin covers the rounding of the lines
-  // and the samples; under FP32 set-up also the samples' drift, at most one rounding per addition.
+  // and the samples, which grows with their coordinates; under FP32 set-up also that of the set-up
+  // itself and the samples' drift, at most one rounding per addition.
   constexpr float kOff = (kGeom == XRH_GEOM_FP64) ? 0.0f : 1.0f;
   const float sA = pick(A, ray.sx, ray.sy, ray.sz), dA = pick(A, ray.dx, ray.dy, ray.dz);
-  float lo = 3.0e38f, hi = -3.0e38f, margin = 0.05f;
+  const float edge = (float)max(max(it.X, it.Y), it.Z);
+  float lo = 3.0e38f, hi = -3.0e38f, margin = kSlabMargin + kSlabMarginEdge * edge;
+  if (kGeom == XRH_GEOM_FP32) margin = fmaf(kSlabMarginSetup, setup_size, margin);
   if (first <= last) {
-    if (kGeom == XRH_GEOM_FP32) margin = fmaf((float)last * (float)max(max(it.X, it.Y), it.Z), 6.0e-8f, margin);
+    if (kGeom == XRH_GEOM_FP32) margin = fmaf((float)last * edge, 6.0e-8f, margin);
     const float p0 = fmaf((float)first, dA, sA) + kOff, p1 = fmaf((float)last, dA, sA) + kOff;
     lo = fminf(p0, p1);
     hi = fmaxf(p0, p1);
@@ -1176,10 +1227,11 @@ int drr_parts(int64_t tiles, float spacing, int slab, int32_t storage)
   return (waves * 2 <= room && spacing < 0.95f) ? 2 : 1;
 }
 
-// LDS bytes of a workgroup's boxes for rays `spacing` voxels apart.
+// LDS bytes of a workgroup's boxes for rays `spacing` voxels apart: eight, four or three workgroups per CU,
+// with the 272 bytes that the kernel holds beside them.
 int slab_lds(float spacing)
 {
-  return !(spacing > 0.0f) ? 0 : (spacing < 0.95f ? 20224 : (spacing < 2.7f ? 40704 : 54272));
+  return !(spacing > 0.0f) ? 0 : (spacing < 0.95f ? 20160 : (spacing < 2.7f ? 40640 : 54208));
 }
 
 }  // namespace
