@@ -417,10 +417,10 @@ __device__ inline float cell_value(const float (&a)[4], const float (&b)[4], flo
     const float p1 = fmaf(wy, fmaf(wx, b[3], b[2]), fmaf(wx, b[1], b[0]));
     return fmaf(wz, p1, p0);
   } else {
-    // the faces at x and x + 1: bilinear in y, z, then linear along x
-    const float p0 = fmaf(wz, fmaf(wy, a[3], a[2]), fmaf(wy, a[1], a[0]));
-    const float p1 = fmaf(wz, fmaf(wy, b[3], b[2]), fmaf(wy, b[1], b[0]));
-    return lerp(p0, p1, wx);
+    // the faces at x and x + 1: their edges along y, between those along z, then along x
+    const float a0 = fmaf(wy, a[1], a[0]), a1 = fmaf(wy, a[3], a[2]);
+    const float b0 = fmaf(wy, b[1], b[0]), b1 = fmaf(wy, b[3], b[2]);
+    return lerp(fmaf(wz, a1 - a0, a0), fmaf(wz, b1 - b0, b0), wx);
   }
 }
 
@@ -681,7 +681,7 @@ __device__ __forceinline__ float cast_ray(const DrrItem& it, int col, int row, b
 //
 // The box comes from the tile's corner rays: the pixel -> position map on a plane across the main
 // axis is projective, so the corners' positions on the slab's two planes bound every ray between
-// them. Slabs end on cell faces, so no cell straddles two. A cell's face coefficients are formed
+// them. Slabs end on cell faces, so no cell straddles two. A cell's faces are formed
 // from its voxels by the float operations that built the face layout (16-bit storage: the gathering
 // march's lerps, from voxels kept as floats), and samples segment as there: the values are the
 // gathering march's bit for bit, and tiles whose box
@@ -986,10 +986,10 @@ __device__ __forceinline__ float cast_ray_slab(const DrrItem& it, const TileRef&
           vb[0] = r00.b;
           va[1] = r10.a - r00.a;
           vb[1] = r10.b - r00.b;
-          va[2] = r01.a - r00.a;
-          vb[2] = r01.b - r00.b;
-          va[3] = (r11.a - r01.a) - va[1];
-          vb[3] = (r11.b - r01.b) - vb[1];
+          va[2] = r01.a;
+          vb[2] = r01.b;
+          va[3] = r11.a - r01.a;
+          vb[3] = r11.b - r01.b;
         } else {
           va[0] = r00.b - r00.a;
           va[1] = r10.b - r10.a;

@@ -206,13 +206,13 @@ __device__ inline uint16_t f2bf_bits(float v)
   return (uint16_t)(r >> 16);
 }
 
-// A face's coefficients from its corners, by the float differences that the slab march takes from
-// the voxels themselves.
+// A face's element: its two edges along y (at z and z + 1), each as a corner and the difference to the
+// other, a float difference and so the exact one rounded once. The slab march forms the same from the
+// voxels themselves. (With the four coefficients c0 + c1 v + c2 w + c3 v w instead, c3 would be a difference
+// of rounded differences wherever it is not formed in double.)
 __device__ inline float4 face(float v00, float v10, float v01, float v11)
 {
-#pragma clang fp contract(off)
-  const float c1 = v10 - v00;
-  return make_float4(v00, c1, v01 - v00, (v11 - v01) - c1);
+  return make_float4(v00, v10 - v00, v01, v11 - v01);
 }
 
 // Builds the padded layout from the raw x-fastest volume. One thread per padded voxel. kLayoutPlain:
@@ -252,8 +252,7 @@ __global__ void build_layout_kernel(const float* __restrict__ src, int X, int Y,
     q.w = V(a + 1, b + 1, c);
     ((float4*)dst)[i] = q;
   } else if (layout == kLayoutFace) {
-    // face normal to x at (a, b, c): corners (b, c), (b+1, c), (b, c+1), (b+1, c+1) over y, z;
-    // bilinear coefficients f(v, w) = c0 + c1 v + c2 w + c3 v w
+    // face normal to x at (a, b, c): corners (b, c), (b+1, c), (b, c+1), (b+1, c+1) over y, z
     ((float4*)dst)[i] = face(V(a, b, c), V(a, b + 1, c), V(a, b, c + 1), V(a, b + 1, c + 1));
   } else if (layout == kLayoutBrick) {
     // the face of (a, b, c) as in kLayoutFace, written to its brick and, when it is the first
@@ -389,7 +388,7 @@ static int default_layout(int storage)
   if (env && std::strcmp(env, "quad") == 0 && storage == XRH_F32) return kLayoutQuad;
   if (env && std::strcmp(env, "coef") == 0 && storage == XRH_F32) return kLayoutCoef;
   if (env && std::strcmp(env, "brick") == 0 && storage == XRH_F32) return kLayoutBrick;
-  // FP32: x-face bilinear coefficients; 16-bit: all corners in one 16-byte element
+  // FP32: the edges of the x-faces; 16-bit: all corners in one 16-byte element
   return (storage == XRH_F32) ? kLayoutFace : kLayoutOct;
 }
 
