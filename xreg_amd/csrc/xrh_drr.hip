@@ -435,11 +435,15 @@ __device__ inline float cell_value(const float (&a)[4], const float (&b)[4], flo
 // first's plus the step (FP64 set-up), which also saves its index arithmetic; under FP32 set-up
 // they are taken from the reference's own position, whose cell is exact. As unsigned integers
 // the three coordinates' largest is below that of 1.0f exactly when all lie in [0, 1).
+// The lanes of a wave wait for each other at the ends of windows, of which the first is that of sample
+// `from` (at most i): at nearly the same depth they fetch the same cells. Which samples form a pair
+// follows from the ray's own first sample alone.
 template <int kGeom, int kOp, int kFmt>
-__device__ __forceinline__ float march_cells(const Ray& ray, const VolView& vv, Pos& pos, int i, int last, int seg)
+__device__ __forceinline__ float march_cells(const Ray& ray, const VolView& vv, Pos& pos, int i, int last, int seg,
+                                             int from)
 {
   float tot = line_init<kOp>(), acc = line_init<kOp>();
-  int seg_last = (seg_of(i, seg) + 1) * seg - 1, win_last = i | (kWindow - 1);
+  int seg_last = (seg_of(i, seg) + 1) * seg - 1, win_last = from | (kWindow - 1);
   float f = (float)i;  // sample indices as floats (exact: n < 2^23)
   for (;;) {
     const float fstop = (float)min(win_last, last), fpair = (float)min(seg_last, last);
@@ -536,13 +540,13 @@ __device__ __forceinline__ float march_samples(const Ray& ray, const VolView& vv
   return acc;
 }
 
-// Samples [i, last] (i <= last) of one ray, summed segment by segment. `pos`: sample i's position
-// under FP32 set-up; it ends past sample `last`.
+// Samples [i, last] (i <= last) of one ray, summed segment by segment; the wave's lanes have their first
+// samples from `from` on. `pos`: sample i's position under FP32 set-up; it ends past sample `last`.
 template <int kGeom, int kOp, int kFmt>
-__device__ __forceinline__ float march(const Ray& ray, const VolView& vv, Pos& pos, int i, int last, int seg)
+__device__ __forceinline__ float march(const Ray& ray, const VolView& vv, Pos& pos, int i, int last, int seg, int from)
 {
   if constexpr (is_cell_fmt(kFmt)) {
-    return march_cells<kGeom, kOp, kFmt>(ray, vv, pos, i, last, seg);
+    return march_cells<kGeom, kOp, kFmt>(ray, vv, pos, i, last, seg, from);
   } else {
     float tot = line_init<kOp>();
     for (int end = (seg_of(i, seg) + 1) * seg - 1; i <= last; end += seg) {
@@ -621,11 +625,11 @@ __device__ inline VolView vol_view(const DrrItem& it)
 // One ray of one item: the line integral (SUM) or maximum (MAX) of its samples times the step,
 // or the kernel's initial value when the ray misses the volume. Called by every lane of the
 // wave (`inside` false for lanes past the detector edge), so that the lanes can agree on a
-// start: with an empty-space map each lane marches from the wave's earliest first sample
-// instead of its own. The samples before a lane's own first lie in empty bricks and are exactly
-// 0, so its sum is unchanged bit for bit, and neighbouring rays, which enter the volume at
+// start, the wave's earliest first sample: neighbouring rays, which enter the volume at
 // nearly the same depth, then fetch the same cells in the same iteration (C2: L1 tag accesses
-// -7.5%, L1 tag-conflict stalls -40%, DRR -2%).
+// -7.5%, L1 tag-conflict stalls -40%, DRR -2%). By cells a lane waits for its own first sample;
+// sample by sample it marches from the common one, over samples that lie in empty bricks and are
+// exactly 0. Either way its sum is the same as from its own first sample, bit for bit.
 template <int kGeom, int kOp, int kFmt>
 __device__ __forceinline__ float cast_range(const DrrItem& it, const Ray& ray, int i, int last)
 {
@@ -636,9 +640,11 @@ __device__ __forceinline__ float cast_range(const DrrItem& it, const Ray& ray, i
   for (int off = 32; off >= 1; off >>= 1) start = min(start, __shfl_xor(start, off, 64));
   if (ray.n >= 0) {
     if (i <= last) {
+      // sample by sample the lanes start together, on samples that are zero
+      if constexpr (!is_cell_fmt(kFmt)) i = start;
       Pos pos{ray.sx, ray.sy, ray.sz};
-      if constexpr (kGeom == XRH_GEOM_FP32) pos.advance(ray, start);
-      acc = march<kGeom, kOp, kFmt>(ray, vol_view(it), pos, start, last, seg_len(ray.n));
+      if constexpr (kGeom == XRH_GEOM_FP32) pos.advance(ray, i);
+      acc = march<kGeom, kOp, kFmt>(ray, vol_view(it), pos, i, last, seg_len(ray.n), start);
     }
     acc = acc * it.step;
   }
@@ -1078,7 +1084,7 @@ __device__ __forceinline__ float cast_ray_split(const DrrItem& it, int col, int 
     float acc = line_init<kOp>();
     if (i <= stop) {
       if constexpr (kGeom == XRH_GEOM_FP32) pos.advance(ray, i - at);
-      acc = march<kGeom, kOp, kFmt>(ray, vol_view(it), pos, i, stop, seg);
+      acc = march<kGeom, kOp, kFmt>(ray, vol_view(it), pos, i, stop, seg, i);
       at = stop + 1;
     }
     sums[k][px] = acc;
