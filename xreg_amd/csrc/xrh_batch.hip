@@ -70,7 +70,7 @@ struct xrh_batch {
   bool variant_set = false;
   DrrVariant variant;
   DrrVariant last_variant;         // the variant of the last staged launch
-  int64_t last_plan = 0;           // and its default way of marching
+  int64_t last_plan = 0;           // and its way of marching
 };
 
 namespace {
@@ -313,6 +313,7 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
   int64_t off = 0;
   double spacing = 0.0;
   uint64_t vol_bytes = 0;
+  bool plain = true;
   groups.clear();
   for (int64_t i = 0; i < n; ++i) {
     const int32_t v = item_view[i * objs];
@@ -332,6 +333,7 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
       p.pad_ = 0;
       spacing += ray_spacing(b->views[vk].vol, b->views[vk].cam, p.pose);
       vol_bytes = std::max<uint64_t>(vol_bytes, b->views[vk].vol->bytes);
+      plain = plain && b->views[vk].vol->raw;
     }
     rows[i] = w.cam.num_det_rows;
     cols[i] = w.cam.num_det_cols;
@@ -399,10 +401,11 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
   D.ncc_tiles_per_item = b->max_img_tiles;
   D.ray_spacing = (float)(spacing / (double)(n * objs));
   D.vol_bytes = vol_bytes;
-  b->last_plan = drr_launch_plan(D);
+  D.plain = plain;
   D.reuse = var.reuse;
   D.wave_shape = var.shape;
   D.objs = objs;
+  b->last_plan = drr_launch_plan(D);
   return D;
 }
 

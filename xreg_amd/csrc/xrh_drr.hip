@@ -435,15 +435,15 @@ __device__ inline float cell_value(const float (&a)[4], const float (&b)[4], flo
 // first's plus the step (FP64 set-up), which also saves its index arithmetic; under FP32 set-up
 // they are taken from the reference's own position, whose cell is exact. As unsigned integers
 // the three coordinates' largest is below that of 1.0f exactly when all lie in [0, 1).
-// The lanes of a wave wait for each other at the ends of windows, of which the first is that of sample
-// `from` (at most i): at nearly the same depth they fetch the same cells. Which samples form a pair
+// The lanes of a wave wait for each other at the ends of windows of `window` samples, of which the first is
+// that of sample `from` (at most i): at nearly the same depth they fetch the same cells. Which samples form a pair
 // follows from the ray's own first sample alone.
 template <int kGeom, int kOp, int kFmt>
 __device__ __forceinline__ float march_cells(const Ray& ray, const VolView& vv, Pos& pos, int i, int last, int seg,
-                                             int from)
+                                             int from, int window)
 {
   float tot = line_init<kOp>(), acc = line_init<kOp>();
-  int seg_last = (seg_of(i, seg) + 1) * seg - 1, win_last = from | (kWindow - 1);
+  int seg_last = (seg_of(i, seg) + 1) * seg - 1, win_last = from | (window - 1);
   float f = (float)i;  // sample indices as floats (exact: n < 2^23)
   for (;;) {
     const float fstop = (float)min(win_last, last), fpair = (float)min(seg_last, last);
@@ -496,7 +496,7 @@ __device__ __forceinline__ float march_cells(const Ray& ray, const VolView& vv, 
       seg_last += seg;
     }
     if (done) break;
-    win_last += kWindow;
+    win_last += window;
   }
   return tot;
 }
@@ -543,10 +543,11 @@ __device__ __forceinline__ float march_samples(const Ray& ray, const VolView& vv
 // Samples [i, last] (i <= last) of one ray, summed segment by segment; the wave's lanes have their first
 // samples from `from` on. `pos`: sample i's position under FP32 set-up; it ends past sample `last`.
 template <int kGeom, int kOp, int kFmt>
-__device__ __forceinline__ float march(const Ray& ray, const VolView& vv, Pos& pos, int i, int last, int seg, int from)
+__device__ __forceinline__ float march(const Ray& ray, const VolView& vv, Pos& pos, int i, int last, int seg, int from,
+                                       int window)
 {
   if constexpr (is_cell_fmt(kFmt)) {
-    return march_cells<kGeom, kOp, kFmt>(ray, vv, pos, i, last, seg, from);
+    return march_cells<kGeom, kOp, kFmt>(ray, vv, pos, i, last, seg, from, window);
   } else {
     float tot = line_init<kOp>();
     for (int end = (seg_of(i, seg) + 1) * seg - 1; i <= last; end += seg) {
@@ -631,7 +632,7 @@ __device__ inline VolView vol_view(const DrrItem& it)
 // sample by sample it marches from the common one, over samples that lie in empty bricks and are
 // exactly 0. Either way its sum is the same as from its own first sample, bit for bit.
 template <int kGeom, int kOp, int kFmt>
-__device__ __forceinline__ float cast_range(const DrrItem& it, const Ray& ray, int i, int last)
+__device__ __forceinline__ float cast_range(const DrrItem& it, const Ray& ray, int i, int last, int window)
 {
   float acc = line_init<kOp>();
   // wave minimum of the first samples of the lanes with samples (all lanes take part)
@@ -644,7 +645,7 @@ __device__ __forceinline__ float cast_range(const DrrItem& it, const Ray& ray, i
       if constexpr (!is_cell_fmt(kFmt)) i = start;
       Pos pos{ray.sx, ray.sy, ray.sz};
       if constexpr (kGeom == XRH_GEOM_FP32) pos.advance(ray, i);
-      acc = march<kGeom, kOp, kFmt>(ray, vol_view(it), pos, i, last, seg_len(ray.n), start);
+      acc = march<kGeom, kOp, kFmt>(ray, vol_view(it), pos, i, last, seg_len(ray.n), start, window);
     }
     acc = acc * it.step;
   }
@@ -667,11 +668,11 @@ __device__ __forceinline__ Ray begin_ray(const DrrItem& it, int col, int row, bo
 }
 
 template <int kGeom, int kOp, int kFmt>
-__device__ __forceinline__ float cast_ray(const DrrItem& it, int col, int row, bool inside)
+__device__ __forceinline__ float cast_ray(const DrrItem& it, int col, int row, bool inside, int window)
 {
   int first, last;
   const Ray ray = begin_ray<kGeom, kOp>(it, col, row, inside, first, last);
-  return cast_range<kGeom, kOp, kFmt>(it, ray, first, last);
+  return cast_range<kGeom, kOp, kFmt>(it, ray, first, last, window);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -814,7 +815,7 @@ __device__ __forceinline__ void tile_corner(const DrrItem& it, double col, doubl
 // floats.
 template <int kGeom, int kOp, int kFmt>
 __device__ __forceinline__ float cast_ray_slab(const DrrItem& it, const TileRef& tr, int col, int row, bool inside,
-                                      float* lds, int budget)
+                                      float* lds, int budget, int window)
 {
   __shared__ double corner[4][3];
   __shared__ double origin[3];
@@ -928,7 +929,7 @@ __device__ __forceinline__ float cast_ray_slab(const DrrItem& it, const TileRef&
       if (b0.wx <= 256 && b1.wx <= 256 && b0.floats() <= budget && b1.floats() <= budget) break;
     }
   }
-  if (depth < 2) return cast_range<kGeom, kOp, kFmt>(it, ray, first, last);
+  if (depth < 2) return cast_range<kGeom, kOp, kFmt>(it, ray, first, last, window);
 
   const auto src = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(it.raw), (short)0, (int)it.raw_bytes, 0x00020000);
   const float flast = (float)last, fseg_len = (float)seg_len(ray.n);
@@ -1084,7 +1085,7 @@ __device__ __forceinline__ float cast_ray_split(const DrrItem& it, int col, int 
     float acc = line_init<kOp>();
     if (i <= stop) {
       if constexpr (kGeom == XRH_GEOM_FP32) pos.advance(ray, i - at);
-      acc = march<kGeom, kOp, kFmt>(ray, vol_view(it), pos, i, stop, seg, i);
+      acc = march<kGeom, kOp, kFmt>(ray, vol_view(it), pos, i, stop, seg, i, kWindow);
       at = stop + 1;
     }
     sums[k][px] = acc;
@@ -1100,14 +1101,16 @@ __device__ __forceinline__ float cast_ray_split(const DrrItem& it, int col, int 
   return acc;
 }
 
-// kParts: the waves that share a ray, 0 for slab marching with `budget` floats of dynamic LDS.
+// kParts: the waves that share a ray, 0 for slab marching with `budget` floats of dynamic LDS. Whole rays that
+// gather by cells wait for each other every `window` samples.
 template <int kGeom, int kOp, int kFmt, int kParts>
-__device__ __forceinline__ float cast_pixel(const DrrItem& it, const TileRef& tr, int col, int row, bool inside, int budget)
+__device__ __forceinline__ float cast_pixel(const DrrItem& it, const TileRef& tr, int col, int row, bool inside,
+                                            int budget, int window)
 {
   if constexpr (kParts == 0) {
     extern __shared__ __attribute__((aligned(16))) float box_lds[];
-    return cast_ray_slab<kGeom, kOp, kFmt>(it, tr, col, row, inside, box_lds, budget);
-  } else if constexpr (kParts == 1) return cast_ray<kGeom, kOp, kFmt>(it, col, row, inside);
+    return cast_ray_slab<kGeom, kOp, kFmt>(it, tr, col, row, inside, box_lds, budget, window);
+  } else if constexpr (kParts == 1) return cast_ray<kGeom, kOp, kFmt>(it, col, row, inside, window);
   else return cast_ray_split<kGeom, kOp, kFmt, kParts>(it, col, row, inside);
 }
 
@@ -1115,7 +1118,7 @@ template <int kGeom, int kOp, int kFmt, int kParts>
 __global__ __launch_bounds__(kThreads * (kParts > 1 ? kParts : 1), kParts == 0 ? 4 : 8) void drr_kernel(
     const DrrItem* __restrict__ items, const uint32_t* __restrict__ band_start, int64_t num_items,
     int bands, float* __restrict__ out, int accumulate, float fill,
-    double* __restrict__ ncc_partials, int ncc_tiles, int shape, int budget)
+    double* __restrict__ ncc_partials, int ncc_tiles, int shape, int budget, int window)
 {
   const TileRef tr = decode_tile(band_start, num_items, bands, items);
   if (!tr.valid) return;
@@ -1123,7 +1126,7 @@ __global__ __launch_bounds__(kThreads * (kParts > 1 ? kParts : 1), kParts == 0 ?
   int col, row;
   lane_pixel(tr.tx, tr.ty, shape, col, row);
   const bool inside = (col < it.cam.cols) && (row < it.cam.rows);
-  const float acc = cast_pixel<kGeom, kOp, kFmt, kParts>(it, tr, col, row, inside, budget);
+  const float acc = cast_pixel<kGeom, kOp, kFmt, kParts>(it, tr, col, row, inside, budget, window);
   // the first part stores the pixels
   const bool mine = inside && (kParts <= 1 || threadIdx.x < kThreads);
   store_pixel<kOp>(it, tr, mine, col, row, acc, out, accumulate, fill, ncc_partials, ncc_tiles);
@@ -1139,7 +1142,7 @@ template <int kGeom, int kOp, int kFmt, int kParts>
 __global__ __launch_bounds__(kThreads * (kParts > 1 ? kParts : 1), kParts == 0 ? 4 : 8) void drr_objects_kernel(
     const DrrItem* __restrict__ items, const uint32_t* __restrict__ band_start, int64_t num_items,
     int bands, float* __restrict__ out, float fill, double* __restrict__ ncc_partials, int ncc_tiles,
-    int shape, int budget, int objs)
+    int shape, int budget, int window, int objs)
 {
   const TileRef tr = decode_tile(band_start, num_items, bands, items, objs);
   if (!tr.valid) return;
@@ -1151,7 +1154,8 @@ __global__ __launch_bounds__(kThreads * (kParts > 1 ? kParts : 1), kParts == 0 ?
   float pix = 0.0f;
   if (inside) pix = it0.bg ? it0.bg[px] : fill;
   for (int k = 0; k < objs; ++k) {
-    const float aa = 0.0f + cast_pixel<kGeom, kOp, kFmt, kParts>(items[tr.item * objs + k], tr, col, row, inside, budget) * 1.0f;
+    const float aa =
+        0.0f + cast_pixel<kGeom, kOp, kFmt, kParts>(items[tr.item * objs + k], tr, col, row, inside, budget, window) * 1.0f;
     if (inside) {
       if constexpr (kOp == XRH_LINE_INT_SUM) pix = pix + aa; else pix = (pix < aa) ? aa : pix;
     }
@@ -1240,13 +1244,72 @@ int slab_lds(float spacing)
   return !(spacing > 0.0f) ? 0 : (spacing < 0.95f ? 20160 : (spacing < 2.7f ? 40640 : 54208));
 }
 
+// Samples between the points where the lanes of whole rays gathering by cells wait for each other. In
+// step, lanes touch the fewest cache lines; apart, every iteration keeps all lanes loading, at two samples
+// a load where the cells allow it. Close rays share lines over many samples, sparse rays none over more than
+// one. us with windows of 16, 8, 4 and 1 samples, by voxels between rays, over 215 MB / 1.7 GB of faces: 0.39
+// 554, 559, 609, 748 / 1441, 1504, 1661, 2041; 0.47 574, 570, 618, 743 / 1178, 1167, 1274, 1568; 0.58 671, 633,
+// 658, 770 / 1067, 984, 995, 1176; 0.67 794, 705, 692, 785 / 1221, 1075, 1042, 1188; 0.78 969, 873, 817, 814 /
+// 1466, 1316, 1210, 1249; 0.93 1203, 1117, 1054, 912 / 1983, 1816, 1670, 1461; with the LDS of gather_lds 1.16
+// 1268, 1221, 1250, 1422 and 1.55 1849, 1783, 1757, 1618. (26 MB: 0.39 313, 323, 355, 423; 0.78 448, 411, 411, 449;
+// 1.55 886, 834, 789, 708.) Bricks and coefficients spread a cell's neighbours over more lines and want the
+// lanes in step earlier (1.7 GB of faces: bricks 0.58 1287, 1217, 1202, 1316, 0.67 1467, 1417, 1362, 1369, 0.78 1978,
+// 1820, 1733, 1623; coefficients 0.58 1398, 1318, 1252, 1299, 0.67 1659, 1515, 1402, 1335).
+int gather_window(float spacing, int32_t layout)
+{
+  const bool face = layout == kLayoutFace;
+  if (!(spacing >= 0.45f)) return kWindow;
+  if (spacing < (face ? 0.63f : 0.55f)) return 8;
+  if (spacing < (face ? 0.85f : 0.63f)) return 4;
+  return (spacing >= 1.1f && spacing < 1.45f) ? 4 : 1;
+}
+
+// LDS bytes that a workgroup of whole gathered rays reserves, unused, over a volume that the caches do not
+// hold: from about a voxel between rays on, four workgroups on a CU leave each other's lines in its L1 and
+// take less time than eight, and from 2.7 voxels on three (us without / with 40 / 54 KB, 215 MB of faces, the
+// best window of each: 1.03 voxels 1100 / 1091 / - , 1.16 1330 / 1221 / 1737, 1.55 1941 / 1618 / 1926, 3.1 3888 /
+// 3340 / 3176; f16 cells 0.78 718 / 731 / 1260, 1.16 1355 / 1123 / 1381, 1.55 1963 / 1665 / 1648, 3.1 4387 / 3788 /
+// 3388).
+int gather_lds(float spacing) { return (spacing >= 1.1f) ? slab_lds(spacing) : 0; }
+
+// How a launch marches. Slabs need the plain voxels of every volume beside a face or oct layout.
+struct March {
+  int parts;   // waves that share a ray
+  bool slabs;  // whole rays by slabs
+  int lds;     // dynamic LDS bytes: the boxes of the slabs, or held unused by whole rays that gather
+  int window;  // samples between the points where the lanes of whole rays wait
+};
+
+March drr_march(const DrrLaunch& L, int64_t tiles)
+{
+  // XRH_CELL_REUSE=0 / =1 force shared rays / whole rays, by slabs whatever the sizes (read per launch, so
+  // a process can switch between calls); otherwise a tuned variant decides, else the launch
+  const char* env = std::getenv("XRH_CELL_REUSE");
+  const int reuse = env ? (std::strcmp(env, "0") != 0 ? 1 : 0) : L.reuse;
+  const bool able = L.plain && (L.storage == XRH_F32 ? L.layout == kLayoutFace : L.layout == kLayoutOct);
+  const int slab = !able ? 0
+                   : (env && reuse > 0) ? slab_lds(L.ray_spacing)
+                                        : drr_slab_lds(L.ray_spacing, L.geom, L.vol_bytes, L.storage, tiles);
+  March m;
+  m.parts = (reuse > 0) ? 1 : (reuse == 0) ? std::max(drr_parts(tiles, 0.0f, 0, L.storage), 2)
+                                           : drr_parts(tiles, L.ray_spacing, slab, L.storage);
+  m.slabs = m.parts == 1 && slab > 0;
+  m.lds = m.slabs ? slab : 0;
+  m.window = gather_window(L.ray_spacing, L.layout);
+  // (launches that could go by slabs and do not are better off without)
+  if (!able && m.parts == 1 && L.vol_bytes >= kSlabBytes &&
+      (L.storage == XRH_F32 ? L.layout != kLayoutQuad && L.layout != kLayoutLinear : L.layout == kLayoutOct)) {
+    m.lds = gather_lds(L.ray_spacing);
+  }
+  return m;
+}
+
 }  // namespace
 
 int64_t drr_launch_plan(const DrrLaunch& L)
 {
-  const int64_t tiles = L.max_band_tiles * L.bands;
-  const int slab = drr_slab_lds(L.ray_spacing, L.geom, L.vol_bytes, L.storage, tiles);
-  return (int64_t)slab * 8 + drr_parts(tiles, L.ray_spacing, slab, L.storage);
+  const March m = drr_march(L, L.max_band_tiles * L.bands);
+  return ((int64_t)m.lds * 64 + m.window) * 16 + m.parts * 2 + (m.slabs ? 1 : 0);
 }
 
 namespace {
@@ -1257,28 +1320,22 @@ void launch_fmt(const DrrLaunch& L, dim3 grid, hipStream_t s, int accumulate, fl
 #define XRH_LAUNCH_PARTS(F, P)                                                                        \
   do {                                                                                                \
     const dim3 threads(kThreads * (P > 1 ? P : 1));                                                   \
-    const int lds = (P == 0) ? slab : 0;                                                              \
     if (L.objs > 1) {                                                                                 \
-      hipLaunchKernelGGL((drr_objects_kernel<kGeom, kOp, F, P>), grid, threads, lds, s, L.items_dev,  \
+      hipLaunchKernelGGL((drr_objects_kernel<kGeom, kOp, F, P>), grid, threads, m.lds, s, L.items_dev,  \
                          L.band_start_dev, L.num_items, L.bands, L.out, fill, L.ncc_partials,         \
-                         L.ncc_tiles_per_item, shape, lds / 4, L.objs);                               \
+                         L.ncc_tiles_per_item, shape, m.lds / 4, m.window, L.objs);                   \
     } else {                                                                                          \
-      hipLaunchKernelGGL((drr_kernel<kGeom, kOp, F, P>), grid, threads, lds, s, L.items_dev,          \
+      hipLaunchKernelGGL((drr_kernel<kGeom, kOp, F, P>), grid, threads, m.lds, s, L.items_dev,          \
                          L.band_start_dev, L.num_items, L.bands, L.out, accumulate, fill,             \
-                         L.ncc_partials, L.ncc_tiles_per_item, shape, lds / 4);                       \
+                         L.ncc_partials, L.ncc_tiles_per_item, shape, m.lds / 4, m.window);            \
     }                                                                                                 \
   } while (0)
 #define XRH_LAUNCH_FMT(F)                         \
   do {                                            \
-    if (parts == 4) XRH_LAUNCH_PARTS(F, 4);       \
-    else if (parts == 2) XRH_LAUNCH_PARTS(F, 2);  \
+    if (m.parts == 4) XRH_LAUNCH_PARTS(F, 4);     \
+    else if (m.parts == 2) XRH_LAUNCH_PARTS(F, 2); \
     else XRH_LAUNCH_PARTS(F, 1);                  \
   } while (0)
-  // Waves per ray. XRH_CELL_REUSE=0 / =1 force shared rays / slabs (read per launch, so a process
-  // can switch between calls); otherwise a tuned variant decides, else the launch size.
-  const char* reuse_env = std::getenv("XRH_CELL_REUSE");
-  const int reuse = reuse_env ? (std::strcmp(reuse_env, "0") != 0 ? 1 : 0) : L.reuse;
-  const int64_t tiles = (int64_t)grid.x * grid.y;
   const int shape = (L.wave_shape >= 0 && L.wave_shape <= 2) ? L.wave_shape : 0;
   const int fmt = (L.storage == XRH_F32)
                       ? (L.layout == kLayoutCoef ? 7
@@ -1287,12 +1344,8 @@ void launch_fmt(const DrrLaunch& L, dim3 grid, hipStream_t s, int accumulate, fl
                                                                                 : (L.layout == kLayoutQuad ? 1 : 0))))
                 : (L.storage == XRH_F16) ? (L.layout == kLayoutOct ? 3 : 2)
                                          : (L.layout == kLayoutOct ? 5 : 4);
-  // (forced whole rays go by slabs whatever the sizes)
-  const int slab = (reuse_env && reuse > 0) ? slab_lds(L.ray_spacing)
-                                            : drr_slab_lds(L.ray_spacing, L.geom, L.vol_bytes, L.storage, tiles);
-  const int parts = (reuse > 0) ? 1 : (reuse == 0) ? std::max(drr_parts(tiles, 0.0f, 0, L.storage), 2)
-                                                   : drr_parts(tiles, L.ray_spacing, slab, L.storage);
-  if (parts == 1 && slab > 0 && (fmt == 11 || fmt == 3 || fmt == 5)) {
+  const March m = drr_march(L, (int64_t)grid.x * grid.y);
+  if (m.slabs) {
     if (fmt == 11) XRH_LAUNCH_PARTS(11, 0);
     else if (fmt == 3) XRH_LAUNCH_PARTS(3, 0);
     else XRH_LAUNCH_PARTS(5, 0);
@@ -1327,7 +1380,7 @@ void launch_fmt(const DrrLaunch& L, dim3 grid, hipStream_t s, int accumulate, fl
 // 0.828, at 1.16 0.787 / 0.625 / 0.940, at 1.55 1.30 / 1.05 / 1.29, at 2.3 2.22 / 1.91 / 2.28; 512 x
 // 512 x 400 voxels at 3.1 6.06 / 5.66 / 5.32.
 //
-// Volumes of under 64 MB gather at any distance (40 MB, 2016 tiles at 0.70 voxels: 179 / 211 us).
+// Volumes of under 64 MB (kSlabBytes) gather at any distance (40 MB, 2016 tiles at 0.70 voxels: 179 / 211 us).
 // With 16-bit storage a gathered sample is one load instead of an FP32 cell's two, so slabs pay later
 // (ns per ray by gathering / slabs, f16): 215 MB, FP64 set-up, at 0.19 voxels 0.315 / 0.316, 0.39 0.348 /
 // 0.360, 0.58 0.364 / 0.401, 0.78 0.495 / 0.440, 1.55 1.31 / 1.02; FP32 set-up 0.39 0.32 / 0.38, 0.78
@@ -1337,7 +1390,7 @@ void launch_fmt(const DrrLaunch& L, dim3 grid, hipStream_t s, int accumulate, fl
 // 2430 at 0.84 339 / 382; 556 MB, 2112 at 1.60 1019 / 937.
 int drr_slab_lds(float spacing, int32_t geom, uint64_t bytes, int32_t storage, int64_t tiles)
 {
-  if (!(spacing > 0.0f) || bytes < (64ull << 20)) return 0;
+  if (!(spacing > 0.0f) || bytes < kSlabBytes) return 0;
   const bool fp32 = geom == XRH_GEOM_FP32;
   if (storage == XRH_F32) {
     if (fp32 && spacing < 0.5f && bytes < (256ull << 20)) return 0;

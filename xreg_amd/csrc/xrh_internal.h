@@ -311,6 +311,7 @@ struct DrrLaunch {
   float ray_spacing;        // mean distance of neighbouring rays at the volumes' centres (voxels),
                             // 0 if not known: with vol_bytes, the largest volume's layout bytes,
   uint64_t vol_bytes;       // it chooses between slab marching and gathering
+  bool plain;               // every volume has its plain voxels (slabs need them)
   int32_t reuse;            // DrrVariant::reuse
   int32_t wave_shape;       // DrrVariant::shape
   int32_t objs;             // objects per item (0 or 1: one); items_dev / poses_dev then hold
@@ -320,9 +321,11 @@ struct DrrLaunch {
 };
 // Key of the tuned-variant table: storage, layout, geometry, line kernel, the largest
 // detector of the launch and its workgroups per CU (rounded down to a power of two).
-// The slab-marching choice of a launch (its dynamic LDS bytes, 0: gathering).
+// Layout bytes from which a volume is not held by the caches.
+constexpr uint64_t kSlabBytes = 64ull << 20;
+// The slab-marching choice of a launch over volumes with plain voxels (its dynamic LDS bytes, 0: gathering).
 int drr_slab_lds(float spacing, int32_t geom, uint64_t bytes, int32_t storage, int64_t tiles);
-// The default way a launch marches, as one number (captured launches are kept by it).
+// The way a launch marches, as one number (captured launches are kept by it).
 int64_t drr_launch_plan(const DrrLaunch& L);
 // Distance (voxels) of neighbouring rays at the volume's centre for a camera and a row-major
 // cam->phys pose.

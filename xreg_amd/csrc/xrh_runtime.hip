@@ -745,6 +745,7 @@ static void line_int_launch(xrh_ctx* ctx, const xrh_volume* vol, const xrh_camer
   for (int64_t p = 0; p < num_projs; ++p) spacing += ray_spacing(vol, cams[cam_for_proj[p]], pin[p].pose);
   L.ray_spacing = (float)(spacing / (double)num_projs);
   L.vol_bytes = vol->bytes;
+  L.plain = vol->raw != nullptr;
   L.reuse = var.reuse;
   L.wave_shape = var.shape;
   launch_drr_setup(L, ctx->stream);
