@@ -855,7 +855,9 @@ __device__ __forceinline__ float cast_ray_slab(const DrrItem& it, const TileRef&
   // this lane's line of the hull: corner lane & 3, axis B or C, as position = u + v * (position on A).
   // (u in double: a source far from the volume is a large number, of which little remains)
   const int hk = lane & 3, hax = (lane & 8) ? C : B;
-  const double hvd = corner[hk][hax] / corner[hk][A];
+  const double hc = corner[hk][hax], ha = corner[hk][A];
+  const float hr = __builtin_amdgcn_rcpf((float)ha), h0 = (float)hc * hr;
+  const double hvd = (double)h0 + fma(-(double)h0, ha, hc) * (double)hr;  // hc / ha to about 1e-13
   const float hv = (float)hvd, hu = (float)(origin[hax] - origin[A] * hvd);
   // the cells along A that the block's samples reach. The margin covers the rounding of the lines
   // and the samples, which grows with their coordinates; under FP32 set-up also that of the set-up
@@ -1139,7 +1141,7 @@ __global__ __launch_bounds__(kThreads * (kParts > 1 ? kParts : 1), kParts == 0 ?
 // launch followed by ACCUM launches. The item's first entry carries the output offset, the
 // detector and the fused NCC reference.
 template <int kGeom, int kOp, int kFmt, int kParts>
-__global__ __launch_bounds__(kThreads * (kParts > 1 ? kParts : 1), kParts == 0 ? 4 : 8) void drr_objects_kernel(
+__global__ __launch_bounds__(kThreads * (kParts > 1 ? kParts : 1), kParts == 0 ? 7 : 8) void drr_objects_kernel(
     const DrrItem* __restrict__ items, const uint32_t* __restrict__ band_start, int64_t num_items,
     int bands, float* __restrict__ out, float fill, double* __restrict__ ncc_partials, int ncc_tiles,
     int shape, int budget, int window, int objs)
