@@ -422,8 +422,8 @@ xrh_status xrh_batch_last_timing(const xrh_batch* batch, float* drr_kernel_ms, f
  * are identical under all of them (fused NCC sums may differ in the last FP64 bits: the
  * per-tile summation order follows the wave footprint).
  *   cell_reuse  1: one lane marches a whole ray; 0: two or four waves share each ray (the most
- *               that keeps every workgroup resident, at least two); -1: by launch size (shared
- *               when at least two waves per ray keep every workgroup resident)
+ *               that keeps every workgroup resident, at least two); -1: chosen for the launch by its
+ *               workgroups, the distance of its rays, the volumes' bytes and storage
  *   wave_shape  pixels per wave64 inside the 16x16 workgroup tile: 0 = 8x8, 1 = 16x4, 2 = 4x16
  *   bands       detector-row bands of the XCD-aware workgroup order, 1..16 (default 8)
  * The environment variable XRH_CELL_REUSE, when set, still overrides cell_reuse. */
@@ -434,7 +434,7 @@ typedef struct xrh_drr_variant {
 } xrh_drr_variant;
 
 typedef struct xrh_tune_result {
-  xrh_drr_variant chosen;  /* cell_reuse resolved to 0 / 1 */
+  xrh_drr_variant chosen;  /* cell_reuse resolved to what runs: 0 / 1 */
   float chosen_ms;         /* DRR kernel time of the chosen variant (minimum over reps) */
   float default_ms;        /* the same for the default variant {-1, 0, 8} */
   int32_t variants_timed;
@@ -446,9 +446,9 @@ typedef struct xrh_tune_result {
  * {0,1,2} x bands {4,8,16}, then the default again), each reps + 1 times with HIP events
  * around the DRR kernel (the minimum of the last reps), and keeps the fastest if it beats the
  * default's better timing by 1%, for this batch and, in the context, for later batch and
- * xrh_line_int launches with the same storage, layout, geometry mode, line kernel, largest
- * detector and workgroups per CU (power-of-two bucket). Synchronous; runs 20 * (reps + 1)
- * submissions. */
+ * xrh_line_int launches with the same storage, layout, geometry mode, line kernel, objects per
+ * item and largest detector, about as many workgroups per CU and bytes in the largest volume (powers
+ * of two) and rays about as far apart (half octaves). Synchronous; runs 20 * (reps + 1) submissions. */
 xrh_status xrh_batch_autotune(xrh_batch* batch, const int32_t* item_view, const double* item_pose,
                               int64_t n_items, int32_t reps, xrh_tune_result* out);
 

@@ -257,8 +257,30 @@ void batch_create(xrh_ctx* ctx, const xrh_view* views, int32_t num_views, int64_
   *out = b;
 }
 
+// What the way of marching n items of `objs` entries each is chosen by.
+DrrLaunch launch_facts(const xrh_batch* b, const int32_t* item_view, const double* item_pose, int64_t n, int32_t objs)
+{
+  DrrLaunch D;
+  std::memset(&D, 0, sizeof(D));
+  D.geom = b->geom;
+  D.kernel = b->views[0].kernel;
+  D.storage = b->storage;
+  D.layout = b->layout;
+  D.objs = objs;
+  D.plain = true;
+  double spacing = 0.0;
+  for (int64_t e = 0; e < n * objs; ++e) {
+    const xrh_view& w = b->views[item_view[e]];
+    spacing += ray_spacing(w.vol, w.cam, item_pose + 16 * e);
+    D.vol_bytes = std::max<uint64_t>(D.vol_bytes, w.vol->bytes);
+    D.plain = D.plain && w.vol->raw;
+  }
+  D.ray_spacing = (float)(spacing / (double)(n * objs));
+  return D;
+}
+
 // Tuned-variant key of a launch over items of these detector sizes.
-std::string tune_key(const xrh_batch* b, const std::vector<int32_t>& rows, const std::vector<int32_t>& cols)
+std::string tune_key(const DrrLaunch& D, const std::vector<int32_t>& rows, const std::vector<int32_t>& cols)
 {
   int32_t mr = 0, mc = 0;
   int64_t wgs = 0;
@@ -267,7 +289,7 @@ std::string tune_key(const xrh_batch* b, const std::vector<int32_t>& rows, const
     mc = std::max(mc, cols[i]);
     wgs += (int64_t)((rows[i] + 15) / 16) * ((cols[i] + 15) / 16);
   }
-  return drr_tune_key(b->storage, b->layout, b->geom, b->views[0].kernel, mr, mc, wgs);
+  return drr_tune_key(D, mr, mc, wgs);
 }
 
 // Fills the pinned staging for n items of `objs` entries each (entry i * objs + k is object k of
@@ -310,10 +332,8 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
     XRH_REQUIRE(w.cam.num_det_rows == w0.cam.num_det_rows && w.cam.num_det_cols == w0.cam.num_det_cols,
                 "the objects of one item must share the detector size");
   }
+  DrrLaunch D = launch_facts(b, item_view, item_pose, n, objs);
   int64_t off = 0;
-  double spacing = 0.0;
-  uint64_t vol_bytes = 0;
-  bool plain = true;
   groups.clear();
   for (int64_t i = 0; i < n; ++i) {
     const int32_t v = item_view[i * objs];
@@ -331,9 +351,6 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
       p.bg = (k == 0 && bg) ? bg + bg_off[(size_t)v] : nullptr;
       p.step = b->views[vk].step;
       p.pad_ = 0;
-      spacing += ray_spacing(b->views[vk].vol, b->views[vk].cam, p.pose);
-      vol_bytes = std::max<uint64_t>(vol_bytes, b->views[vk].vol->bytes);
-      plain = plain && b->views[vk].vol->raw;
     }
     rows[i] = w.cam.num_det_rows;
     cols[i] = w.cam.num_det_cols;
@@ -370,7 +387,7 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
   DrrVariant var = b->variant;
   if (!b->variant_set) {
     var = DrrVariant();
-    const std::string key = tune_key(b, rows, cols);
+    const std::string key = tune_key(D, rows, cols);
     std::lock_guard<std::mutex> lk(b->ctx->mu);
     auto it = b->ctx->tuned.find(key);
     if (it != b->ctx->tuned.end()) var = it->second;
@@ -380,8 +397,6 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
   XRH_REQUIRE(plan.band_start.size() <= L.band_words, "band plan exceeds its staging");
   std::memcpy(b->blob_host + L.off_band, plan.band_start.data(), sizeof(uint32_t) * plan.band_start.size());
 
-  DrrLaunch D;
-  std::memset(&D, 0, sizeof(D));
   D.poses_dev = (const PoseIn*)(b->blob_host_dev + L.off_pose);
   D.vols_dev = b->vols_dev;
   D.cams_dev = b->cams_dev;
@@ -390,21 +405,13 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
   D.num_items = n;
   D.bands = plan.bands;
   D.max_band_tiles = plan.max_band_tiles;
-  D.geom = b->geom;
-  D.kernel = b->views[0].kernel;
   D.store = XRH_STORE_REPLACE;
   D.fill = 0.0f;
-  D.storage = b->storage;
-  D.layout = b->layout;
   D.out = drr;
   D.ncc_partials = b->ncc_partials_dev;
   D.ncc_tiles_per_item = b->max_img_tiles;
-  D.ray_spacing = (float)(spacing / (double)(n * objs));
-  D.vol_bytes = vol_bytes;
-  D.plain = plain;
   D.reuse = var.reuse;
   D.wave_shape = var.shape;
-  D.objs = objs;
   b->last_plan = drr_launch_plan(D);
   return D;
 }
@@ -598,14 +605,17 @@ void autotune(xrh_batch* b, const int32_t* item_view, const double* item_pose, i
   restore();
   b->variant = best_v;
   b->variant_set = true;
-  int64_t wgs = 0;
-  for (size_t i = 0; i < rows.size(); ++i) wgs += (int64_t)((rows[i] + 15) / 16) * ((cols[i] + 15) / 16);
+  DrrLaunch D = launch_facts(b, item_view, item_pose, n, 1);
   {
-    const std::string key = tune_key(b, rows, cols);
+    const std::string key = tune_key(D, rows, cols);
     std::lock_guard<std::mutex> lk(b->ctx->mu);
     b->ctx->tuned[key] = best_v;
   }
-  out->chosen.cell_reuse = best_v.reuse >= 0 ? best_v.reuse : (drr_default_reuse(wgs) ? 1 : 0);
+  const TilePlan plan = build_tiles(rows, cols, best_v.bands);
+  D.bands = plan.bands;
+  D.max_band_tiles = plan.max_band_tiles;
+  D.reuse = best_v.reuse;
+  out->chosen.cell_reuse = drr_whole_rays(D) ? 1 : 0;
   out->chosen.wave_shape = best_v.shape;
   out->chosen.bands = best_v.bands;
   out->chosen_ms = best_ms;

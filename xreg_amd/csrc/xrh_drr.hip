@@ -31,6 +31,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 
@@ -1405,18 +1406,20 @@ int drr_slab_lds(float spacing, int32_t geom, uint64_t bytes, int32_t storage, i
   return slab_lds(spacing);
 }
 
-bool drr_default_reuse(int64_t workgroups) { return drr_parts(workgroups, 0.0f, 0, XRH_F32) == 1; }
+bool drr_whole_rays(const DrrLaunch& L) { return drr_march(L, L.max_band_tiles * L.bands).parts == 1; }
 
-std::string drr_tune_key(int32_t storage, int32_t layout, int32_t geom, int32_t kernel, int32_t max_rows,
-                         int32_t max_cols, int64_t workgroups)
+std::string drr_tune_key(const DrrLaunch& L, int32_t max_rows, int32_t max_cols, int64_t workgroups)
 {
-  const int64_t per_cu = workgroups / (int64_t)device_cus();
-  int lg = 0;
-  while (lg < 40 && (2ll << lg) <= per_cu) ++lg;
-  char buf[160];
-  std::snprintf(buf, sizeof(buf), "s%d.l%d.g%d.k%d.%dx%d.wg%d", storage, layout, geom, kernel, max_rows, max_cols,
-                per_cu > 0 ? lg : -1);
-  return buf;
+  auto octave = [](double x) { return x > 0.0 ? std::ilogb(x) : INT_MIN; };
+  const int per_cu = octave((double)(workgroups / std::max(device_cus(), 1)));
+  const int spacing = L.ray_spacing > 0.0f ? octave((double)L.ray_spacing * L.ray_spacing) : INT_MIN;  // half octaves
+  std::string key;
+  for (int64_t v : {(int64_t)L.storage, (int64_t)L.layout, (int64_t)L.geom, (int64_t)L.kernel,
+                    (int64_t)std::max(L.objs, 1), (int64_t)L.plain, (int64_t)max_rows, (int64_t)max_cols,
+                    (int64_t)per_cu, (int64_t)octave((double)L.vol_bytes), (int64_t)spacing}) {
+    key += std::to_string(v) + " ";
+  }
+  return key;
 }
 
 TilePlan build_tiles(const std::vector<int32_t>& rows, const std::vector<int32_t>& cols, int32_t bands)

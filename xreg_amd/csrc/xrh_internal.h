@@ -319,8 +319,6 @@ struct DrrLaunch {
                             // the item's pixels (first onto its background or fill, the rest
                             // added), REPLACE only
 };
-// Key of the tuned-variant table: storage, layout, geometry, line kernel, the largest
-// detector of the launch and its workgroups per CU (rounded down to a power of two).
 // Layout bytes from which a volume is not held by the caches.
 constexpr uint64_t kSlabBytes = 64ull << 20;
 // The slab-marching choice of a launch over volumes with plain voxels (its dynamic LDS bytes, 0: gathering).
@@ -330,10 +328,12 @@ int64_t drr_launch_plan(const DrrLaunch& L);
 // Distance (voxels) of neighbouring rays at the volume's centre for a camera and a row-major
 // cam->phys pose.
 float ray_spacing(const xrh_volume* vol, const xrh_camera& cam, const double pose[16]);
-std::string drr_tune_key(int32_t storage, int32_t layout, int32_t geom, int32_t kernel, int32_t max_rows,
-                         int32_t max_cols, int64_t workgroups);
-// Whether an untuned launch of `workgroups` workgroups marches whole rays (reuse = -1).
-bool drr_default_reuse(int64_t workgroups);
+// Key of the tuned-variant table: what the best variant turns on -- storage, layout, geometry, line kernel,
+// objects per item and whether slabs are possible; the largest detector; and, in powers of two, the
+// launch's workgroups per CU and its largest volume's bytes; in half octaves the distance of its rays.
+std::string drr_tune_key(const DrrLaunch& L, int32_t max_rows, int32_t max_cols, int64_t workgroups);
+// Whether a launch marches whole rays (otherwise several waves share each).
+bool drr_whole_rays(const DrrLaunch& L);
 constexpr int32_t kMaxDrrBands = 16;
 // Words copied beside the set-up, from pinned host memory into device memory.
 struct SetupCopy {

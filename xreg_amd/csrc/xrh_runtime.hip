@@ -661,11 +661,26 @@ static void line_int_launch(xrh_ctx* ctx, const xrh_volume* vol, const xrh_camer
   ctx_check_range(ctx, drr_dev, (uint64_t)(npx * num_projs) * 4, "DRR buffer");
   if (bg_dev) ctx_check_range(ctx, bg_dev, (uint64_t)(npx * num_cams) * 4, "background images");
 
-  // a variant tuned for this launch shape (xrh_batch_autotune), else the defaults
+  DrrLaunch L;
+  std::memset(&L, 0, sizeof(L));
+  L.geom = geom;
+  L.kernel = kernel;
+  L.storage = vol->desc.storage;
+  L.layout = vol->desc.layout;
+  double spacing = 0.0;
+  for (int64_t p = 0; p < num_projs; ++p) {
+    double pose[16];
+    for (int i = 0; i < 16; ++i) pose[i] = (double)xforms[16 * p + i];
+    spacing += ray_spacing(vol, cams[cam_for_proj[p]], pose);
+  }
+  L.ray_spacing = (float)(spacing / (double)num_projs);
+  L.vol_bytes = vol->bytes;
+  L.plain = vol->raw != nullptr;
+  // a variant tuned for launches like this one (xrh_batch_autotune), else the defaults
   DrrVariant var;
   if (!fixed) {
     const int64_t wgs = (int64_t)((rows + 15) / 16) * ((cols + 15) / 16) * num_projs;
-    const std::string key = drr_tune_key(vol->desc.storage, vol->desc.layout, geom, kernel, rows, cols, wgs);
+    const std::string key = drr_tune_key(L, rows, cols, wgs);
     std::lock_guard<std::mutex> lk(ctx->mu);
     auto it = ctx->tuned.find(key);
     if (it != ctx->tuned.end()) var = it->second;
@@ -723,8 +738,6 @@ static void line_int_launch(xrh_ctx* ctx, const xrh_volume* vol, const xrh_camer
       XRH_HIP_CHECK(hipGetLastError());
     }
   }
-  DrrLaunch L;
-  std::memset(&L, 0, sizeof(L));
   L.poses_dev = (const PoseIn*)(dev + off_pose);
   L.vols_dev = (const VolDesc*)(dev + off_vol);
   L.cams_dev = (const CamDev*)(dev + off_cam);
@@ -733,19 +746,10 @@ static void line_int_launch(xrh_ctx* ctx, const xrh_volume* vol, const xrh_camer
   L.num_items = num_projs;
   L.bands = bands;
   L.max_band_tiles = max_band_tiles;
-  L.geom = geom;
-  L.kernel = kernel;
   L.store = (store == XRH_STORE_ACCUM || bg_dev) ? XRH_STORE_ACCUM : XRH_STORE_REPLACE;
   L.fill = default_bg;
-  L.storage = vol->desc.storage;
-  L.layout = vol->desc.layout;
   L.out = drr_dev;
   L.sample_counter = samples_out ? (uint64_t*)(dev + off_cnt) : nullptr;
-  double spacing = 0.0;
-  for (int64_t p = 0; p < num_projs; ++p) spacing += ray_spacing(vol, cams[cam_for_proj[p]], pin[p].pose);
-  L.ray_spacing = (float)(spacing / (double)num_projs);
-  L.vol_bytes = vol->bytes;
-  L.plain = vol->raw != nullptr;
   L.reuse = var.reuse;
   L.wave_shape = var.shape;
   launch_drr_setup(L, ctx->stream);
