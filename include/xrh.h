@@ -131,7 +131,9 @@ xrh_status xrh_ctx_destroy(xrh_ctx* ctx);
 xrh_status xrh_ctx_synchronize(xrh_ctx* ctx);
 /* The context's hipStream_t, for callers that order their own work against it. */
 void* xrh_ctx_stream(xrh_ctx* ctx);
-/* Bytes currently charged to the budget. */
+/* Bytes currently charged to the budget. The plain voxels that the context keeps beside its volumes'
+ * default layouts (4 bytes per padded voxel, for marching by slabs) are not: they are kept while the budget
+ * and the device have room, and given back when an allocation needs it. */
 uint64_t xrh_ctx_bytes_in_use(const xrh_ctx* ctx);
 
 /* Device memory charged to the context budget (DRR buffers, background images...). */
@@ -176,8 +178,8 @@ xrh_status xrh_volume_create_layout(xrh_ctx* ctx, const float* vox, const int64_
 xrh_status xrh_volume_create_hu(xrh_ctx* ctx, const float* vox_hu, const int64_t size[3],
                                 const float idx_to_phys[16], int32_t storage, int32_t layout,
                                 double hu_lower, double mu_water, double mu_air, xrh_volume** out);
-/* Device bytes held by the volume: its layout, the plain voxels kept beside it (4 bytes per padded
- * voxel of the default layouts; none in a context with an HBM budget) and any interpolation grids. */
+/* Device bytes held by the volume: its layout and any interpolation grids (not the plain voxels that the
+ * context may keep beside it, see xrh_ctx_bytes_in_use). */
 uint64_t xrh_volume_bytes(const xrh_volume* vol);
 /* Storage type and HBM layout a volume was built with (the automatic choice included: a
  * volume whose packed layout would pass 4 GiB is kept linear). Volumes batched together must

@@ -10,12 +10,16 @@ from tests.helpers import poses_f32
 pytestmark = pytest.mark.gpu
 
 
+BUDGET = 1 << 30
+
+
 @pytest.fixture(scope="module")
 def gather_ctx():
-    """A context whose volumes keep no plain voxels: whole rays gather."""
+    """A context with a budget: taking all of it that is free makes its volumes give up their plain voxels,
+    and whole rays gather then."""
     from xreg_amd import _xrh as X
 
-    c = X.Context(0, hbm_budget_bytes=8 << 30)
+    c = X.Context(0, hbm_budget_bytes=BUDGET)
     yield c
     c.close()
 
@@ -55,6 +59,8 @@ def test_all_marches_equal(ctx, gather_ctx, monkeypatch, spacing, geom, layout):
     for c, reuse in ((ctx, "1"), (gather_ctx, "1"), (ctx, "0"), (gather_ctx, "0")):
         monkeypatch.setenv("XRH_CELL_REUSE", reuse)
         vol = X.Volume(c, vox, G.idx_to_phys(1.0), layout=lay)
+        if c is gather_ctx:
+            c.alloc(BUDGET - c.bytes_in_use()).free()
         buf = c.alloc(4 * n * rows * cols)
         X.line_int(c, vol, [cam], poses_f32(poses), np.zeros(n, np.int64), 0.43, buf, geom=geom)
         got.append(buf.download(np.float32))

@@ -31,6 +31,7 @@ struct xrh_batch {
   // current view table
   std::vector<xrh_view> views;
   std::vector<int32_t> view_vol;   // view -> index into the volume table
+  uint64_t plain_epoch = 0;        // of the volume table (xrh_ctx::plain_epoch)
   int32_t storage = XRH_F32, layout = kLayoutQuad;
   int max_img_tiles = 0, max_patch_tiles = 0, max_lds = 0;
   bool fuse_ncc = true;            // NCC sums in the DRR epilogue (off if any NCC view is masked)
@@ -183,6 +184,7 @@ void set_views(xrh_batch* b, const xrh_view* views, int32_t num_views)
   XRH_REQUIRE(b && views, "null argument");
   XRH_REQUIRE(!b->pending, "batch has a launch in flight");
   XRH_REQUIRE(num_views >= 1 && num_views <= b->cap_views, "view count exceeds the batch capacity");
+  std::lock_guard<std::recursive_mutex> plain(b->ctx->plain_mu);
   std::vector<CamDev> cams;
   std::vector<VolDesc> vds;
   std::vector<const xrh_volume*> vols;
@@ -222,6 +224,7 @@ void set_views(xrh_batch* b, const xrh_view* views, int32_t num_views)
   }
   hipStream_t s = b->ctx->stream;
   XRH_HIP_CHECK(hipStreamSynchronize(s));
+  b->plain_epoch = b->ctx->plain_epoch;
   XRH_HIP_CHECK(hipMemcpyAsync(b->vols_dev, vds.data(), sizeof(VolDesc) * vds.size(), hipMemcpyHostToDevice, s));
   XRH_HIP_CHECK(hipMemcpyAsync(b->cams_dev, cams.data(), sizeof(CamDev) * cams.size(), hipMemcpyHostToDevice, s));
   XRH_HIP_CHECK(hipStreamSynchronize(s));
@@ -255,6 +258,21 @@ void batch_create(xrh_ctx* ctx, const xrh_view* views, int32_t num_views, int64_
     throw;
   }
   *out = b;
+}
+
+// Brings the volume table up to date when plain voxels were given back since it was written (no launch of
+// the batch is in flight, and the caller holds the context's plain_mu).
+void refresh_volumes(xrh_batch* b)
+{
+  if (b->plain_epoch == b->ctx->plain_epoch) return;
+  std::vector<VolDesc> vds;
+  for (size_t v = 0; v < b->views.size(); ++v) {
+    if (b->view_vol[v] == (int32_t)vds.size()) vds.push_back(b->views[v].vol->desc);
+  }
+  hipStream_t s = b->ctx->stream;
+  XRH_HIP_CHECK(hipMemcpyAsync(b->vols_dev, vds.data(), sizeof(VolDesc) * vds.size(), hipMemcpyHostToDevice, s));
+  XRH_HIP_CHECK(hipStreamSynchronize(s));
+  b->plain_epoch = b->ctx->plain_epoch;
 }
 
 // What the way of marching n items of `objs` entries each is chosen by.
@@ -301,6 +319,7 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
                 const float* bg = nullptr)
 {
   XRH_REQUIRE(!b->views.empty(), "batch has no views");
+  refresh_volumes(b);
   XRH_REQUIRE(objs >= 1 && n * objs <= b->max_items, "items x objects exceed the batch capacity (max_items)");
   const BlobLayout L = blob_layout(b->max_items);
   PoseIn* pin = (PoseIn*)(b->blob_host + L.off_pose);
@@ -476,6 +495,7 @@ void launch(xrh_batch* b, const int32_t* item_view, const double* item_pose, int
   XRH_REQUIRE(!b->pending, "previous launch not yet waited for");
   hipStream_t s = b->ctx->stream;
   XRH_HIP_CHECK(hipStreamSynchronize(s));  // pinned staging is reused
+  std::lock_guard<std::recursive_mutex> plain(b->ctx->plain_mu);  // (until the launch is queued)
   std::vector<std::pair<int, std::vector<int64_t>>> groups;
   const DrrLaunch D = stage(b, item_view, item_pose, n, drr_out, groups, objs, bg);
   const bool timed = b->time_kernels || !b->use_graph;
@@ -605,6 +625,7 @@ void autotune(xrh_batch* b, const int32_t* item_view, const double* item_pose, i
   restore();
   b->variant = best_v;
   b->variant_set = true;
+  std::lock_guard<std::recursive_mutex> plain(b->ctx->plain_mu);
   DrrLaunch D = launch_facts(b, item_view, item_pose, n, 1);
   {
     const std::string key = tune_key(D, rows, cols);
@@ -634,11 +655,11 @@ void count_samples(xrh_batch* b, const int32_t* item_view, const double* item_po
   XRH_REQUIRE(n >= 1 && n <= b->max_items, "item count must be in [1, max_items]");
   hipStream_t s = b->ctx->stream;
   XRH_HIP_CHECK(hipStreamSynchronize(s));
+  std::lock_guard<std::recursive_mutex> plain(b->ctx->plain_mu);
+  uint64_t* cnt = (uint64_t*)ctx_scratch(b->ctx, 16);
   std::vector<std::pair<int, std::vector<int64_t>>> groups;
   // staged as if writing DRRs to steps_dev, so every item's out_off indexes that buffer
   DrrLaunch D = stage(b, item_view, item_pose, n, (float*)steps_dev, groups);
-  const BlobLayout L = blob_layout(b->max_items);
-  uint64_t* cnt = (uint64_t*)ctx_scratch(b->ctx, 16);
   uint64_t both[2] = {0, 0};
   XRH_HIP_CHECK(hipMemcpyAsync(cnt, both, 16, hipMemcpyHostToDevice, s));
   D.sample_counter = cnt;

@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <map>
 #include <mutex>
+#include <set>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -187,6 +188,8 @@ struct DrrVariant {
 };
 }  // namespace xrh
 
+struct xrh_volume;
+
 struct xrh_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -195,6 +198,14 @@ struct xrh_ctx {
   std::mutex mu;
   std::unordered_map<void*, uint64_t> allocs;
   int num_cus = 0;
+  // Plain voxels beside the layouts of the context's volumes: kept while there is room, given back when an
+  // allocation needs theirs, and charged to no one. A launch holds plain_mu from reading a volume's
+  // description until its work is queued, so what it queued is complete before the voxels are freed; plain_epoch
+  // tells copies of the descriptions that they are stale. (mu guards plain_bytes.)
+  std::recursive_mutex plain_mu;
+  std::set<xrh_volume*> plain;
+  uint64_t plain_bytes = 0;
+  uint64_t plain_epoch = 0;
   // reusable staging for xrh_line_int / xrh_sim_compute
   void* scratch = nullptr;
   uint64_t scratch_bytes = 0;
@@ -228,9 +239,9 @@ constexpr int kGridBSpline = 1;
 struct xrh_volume {
   xrh_ctx* ctx = nullptr;
   xrh::VolDesc desc{};
-  void* data = nullptr;  // the allocation: the layout, the map and the plain voxels
+  void* data = nullptr;  // the layout and the map
   void* skip = nullptr;
-  void* raw = nullptr;
+  void* raw = nullptr;   // the plain voxels, or null
   uint64_t bytes = 0;    // of the layout
   int64_t size[3] = {0, 0, 0};
   double center[3] = {0, 0, 0};  // physical
@@ -243,7 +254,8 @@ struct xrh_volume {
 
 namespace xrh {
 
-// context-budgeted allocation helpers (defined in xrh_runtime.hip)
+// context-budgeted allocation helpers (defined in xrh_runtime.hip); where room is short, the context's
+// plain voxels go first
 void* ctx_alloc(xrh_ctx* ctx, uint64_t bytes);
 void ctx_free(xrh_ctx* ctx, void* p);
 // Fails with XRH_ERR_INVALID when [p, p + bytes) starts inside one of the context's

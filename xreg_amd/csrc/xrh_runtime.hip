@@ -18,9 +18,65 @@ void set_error(const std::string& msg) { g_last_error = msg; }
 
 [[noreturn]] void fail(xrh_status s, const std::string& msg) { throw Error{s, msg}; }
 
+// Frees plain voxels of the context's volumes until `bytes` are free'd or none are left (the caller holds
+// plain_mu). Everything that may read them is on the context's stream.
+static void plain_free(xrh_ctx* ctx, uint64_t bytes)
+{
+  XRH_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+  for (uint64_t done = 0; done < bytes && !ctx->plain.empty();) {
+    xrh_volume* v = *ctx->plain.begin();
+    const uint64_t n = v->desc.raw_bytes;
+    void* p = v->raw;
+    v->raw = nullptr;
+    v->desc.raw = nullptr;
+    v->desc.raw_bytes = 0;
+    ctx->plain.erase(ctx->plain.begin());
+    ++ctx->plain_epoch;
+    {
+      std::lock_guard<std::mutex> lk(ctx->mu);
+      ctx->plain_bytes -= n;
+    }
+    done += n;
+    XRH_HIP_CHECK(hipFree(p));
+  }
+}
+
+// Memory for the plain voxels of a volume whose upload takes `upload` bytes, or null: only where an eighth of
+// the device stays free and within the budget, which is to allow the upload beside them.
+static void* plain_alloc(xrh_ctx* ctx, uint64_t bytes, uint64_t upload)
+{
+  size_t room = 0, total = 0;
+  if (hipMemGetInfo(&room, &total) != hipSuccess || room < bytes + total / 8) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  {
+    std::lock_guard<std::mutex> lk(ctx->mu);
+    if (ctx->budget && ctx->in_use + ctx->plain_bytes + bytes + upload > ctx->budget) return nullptr;
+    ctx->plain_bytes += bytes;
+  }
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    std::lock_guard<std::mutex> lk(ctx->mu);
+    ctx->plain_bytes -= bytes;
+    return nullptr;
+  }
+  return p;
+}
+
+// Frees plain voxels that no volume holds any more.
+static void plain_drop(xrh_ctx* ctx, void* p, uint64_t bytes)
+{
+  (void)hipFree(p);
+  std::lock_guard<std::mutex> lk(ctx->mu);
+  ctx->plain_bytes -= bytes;
+}
+
 void* ctx_alloc(xrh_ctx* ctx, uint64_t bytes)
 {
   if (bytes == 0) bytes = 256;
+  uint64_t over = 0;  // of the budget, with the plain voxels
   {
     std::lock_guard<std::mutex> lk(ctx->mu);
     if (ctx->budget && ctx->in_use + bytes > ctx->budget) {
@@ -28,14 +84,35 @@ void* ctx_alloc(xrh_ctx* ctx, uint64_t bytes)
                                std::to_string(bytes) + " > " + std::to_string(ctx->budget));
     }
     ctx->in_use += bytes;
+    if (ctx->budget && ctx->in_use + ctx->plain_bytes > ctx->budget) over = ctx->in_use + ctx->plain_bytes - ctx->budget;
   }
   void* p = nullptr;
-  const hipError_t e = hipMalloc(&p, bytes);
-  if (e != hipSuccess) {
+  try {
+    if (over) {
+      std::lock_guard<std::recursive_mutex> lk(ctx->plain_mu);
+      plain_free(ctx, over);
+    }
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      // once more without the plain voxels, if that can be enough
+      std::lock_guard<std::recursive_mutex> lk(ctx->plain_mu);
+      size_t room = 0, total = 0;
+      uint64_t plain = 0;
+      for (xrh_volume* v : ctx->plain) plain += v->desc.raw_bytes;
+      if (plain && hipMemGetInfo(&room, &total) == hipSuccess && room + plain >= bytes) {
+        plain_free(ctx, plain);
+        e = hipMalloc(&p, bytes);
+      }
+    }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      fail(XRH_ERR_OOM, "hipMalloc(" + std::to_string(bytes) + ") failed: " + hipGetErrorString(e));
+    }
+  } catch (...) {
     std::lock_guard<std::mutex> lk(ctx->mu);
     ctx->in_use -= bytes;
-    (void)hipGetLastError();
-    fail(XRH_ERR_OOM, "hipMalloc(" + std::to_string(bytes) + ") failed: " + hipGetErrorString(e));
+    throw;
   }
   std::lock_guard<std::mutex> lk(ctx->mu);
   ctx->allocs[p] = bytes;
@@ -215,12 +292,12 @@ __device__ inline float4 face(float v00, float v10, float v01, float v11)
   return make_float4(v00, v10 - v00, v01, v11 - v01);
 }
 
-// Builds the padded layout from the raw x-fastest volume. One thread per padded voxel. kLayoutPlain:
-// the values that the storage type holds, as floats.
+// Builds the padded layout from the raw x-fastest volume, or (`padded`) from its plain voxels. One thread per
+// padded voxel. kLayoutPlain: the values that the storage type holds, as floats.
 constexpr int kLayoutPlain = -1;
 
 __global__ void build_layout_kernel(const float* __restrict__ src, int X, int Y, int Z,
-                                    void* __restrict__ dst, int storage, int layout)
+                                    void* __restrict__ dst, int storage, int layout, bool padded)
 {
   const int64_t Xp = X + 2, Yp = Y + 2, Zp = Z + 2;
   const int64_t n = Xp * Yp * Zp;
@@ -230,6 +307,7 @@ __global__ void build_layout_kernel(const float* __restrict__ src, int X, int Y,
   const int b = (int)((i / Xp) % Yp);
   const int c = (int)(i / (Xp * Yp));
   auto V = [&](int aa, int bb, int cc) -> float {
+    if (padded) return src[min(aa, X + 1) + Xp * (min(bb, Y + 1) + Yp * min(cc, Z + 1))];
     // padded index -> source index with edge replication
     int x = min(max(aa - 1, 0), X - 1);
     int y = min(max(bb - 1, 0), Y - 1);
@@ -450,6 +528,16 @@ static void volume_create(xrh_ctx* ctx, const float* vox, const int64_t size[3],
   const uint64_t bytes = (layout == kLayoutBrick) ? (uint64_t)(nbx * nby * nbz * kBrickFaces * 16)
                                                   : (uint64_t)(padded * esize);
   XRH_REQUIRE(bytes < 0xFFFFF000ull, "volume layout exceeds 4 GiB; use the linear layout or split the volume");
+  float ms = INFINITY;
+  double chord = 0.0;
+  const int64_t dims[3] = {X, Y, Z};
+  for (int c = 0; c < 3; ++c) {
+    const float n = std::sqrt(idx_to_phys[c] * idx_to_phys[c] + idx_to_phys[4 + c] * idx_to_phys[4 + c] +
+                              idx_to_phys[8 + c] * idx_to_phys[8 + c]);
+    ms = std::min(ms, n);
+    chord += (double)n * (double)(dims[c] + 1);  // +1: the nudge and edge samples
+  }
+  XRH_REQUIRE(ms > 0.0f && std::isfinite(ms), "idx_to_phys has a zero or non-finite column");
   auto* v = new xrh_volume();
   v->ctx = ctx;
   v->size[0] = X;
@@ -462,33 +550,26 @@ static void volume_create(xrh_ctx* ctx, const float* vox, const int64_t size[3],
   const int64_t sgx = (X + SB - 1) / SB, sgy = (Y + SB - 1) / SB, sgz = (Z + SB - 1) / SB, nb = sgx * sgy * sgz;
   // the walk indexes the map with 24-bit multiply-adds: larger maps go without skipping
   const bool skip = skip_enabled() && nb < (int64_t(1) << 24) && sgy * sgz < (int64_t(1) << 24);
-  // one allocation: the layout, the empty-space map and the plain voxels beside the packed layout. A context
-  // with a budget goes without the plain voxels (4 bytes a voxel more, used by the slabs only), so
-  // what fitted a budget without them fits it still
-  bool plain = (layout == kLayoutFace || layout == kLayoutOct) && !ctx->budget;
-  auto pad = [](uint64_t x) { return (x + 255) & ~uint64_t(255); };
-  const uint64_t map_end = bytes + (skip ? (uint64_t)nb : 0), off_plain = pad(map_end);
+  // One allocation for the layout and the empty-space map. With plain voxels (for slab marching, if there is
+  // room) the upload lies in the layout's memory, which is built from them last (one allocation and
+  // release less: 256 x 256 x 200 voxels 2476 us, 2856 with three); else in memory of its own.
+  const uint64_t map_end = bytes + (skip ? (uint64_t)nb : 0), up_bytes = (uint64_t)(X * Y * Z) * 4;
+  const int64_t up_off = (int64_t)((bytes - std::min(bytes, up_bytes)) & ~uint64_t(255));
   try {
-    if (plain) {
-      try {
-        v->data = ctx_alloc(ctx, off_plain + raw_alloc_bytes(padded));
-        v->raw = (char*)v->data + off_plain;
-      } catch (const Error&) {
-        plain = false;  // memory nearly full: without them too
-      }
-    }
-    if (!plain) v->data = ctx_alloc(ctx, map_end);
+    v->data = ctx_alloc(ctx, map_end);
     v->bytes = bytes;
     if (skip) v->skip = (char*)v->data + bytes;
-    raw = ctx_alloc(ctx, (uint64_t)(X * Y * Z) * 4);
-    XRH_HIP_CHECK(hipMemcpyAsync(raw, vox, (size_t)(X * Y * Z) * 4, hipMemcpyHostToDevice, ctx->stream));
+    if (layout == kLayoutFace || layout == kLayoutOct) v->raw = plain_alloc(ctx, raw_alloc_bytes(padded), up_bytes);
+    if (!v->raw) raw = ctx_alloc(ctx, up_bytes);
+    float* up = (float*)(v->raw ? (char*)v->data + up_off : (char*)raw);
+    XRH_HIP_CHECK(hipMemcpyAsync(up, vox, (size_t)up_bytes, hipMemcpyHostToDevice, ctx->stream));
     const int threads = 256;
     auto grid = [&](int64_t n) { return dim3((unsigned)((n + threads - 1) / threads)); };
     if (hu) {
       const double hu_scale = (hu->mu_water - hu->mu_air) * 1.0e-3;
       const double mu_lower = (hu->hu_lower * hu_scale) + hu->mu_water;
       const int64_t nv = X * Y * Z;
-      hipLaunchKernelGGL(hu_to_lin_att_kernel, grid(nv), dim3(threads), 0, ctx->stream, (float*)raw, nv, hu_scale,
+      hipLaunchKernelGGL(hu_to_lin_att_kernel, grid(nv), dim3(threads), 0, ctx->stream, up, nv, hu_scale,
                          hu->mu_water, mu_lower);
       XRH_HIP_CHECK(hipGetLastError());
     }
@@ -497,12 +578,13 @@ static void volume_create(xrh_ctx* ctx, const float* vox, const int64_t size[3],
       skip_dims[1] = (int)sgy;
       skip_dims[2] = (int)sgz;
       // work space: the layout's memory, which is built afterwards (bricks are at least two voxels
-      // wide, so at two bytes a padded voxel it holds a byte per brick of every row and two maps)
+      // wide, so at two bytes a padded voxel, or twelve in front of an upload there, it holds a byte per
+      // brick of every row and two maps)
       uint8_t* rowocc = (uint8_t*)v->data;
       uint8_t *ma = rowocc + sgx * Y * Z, *mb = ma + nb;
-      XRH_REQUIRE((uint64_t)(sgx * Y * Z + 2 * nb) <= bytes, "empty-space map work space");
-      hipLaunchKernelGGL(row_occupancy_kernel, grid(sgx * Y * Z), dim3(threads), 0, ctx->stream, (const float*)raw,
-                         (int)X, Y * Z, SB, (int)sgx, rowocc);
+      XRH_REQUIRE(sgx * Y * Z + 2 * nb <= (v->raw ? up_off : (int64_t)bytes), "empty-space map work space");
+      hipLaunchKernelGGL(row_occupancy_kernel, grid(sgx * Y * Z), dim3(threads), 0, ctx->stream, up, (int)X, Y * Z, SB,
+                         (int)sgx, rowocc);
       hipLaunchKernelGGL(brick_occupancy_kernel, grid(nb), dim3(threads), 0, ctx->stream, (const uint8_t*)rowocc, (int)Y,
                          (int)Z, SB, (int)sgx, (int)sgy, (int)sgz, ma);
       hipLaunchKernelGGL(chessboard_axis_kernel<true>, grid(nb), dim3(threads), 0, ctx->stream, (const uint8_t*)ma, sgx,
@@ -515,21 +597,23 @@ static void volume_create(xrh_ctx* ctx, const float* vox, const int64_t size[3],
     }
     // brick entries past the volume's faces are never sampled; zero them all the same
     if (layout == kLayoutBrick) XRH_HIP_CHECK(hipMemsetAsync(v->data, 0, bytes, ctx->stream));
-    hipLaunchKernelGGL(build_layout_kernel, grid(padded), dim3(threads), 0, ctx->stream, (const float*)raw, (int)X,
-                       (int)Y, (int)Z, v->data, storage, layout);
-    XRH_HIP_CHECK(hipGetLastError());
-    if (plain) {
-      hipLaunchKernelGGL(build_layout_kernel, grid(padded), dim3(threads), 0, ctx->stream, (const float*)raw, (int)X,
-                         (int)Y, (int)Z, v->raw, storage, kLayoutPlain);
+    if (v->raw) {
+      hipLaunchKernelGGL(build_layout_kernel, grid(padded), dim3(threads), 0, ctx->stream, up, (int)X, (int)Y, (int)Z,
+                         v->raw, storage, kLayoutPlain, false);
       XRH_HIP_CHECK(hipGetLastError());
     }
+    hipLaunchKernelGGL(build_layout_kernel, grid(padded), dim3(threads), 0, ctx->stream,
+                       v->raw ? (const float*)v->raw : up, (int)X, (int)Y, (int)Z, v->data, storage, layout,
+                       v->raw != nullptr);
+    XRH_HIP_CHECK(hipGetLastError());
     XRH_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-    ctx_free(ctx, raw);
+    if (raw) ctx_free(ctx, raw);
     raw = nullptr;
   } catch (...) {
     (void)hipStreamSynchronize(ctx->stream);
     if (raw) ctx_free(ctx, raw);
     if (v->data) ctx_free(ctx, v->data);
+    if (v->raw) plain_drop(ctx, v->raw, raw_alloc_bytes(padded));
     delete v;
     throw;
   }
@@ -559,16 +643,6 @@ static void volume_create(xrh_ctx* ctx, const float* vox, const int64_t size[3],
   }
   d.storage = storage;
   d.layout = layout;
-  float ms = INFINITY;
-  double chord = 0.0;
-  const int64_t dims[3] = {X, Y, Z};
-  for (int c = 0; c < 3; ++c) {
-    const float n = std::sqrt(idx_to_phys[c] * idx_to_phys[c] + idx_to_phys[4 + c] * idx_to_phys[4 + c] +
-                              idx_to_phys[8 + c] * idx_to_phys[8 + c]);
-    ms = std::min(ms, n);
-    chord += (double)n * (double)(dims[c] + 1);  // +1: the nudge and edge samples
-  }
-  XRH_REQUIRE(ms > 0.0f && std::isfinite(ms), "idx_to_phys has a zero or non-finite column");
   d.min_spacing = ms;
   v->spacing = 1.0;
   for (int c = 0; c < 3; ++c) {
@@ -581,6 +655,10 @@ static void volume_create(xrh_ctx* ctx, const float* vox, const int64_t size[3],
     v->spacing *= std::cbrt(std::sqrt(n2));
   }
   d.max_chord = (float)chord;
+  if (v->raw) {
+    std::lock_guard<std::recursive_mutex> lk(ctx->plain_mu);
+    ctx->plain.insert(v);
+  }
   *out = v;
 }
 
@@ -658,6 +736,7 @@ static void line_int_launch(xrh_ctx* ctx, const xrh_volume* vol, const xrh_camer
   }
   const int64_t npx = (int64_t)rows * cols;
   XRH_REQUIRE(npx * num_projs < (1ll << 40), "DRR buffer too large");
+  std::lock_guard<std::recursive_mutex> plain(ctx->plain_mu);  // (to the end of the launch)
   ctx_check_range(ctx, drr_dev, (uint64_t)(npx * num_projs) * 4, "DRR buffer");
   if (bg_dev) ctx_check_range(ctx, bg_dev, (uint64_t)(npx * num_cams) * 4, "background images");
 
@@ -724,6 +803,7 @@ static void line_int_launch(xrh_ctx* ctx, const xrh_volume* vol, const xrh_camer
   CamDev* cd = (CamDev*)(host + off_cam);
   for (int32_t c = 0; c < num_cams; ++c) cd[c] = make_cam_dev(cams[c]);
   std::memcpy(host + off_vol, &vol->desc, sizeof(VolDesc));
+  L.plain = vol->raw != nullptr;  // (the staging's allocation may have needed their room)
   std::memcpy(host + off_c4p, cam_for_proj, sizeof(int64_t) * num_projs);
   std::memset(host + off_cnt, 0, 16);
   XRH_HIP_CHECK(hipMemcpyAsync(dev, host, blob, hipMemcpyHostToDevice, ctx->stream));
@@ -854,6 +934,8 @@ xrh_status xrh_ctx_destroy(xrh_ctx* ctx)
     if (ctx->pinned) XRH_HIP_CHECK(hipHostFree(ctx->pinned));
     for (auto& kv : ctx->allocs) (void)hipFree(kv.first);
     ctx->allocs.clear();
+    for (xrh_volume* v : ctx->plain) (void)hipFree(v->raw);
+    ctx->plain.clear();
     XRH_HIP_CHECK(hipStreamDestroy(ctx->stream));
     delete ctx;
   });
@@ -971,6 +1053,10 @@ xrh_status xrh_volume_destroy(xrh_volume* vol)
   return guarded([&] {
     if (!vol) return;
     XRH_HIP_CHECK(hipStreamSynchronize(vol->ctx->stream));
+    {
+      std::lock_guard<std::recursive_mutex> lk(vol->ctx->plain_mu);
+      if (vol->ctx->plain.erase(vol)) plain_drop(vol->ctx, vol->raw, vol->desc.raw_bytes);
+    }
     ctx_free(vol->ctx, vol->data);
     for (void* g : vol->grid_mem) {
       if (g) ctx_free(vol->ctx, g);
@@ -981,7 +1067,7 @@ xrh_status xrh_volume_destroy(xrh_volume* vol)
 
 uint64_t xrh_volume_bytes(const xrh_volume* vol)
 {
-  return vol ? vol->bytes + vol->desc.raw_bytes + vol->grid_bytes[0] + vol->grid_bytes[1] : 0;
+  return vol ? vol->bytes + vol->grid_bytes[0] + vol->grid_bytes[1] : 0;
 }
 
 xrh_status xrh_volume_info(const xrh_volume* vol, int32_t* storage, int32_t* layout)
