@@ -211,8 +211,9 @@ struct xrh_ctx {
   uint64_t scratch_bytes = 0;
   void* pinned = nullptr;
   uint64_t pinned_bytes = 0;
-  // workspace of the image operations (work_mu held from ctx_work to the end of the work)
-  std::mutex work_mu;
+  // workspace of the image operations in a context without a budget (work_mu held from ctx_work to the end of
+  // the work); charged to no one, given back when an allocation fails
+  std::recursive_mutex work_mu;
   void* work = nullptr;
   uint64_t work_bytes = 0;
   // DRR variants chosen by xrh_batch_autotune, keyed by drr_tune_key
@@ -264,7 +265,7 @@ void ctx_check_range(xrh_ctx* ctx, const void* p, uint64_t bytes, const char* wh
 // grows ctx->scratch to at least `bytes` (device) and returns it
 void* ctx_scratch(xrh_ctx* ctx, uint64_t bytes);
 void* ctx_pinned(xrh_ctx* ctx, uint64_t bytes);
-// grows ctx->work to at least `bytes` (device) and returns it; the caller holds ctx->work_mu
+// grows ctx->work to at least `bytes` (device) and returns it; the caller holds ctx->work_mu (no budget)
 void* ctx_work(xrh_ctx* ctx, uint64_t bytes);
 
 // host-side helpers (xrh_runtime.hip)

@@ -355,18 +355,17 @@ xrh_status xrh_downsample_image(xrh_ctx* ctx, const float* img, int32_t rows, in
       const double s = (sigma < 0.0) ? 0.5 / factor : sigma;
       w = gaussian_kernel(s * s, 0.01, 32);
     }
-    auto pad = [](uint64_t x) { return (x + 255) & ~uint64_t(255); };
-    const uint64_t off_a = pad((uint64_t)n * 4), off_b = off_a + pad((uint64_t)n * 8), off_w = off_b + pad((uint64_t)n * 8),
-                   off_out = off_w + pad(w.size() * 8), total = off_out + pad((uint64_t)on * 4);
-    // the context's image workspace while no other thread has it and it stays small, beside its
-    // budget too (allocating and releasing it were a fifth of a 768 x 768 call); else memory of this
-    // call's own
-    std::unique_lock<std::mutex> lk(ctx->work_mu, std::try_to_lock);
-    const bool own = !lk.owns_lock() || total > (64ull << 20) || (ctx->budget && ctx->in_use + 16 * total > ctx->budget);
+    // two planes of doubles, the weights and the output; the image lies in the plane that its first pass
+    // does not write
+    const uint64_t off_b = (uint64_t)n * 8, off_w = off_b + (uint64_t)n * 8, off_out = off_w + w.size() * 8,
+                   total = off_out + (uint64_t)on * 4;
+    // the context's image workspace while no other thread has it and it stays small (allocating and
+    // releasing it were a fifth of a 768 x 768 call); with a budget, or else, memory of this call's own
+    std::unique_lock<std::recursive_mutex> lk(ctx->work_mu, std::defer_lock);
+    const bool own = ctx->budget || total > (64ull << 20) || !lk.try_lock();
     char* mem = (char*)(own ? ctx_alloc(ctx, total) : ctx_work(ctx, total));
-    float* d_img = (float*)mem;
-    double *d_a = (double*)(mem + off_a), *d_b = (double*)(mem + off_b), *d_w = (double*)(mem + off_w);
-    float* d_out = (float*)(mem + off_out);
+    double *d_a = (double*)mem, *d_b = (double*)(mem + off_b), *d_w = (double*)(mem + off_w);
+    float *d_img = (float*)(smooth ? d_a : d_b), *d_out = (float*)(mem + off_out);
     try {
       hipStream_t s = ctx->stream;
       XRH_HIP_CHECK(hipMemcpyAsync(d_img, img, (size_t)n * 4, hipMemcpyHostToDevice, s));

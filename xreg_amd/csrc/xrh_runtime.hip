@@ -73,6 +73,39 @@ static void plain_drop(xrh_ctx* ctx, void* p, uint64_t bytes)
   ctx->plain_bytes -= bytes;
 }
 
+// hipMalloc; when it fails, once more without the context's plain voxels and idle workspace, if that can be
+// enough. Throws XRH_ERR_OOM.
+static void* device_malloc(xrh_ctx* ctx, uint64_t bytes)
+{
+  void* p = nullptr;
+  hipError_t e = hipMalloc(&p, bytes);
+  if (e == hipSuccess) return p;
+  (void)hipGetLastError();
+  {
+    // (a thread that holds work_mu itself has taken the workspace out of the context before it allocates)
+    std::unique_lock<std::recursive_mutex> wk(ctx->work_mu, std::try_to_lock);
+    std::lock_guard<std::recursive_mutex> lk(ctx->plain_mu);
+    size_t room = 0, total = 0;
+    uint64_t plain = 0;
+    for (xrh_volume* v : ctx->plain) plain += v->desc.raw_bytes;
+    const uint64_t work = wk.owns_lock() ? ctx->work_bytes : 0;
+    if (plain + work && hipMemGetInfo(&room, &total) == hipSuccess && room + plain + work >= bytes) {
+      if (work) {
+        (void)hipFree(ctx->work);  // (its last user synchronised)
+        ctx->work = nullptr;
+        ctx->work_bytes = 0;
+      }
+      plain_free(ctx, plain);
+      e = hipMalloc(&p, bytes);
+    }
+  }
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    fail(XRH_ERR_OOM, "hipMalloc(" + std::to_string(bytes) + ") failed: " + hipGetErrorString(e));
+  }
+  return p;
+}
+
 void* ctx_alloc(xrh_ctx* ctx, uint64_t bytes)
 {
   if (bytes == 0) bytes = 256;
@@ -92,23 +125,7 @@ void* ctx_alloc(xrh_ctx* ctx, uint64_t bytes)
       std::lock_guard<std::recursive_mutex> lk(ctx->plain_mu);
       plain_free(ctx, over);
     }
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      // once more without the plain voxels, if that can be enough
-      std::lock_guard<std::recursive_mutex> lk(ctx->plain_mu);
-      size_t room = 0, total = 0;
-      uint64_t plain = 0;
-      for (xrh_volume* v : ctx->plain) plain += v->desc.raw_bytes;
-      if (plain && hipMemGetInfo(&room, &total) == hipSuccess && room + plain >= bytes) {
-        plain_free(ctx, plain);
-        e = hipMalloc(&p, bytes);
-      }
-    }
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      fail(XRH_ERR_OOM, "hipMalloc(" + std::to_string(bytes) + ") failed: " + hipGetErrorString(e));
-    }
+    p = device_malloc(ctx, bytes);
   } catch (...) {
     std::lock_guard<std::mutex> lk(ctx->mu);
     ctx->in_use -= bytes;
@@ -173,9 +190,9 @@ void* ctx_work(xrh_ctx* ctx, uint64_t bytes)
     void* old = ctx->work;
     ctx->work = nullptr;
     ctx->work_bytes = 0;
-    ctx_free(ctx, old);  // (its last user synchronised)
+    XRH_HIP_CHECK(hipFree(old));  // (its last user synchronised)
   }
-  ctx->work = ctx_alloc(ctx, bytes);
+  ctx->work = device_malloc(ctx, bytes);
   ctx->work_bytes = bytes;
   return ctx->work;
 }
@@ -934,6 +951,7 @@ xrh_status xrh_ctx_destroy(xrh_ctx* ctx)
     if (ctx->pinned) XRH_HIP_CHECK(hipHostFree(ctx->pinned));
     for (auto& kv : ctx->allocs) (void)hipFree(kv.first);
     ctx->allocs.clear();
+    if (ctx->work) (void)hipFree(ctx->work);
     for (xrh_volume* v : ctx->plain) (void)hipFree(v->raw);
     ctx->plain.clear();
     XRH_HIP_CHECK(hipStreamDestroy(ctx->stream));
