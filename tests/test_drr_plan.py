@@ -82,3 +82,16 @@ def test_whole_rays_reported_as_run(planner):
                    dict(tiles=546, spacing=0.4, reuse=1))
     assert [r[4] for r in rows] == [False, True, False, True]
     assert all((r[0] == 1) == r[4] for r in rows)
+
+
+def test_launches_of_the_slab_tests_take_slabs(planner):
+    """The launches that test_gpu_drr_budget.py compares with and without plain voxels, and the forced choice
+    that the slab tests make."""
+    rows = planner(dict(tiles=1296, mb=75, spacing=0.8), dict(tiles=1296, mb=75, spacing=0.8, objs=2),
+                   dict(tiles=2592, mb=75, spacing=1.3, geom=0))
+    assert all(r[1] for r in rows)
+    forced = planner(dict(tiles=30, mb=1, spacing=0.4, objs=2), dict(tiles=30, mb=1, spacing=3.2, objs=3, geom=0),
+                     dict(tiles=30, mb=1, spacing=0.4, storage=F16, layout=OCT), env={"XRH_CELL_REUSE": "1"})
+    assert all(r[1] for r in forced)
+    shared = planner(dict(tiles=30, mb=1, spacing=0.4), env={"XRH_CELL_REUSE": "0"})
+    assert not shared[0][1] and shared[0][0] == 4
