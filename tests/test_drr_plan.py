@@ -95,3 +95,11 @@ def test_launches_of_the_slab_tests_take_slabs(planner):
     assert all(r[1] for r in forced)
     shared = planner(dict(tiles=30, mb=1, spacing=0.4), env={"XRH_CELL_REUSE": "0"})
     assert not shared[0][1] and shared[0][0] == 4
+
+
+def test_sparse_rays_of_small_launches(planner):
+    """Few sparse FP32 rays are shared by four waves whose lanes keep in step, more by two; close ones
+    keep the long window."""
+    rows = planner(*[dict(tiles=t, spacing=s, geom=0) for t, s in ((64, 2.3), (100, 3.5), (200, 2.8), (72, 1.43), (256, 0.6))])
+    assert [r[0] for r in rows] == [4, 4, 2, 4, 4]
+    assert [r[3] for r in rows] == [4, 1, 16, 4, 16]

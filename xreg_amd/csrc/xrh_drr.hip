@@ -1058,7 +1058,7 @@ __device__ __forceinline__ float cast_ray_slab(const DrrItem& it, const TileRef&
 // segments in order, so the value is cast_ray's bit for bit. The first two parts walk over the
 // empty space from one end each. Every thread of the block calls it (it synchronises).
 template <int kGeom, int kOp, int kFmt, int kParts>
-__device__ __forceinline__ float cast_ray_split(const DrrItem& it, int col, int row, bool inside)
+__device__ __forceinline__ float cast_ray_split(const DrrItem& it, int col, int row, bool inside, int window)
 {
   static_assert(kParts >= 2 && kSegs % kParts == 0, "segments are dealt evenly");
   __shared__ float sums[kSegs][kThreads];
@@ -1088,7 +1088,7 @@ __device__ __forceinline__ float cast_ray_split(const DrrItem& it, int col, int 
     float acc = line_init<kOp>();
     if (i <= stop) {
       if constexpr (kGeom == XRH_GEOM_FP32) pos.advance(ray, i - at);
-      acc = march<kGeom, kOp, kFmt>(ray, vol_view(it), pos, i, stop, seg, i, kWindow);
+      acc = march<kGeom, kOp, kFmt>(ray, vol_view(it), pos, i, stop, seg, i, window);
       at = stop + 1;
     }
     sums[k][px] = acc;
@@ -1104,8 +1104,8 @@ __device__ __forceinline__ float cast_ray_split(const DrrItem& it, int col, int 
   return acc;
 }
 
-// kParts: the waves that share a ray, 0 for slab marching with `budget` floats of dynamic LDS. Whole rays that
-// gather by cells wait for each other every `window` samples.
+// kParts: the waves that share a ray, 0 for slab marching with `budget` floats of dynamic LDS. Rays
+// that gather by cells wait for each other every `window` samples.
 template <int kGeom, int kOp, int kFmt, int kParts>
 __device__ __forceinline__ float cast_pixel(const DrrItem& it, const TileRef& tr, int col, int row, bool inside,
                                             int budget, int window)
@@ -1114,7 +1114,7 @@ __device__ __forceinline__ float cast_pixel(const DrrItem& it, const TileRef& tr
     extern __shared__ __attribute__((aligned(16))) float box_lds[];
     return cast_ray_slab<kGeom, kOp, kFmt>(it, tr, col, row, inside, box_lds, budget, window);
   } else if constexpr (kParts == 1) return cast_ray<kGeom, kOp, kFmt>(it, col, row, inside, window);
-  else return cast_ray_split<kGeom, kOp, kFmt, kParts>(it, col, row, inside);
+  else return cast_ray_split<kGeom, kOp, kFmt, kParts>(it, col, row, inside, window);
 }
 
 template <int kGeom, int kOp, int kFmt, int kParts>
@@ -1223,8 +1223,8 @@ int device_cus()
 // same rays then evict each other's: over 512 tiles a wave takes whole rays from 0.95 voxels on (us,
 // shared by two / whole: 546 tiles at 1.94 voxels 478 / 386, 686 at 2.26 1037 / 790, 624 at 1.0 510 /
 // 387); up to 512 FP32 rays are shared by four while there are few or they are close, else by two (four /
-// two: 252 tiles at 1.03 80 / 95, 98 at 1.64 129 / 132, 507 at 1.01 177 / 161; whole / two: 72 at 2.77 427 /
-// 260, 100 at 3.55 427 / 374, 200 at 2.66 339 / 275), and 16-bit rays, with half the loads, by four up to
+// two: 252 tiles at 1.03 80 / 95, 64 at 1.88 217 / 240, 128 at 1.88 214 / 227, 100 at 3.0 248 / 259, 200 at 3.0 243 /
+// 239, 507 at 1.01 177 / 161; whole / two: 72 at 2.77 427 / 260, 200 at 2.66 339 / 275), and 16-bit rays, with half the loads, by four up to
 // 1.75 voxels (210 tiles at 1.67 four / two 111 / 117), from there by two only up to 128 tiles (whole / two:
 // 50 at 3.76 286 / 263, 280 at 3.22 267 / 281, 440 at 1.82 181 / 199).
 // Where rays are close and gather, sharing by two pays up to twice as many tiles (16-bit, whole / shared:
@@ -1234,7 +1234,7 @@ int drr_parts(int64_t tiles, float spacing, int slab, int32_t storage)
   const int64_t waves = tiles * (kThreads / 64), room = 32ll * device_cus();
   if (waves * 4 <= room) {
     if (storage != XRH_F32) return spacing < 1.75f ? 4 : (waves * 16 <= room ? 2 : 1);
-    return (spacing < 0.95f || (spacing < 1.65f && waves * 8 <= room)) ? 4 : 2;
+    return (spacing < 0.95f || waves * (spacing < 1.65f ? 8 : 16) <= room) ? 4 : 2;
   }
   if (slab == 0 && spacing > 0.0f && spacing < 0.75f && waves <= room) return 2;
   return (waves * 2 <= room && spacing < 0.95f) ? 2 : 1;
@@ -1275,12 +1275,17 @@ int gather_window(float spacing, int32_t layout)
 // 3388).
 int gather_lds(float spacing) { return (spacing >= 1.1f) ? slab_lds(spacing) : 0; }
 
+// The same where four waves share a ray: they are at four depths of it, and sparse rays meet no lines of each
+// other's (us, 16 / 4 / 1 samples: 128 tiles at 1.16 voxels 92 / 97 / 114, 72 at 1.43 116 / 111 / 110, at 1.55 102 / 102 /
+// 116, 64 at 1.88 232 / 217 / 218, at 2.33 122 / 114 / 120, 100 at 3.0 282 / 257 / 248).
+int shared_window(float spacing) { return spacing >= 2.7f ? 1 : (spacing >= 1.3f ? 4 : kWindow); }
+
 // How a launch marches. Slabs need the plain voxels of every volume beside a face or oct layout.
 struct March {
   int parts;   // waves that share a ray
   bool slabs;  // whole rays by slabs
   int lds;     // dynamic LDS bytes: the boxes of the slabs, or held unused by whole rays that gather
-  int window;  // samples between the points where the lanes of whole rays wait
+  int window;  // samples between the points where a wave's lanes wait
 };
 
 March drr_march(const DrrLaunch& L, int64_t tiles)
@@ -1298,7 +1303,7 @@ March drr_march(const DrrLaunch& L, int64_t tiles)
                                            : drr_parts(tiles, L.ray_spacing, slab, L.storage);
   m.slabs = m.parts == 1 && slab > 0;
   m.lds = m.slabs ? slab : 0;
-  m.window = gather_window(L.ray_spacing, L.layout);
+  m.window = m.parts == 1 ? gather_window(L.ray_spacing, L.layout) : (m.parts == 4 ? shared_window(L.ray_spacing) : kWindow);
   // (launches that could go by slabs and do not are better off without)
   if (!able && m.parts == 1 && L.vol_bytes >= kSlabBytes &&
       (L.storage == XRH_F32 ? L.layout != kLayoutQuad && L.layout != kLayoutLinear : L.layout == kLayoutOct)) {
