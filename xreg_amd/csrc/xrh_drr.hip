@@ -695,10 +695,10 @@ __device__ __forceinline__ float cast_ray(const DrrItem& it, int col, int row, b
 // gathering march's bit for bit, and tiles whose box
 // does not fit (rays several voxels apart, oblique tiles) take that march.
 //
-// Measured, FP64 set-up, ns per ray, gathering sample by sample (before) / by cells / slabs: 256 x
-// 256 x 200 voxels at 0.39 voxels between rays 0.412 / 0.355 / 0.330, 0.78: 0.582 / 0.644 / 0.427,
-// 1.55: 1.33 / 1.53 / 1.01; 512 x 512 x 400 voxels at 0.39: 0.942 / 0.748 / 0.554, 0.78: 1.16 / 1.69
-// / 0.746, 1.55: 3.5 / 3.8 / 1.79. Layers per slab:
+// Measured, FP64 set-up, launches of 1 to 1.8 million rays, ns per ray, gathering sample by sample (before) / by
+// cells / slabs: 256 x 256 x 200 voxels at 0.39 voxels between rays 0.430 / 0.372 / 0.349, 0.78: 0.60 / 0.553 /
+// 0.438, 1.55: 1.39 / 1.07 / 1.02; 512 x 512 x 400 voxels at 0.39: 1.01 / 0.817 / 0.585, 0.78: 1.34 / 1.36 / 0.841,
+// 1.55: 3.5 / 2.8 / 1.84. Layers per slab:
 // 8 / 12 / 16 at 0.39: 0.386 / 0.351 / 0.353; along x one 64-byte row of 16 voxels.
 constexpr int kSlabDepth = 12, kSlabDepthX = 15;
 
