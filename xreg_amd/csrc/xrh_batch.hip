@@ -406,10 +406,11 @@ DrrLaunch stage(xrh_batch* b, const int32_t* item_view, const double* item_pose,
   DrrVariant var = b->variant;
   if (!b->variant_set) {
     var = DrrVariant();
-    const std::string key = tune_key(D, rows, cols);
     std::lock_guard<std::mutex> lk(b->ctx->mu);
-    auto it = b->ctx->tuned.find(key);
-    if (it != b->ctx->tuned.end()) var = it->second;
+    if (!b->ctx->tuned.empty()) {  // (a key takes a microsecond, a single pose's evaluation 60)
+      auto it = b->ctx->tuned.find(tune_key(D, rows, cols));
+      if (it != b->ctx->tuned.end()) var = it->second;
+    }
   }
   b->last_variant = var;
   const TilePlan plan = build_tiles(rows, cols, var.bands);

@@ -776,10 +776,11 @@ static void line_int_launch(xrh_ctx* ctx, const xrh_volume* vol, const xrh_camer
   DrrVariant var;
   if (!fixed) {
     const int64_t wgs = (int64_t)((rows + 15) / 16) * ((cols + 15) / 16) * num_projs;
-    const std::string key = drr_tune_key(L, rows, cols, wgs);
     std::lock_guard<std::mutex> lk(ctx->mu);
-    auto it = ctx->tuned.find(key);
-    if (it != ctx->tuned.end()) var = it->second;
+    if (!ctx->tuned.empty()) {
+      auto it = ctx->tuned.find(drr_tune_key(L, rows, cols, wgs));
+      if (it != ctx->tuned.end()) var = it->second;
+    }
   }
   const int32_t bands = std::min(std::max(var.bands, 1), kMaxDrrBands);
 
