@@ -111,6 +111,19 @@ def test_budget_is_what_it_was(ctx):
     c.close()
 
 
+def test_not_counted_without_a_budget(ctx):
+    """A server admits jobs by the bytes in use of a context that has no budget itself."""
+    from xreg_amd import _xrh as X
+
+    print("case: bytes in use without a budget", flush=True)
+    vox, i2p, _, _, _ = _scene(0.8)
+    used = ctx.bytes_in_use()
+    v = X.Volume(ctx, vox, i2p)
+    assert v.nbytes <= ctx.bytes_in_use() - used < v.nbytes + PLAIN
+    v.close()
+    assert ctx.bytes_in_use() == used
+
+
 def test_given_back_while_another_thread_evaluates():
     from xreg_amd import _xrh as X
 
